@@ -6,11 +6,9 @@
 // applied to magnitudes), so results are bit-identical. Two forms of the product: one thread
 // streams it word by word from LDS operands into its consumer (store, subtract, accumulate), or
 // one wave holds a word per lane, sums the columns on the lanes and normalises them with shuffles
-// and ballot carry-lookahead (lane_mulfx). When the tile's lower triangle fits in LDS
+// and ballot carry-lookahead (lane_mul). When the tile's lower triangle fits in LDS
 // (k_tile_chol_lds) the factorisation runs there and the inverse is built column-parallel
 // (k_tile_inverse); otherwise k_tile_factor works on the tile in HBM.
-#include <cstdlib>
-
 #include "common.hpp"
 
 namespace {
@@ -268,12 +266,20 @@ __device__ void wave_rsqrt(const Pivot& P) {
 }
 
 // ---------------------------------------------------------------- lane-parallel pivot arithmetic
-// For WL <= 64 the pivot chain runs on wave 0 with one word per lane (word k in lane k, lanes >= WL
-// hold 0): magnitudes and additions use a carry lookahead over ballots, products sum their
-// columns on the lanes and normalise the column sums with shuffles and one more lookahead. The
+// For WL <= 64 a number is held by one wave with one word per lane (word k in lane k, zero in lanes >= WL):
+// carries come from one 64-bit lookahead over ballots, and a product sums its columns on the lanes. The
 // results are word for word those of wave_mul / wave_rsqrt above (the same truncated product).
+//
+// A 32 x 32 tile at L = 24 is bound by the latency of these products: a pivot is a chain of 16 of them. On
+// one wave an instruction that depends on the one before costs 8 cycles, a ballot or a lane read whose
+// scalar is used at once 30, and an LDS round trip 56 (in-kernel clock, one MI355X); so nothing but
+// the operand words goes through LDS, magnitudes, signs and top words are found once per operand and not
+// once per product, and the lane lookahead and the products are always inlined (out of line their LDS
+// operands turn into flat accesses). The product took 2300 cycles out of line with its lane exchanges
+// through the LDS crossbar.
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ u32 lane_get(u32 v, int src) { return (u32)__shfl((int)v, src, 64); }
+__device__ __forceinline__ u32 lane_read(u32 v, int src) { return (u32)__builtin_amdgcn_readlane((int)v, src); }
 __device__ __forceinline__ u64 lane_get64(u64 v, int src) {
     return ((u64)lane_get((u32)(v >> 32), src) << 32) | lane_get((u32)v, src);
 }
@@ -283,47 +289,122 @@ __device__ __forceinline__ u64 from_below64(u64 v) {
     const u64 r = lane_get64(v, l > 0 ? l - 1 : 0);
     return l > 0 ? r : 0;
 }
+__device__ __forceinline__ u64 ballot64(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+// 1 in the lanes of the mask m (uniform)
+__device__ __forceinline__ u32 mask_bit(u64 m) { return __builtin_amdgcn_inverse_ballot_w64(m) ? 1u : 0u; }
+
+// LDS words of one wave's products: the left magnitude with zeros above, the right one with zeros on both
+// sides (column c reads word c - i for every term i). Terms are read in groups that reach up to 32 past the
+// top word ta <= LF + 23: words up to LF + 55 on the left, LF - 2 - ta - 32 to LF - 2 + 63 on the right
+// (LF <= 40)
+constexpr int LANE_X = 96, LANE_Y0 = 60, LANE_Y = LANE_Y0 + 104, LANE_LDS = LANE_X + LANE_Y;
+
+// what the lane operations share: sizes, this lane's word mask (ones below WL), the wave's LDS words
+struct Lane {
+    int WL, LF;
+    u32 in;
+    u32* buf;
+    __device__ __forceinline__ Lane(int wl, int lf, u32* b) : WL(wl), LF(lf), in(lane_id() < wl ? ~0u : 0u), buf(b) {
+        for (int q = lane_id(); q < LANE_LDS; q += 64) buf[q] = 0u;
+        wave_sync();
+    }
+};
 
 // top word index of the number (>= 1), else 0 (topl_slot semantics)
-__device__ __forceinline__ int lane_top(u32 w, int WL) {
-    const u64 nz = __ballot(lane_id() < WL && w != 0);
+__device__ __forceinline__ int lane_top(u32 w) {
+    const u64 nz = ballot64(w != 0);
     return nz ? 63 - __builtin_clzll(nz) : 0;
 }
 
 // two's complement negation over WL words: ~w + 1, the +1 absorbed by the lowest nonzero word
-__device__ u32 lane_neg(u32 w, int WL) {
-    const int l = lane_id();
-    const u64 nz = __ballot(l < WL && w != 0);
-    const int first = nz ? __builtin_ctzll(nz) : 64;
-    if (l >= WL) return 0u;
-    return l < first ? 0u : (l == first ? ~w + 1u : ~w);
+__device__ __forceinline__ u32 lane_neg(const Lane& Q, u32 w) {
+    const u64 nz = ballot64(w != 0);
+    const u64 low = nz & (0 - nz);                       // the lowest nonzero word's lane
+    return ((__builtin_amdgcn_inverse_ballot_w64(~(low | (low - 1))) ? ~w : 0u) |
+            (__builtin_amdgcn_inverse_ballot_w64(low) ? 0u - w : 0u)) & Q.in;
 }
 
 // a + b + cin mod 2^(32 WL): generate / propagate masks from two ballots, the carry into every word
 // from one 64-bit addition ((G|P) + G + cin) ^ (G|P) ^ G
-__device__ u32 lane_add(u32 a, u32 b, unsigned cin, int WL) {
-    const int l = lane_id();
-    const u64 s = (u64)a + b;
-    const u64 G = __ballot(l < WL && (s >> 32) != 0);
-    const u64 P = __ballot(l < WL && (u32)s == 0xffffffffu);
+__device__ __forceinline__ u32 lane_add(const Lane& Q, u32 a, u32 b, unsigned cin) {
+    const u32 s = a + b;
+    const u64 G = ballot64(s < a), P = ballot64(s == 0xffffffffu);
     const u64 X = G | P;
-    const u64 carries = (X + G + cin) ^ X ^ G;
-    return l < WL ? (u32)s + (u32)((carries >> l) & 1u) : 0u;
+    return (s + mask_bit((X + G + cin) ^ X ^ G)) & Q.in;
 }
 
-// mulfx(a, b, t) of two's complement lane numbers; xs, ys: WL words of LDS for the magnitudes
-__device__ u32 lane_mulfx(u32 a, u32 b, int t, int WL, int LF, u32* xs, u32* ys) {
-    const int l = lane_id();
-    const bool sa = (lane_get(a, WL - 1) >> 31) != 0, sb = (lane_get(b, WL - 1) >> 31) != 0;
-    const u32 ma = sa ? lane_neg(a, WL) : a, mb = sb ? lane_neg(b, WL) : b;
-    const int ta = lane_top(ma, WL), tb = lane_top(mb, WL);
-    __builtin_amdgcn_wave_barrier();                     // earlier readers of xs / ys are done
-    if (l < WL) {
-        xs[l] = ma;
-        ys[l] = mb;
+// the words of sum_l (w0 + w1 2^32 + w2 2^64) 2^(32 l) over the lanes of `live` (a run of low lanes;
+// w2 < 2^30), carries out of it dropped
+__device__ __forceinline__ u32 lane_digits(u32 w0, u32 w1, u32 w2, u64 live) {
+    const u64 d = (u64)w0 + lane_below(w1) + lane_below(lane_below(w2));
+    const u32 d0 = (u32)d, e = d0 + lane_below((u32)(d >> 32));
+    const u64 G = ballot64(e < d0) & live, P = ballot64(e == 0xffffffffu) & live;
+    const u64 X = G | P;
+    return e + mask_bit((X + G) ^ X ^ G);
+}
+
+// a number as magnitude, sign and top word
+struct LaneMag {
+    u32 m;
+    int top;
+    bool neg;
+};
+__device__ __forceinline__ LaneMag lane_mag(const Lane& Q, u32 a) {
+    LaneMag r;
+    r.neg = (lane_read(a, Q.WL - 1) >> 31) != 0;
+    r.m = r.neg ? lane_neg(Q, a) : a;
+    r.top = lane_top(r.m);
+    return r;
+}
+// lane_mag of a number that has its top bit clear unless it overflowed: the sign is looked at only when
+// the top word is set at all
+__device__ __forceinline__ LaneMag lane_mag_pos(const Lane& Q, u32 a) {
+    LaneMag r{a, lane_top(a), false};
+    if (r.top == Q.WL - 1) r = lane_mag(Q, a);
+    return r;
+}
+__device__ __forceinline__ u32 lane_signed(const Lane& Q, u32 w, bool neg) { return neg ? lane_neg(Q, w) : w; }
+
+// Column sums of the magnitudes in Q.buf (x words la..ta, y words with zeros outside their range) as
+// 96-bit values: the lane's column is LF - 2 + lane. HALF: the columns fit the lower 32 lanes; the two
+// lane halves take the even and the odd terms and both end up with the sums. U terms per lane and
+// group, all their words requested before the first multiply (terms past ta are zero): a group costs one
+// LDS latency and 14 cycles a term.
+template <bool HALF, int U>
+__device__ __forceinline__ void lane_columns(const Lane& Q, int la, int ta, u64& s, u32& o) {
+    constexpr int ST = HALF ? 2 : 1;                     // terms between two terms of one lane
+    const int l = lane_id(), c = HALF ? (l & 31) : l, h = HALF ? (l >> 5) : 0;
+    const u32* xp = Q.buf + la + h;
+    const u32* yp = Q.buf + LANE_X + LANE_Y0 + Q.LF - 2 + c - la - h;
+    s = 0;
+    o = 0;
+    for (int i = la; i <= ta; i += U * ST) {
+        u32 x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            x[u] = xp[ST * u];
+            y[u] = yp[-ST * u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u += 4) SDPV_MAC96_CHAIN4(s, o, x + u, y + u);
+        xp += U * ST;
+        yp -= U * ST;
     }
-    __builtin_amdgcn_wave_barrier();
-    const int la = t ? max(0, ta - t + 1) : 0, lb = t ? max(0, tb - t + 1) : 0;
+    SDPV_SETTLE(s, o);
+    if (HALF) {
+        u32 a0 = (u32)s, b0 = a0, a1 = (u32)(s >> 32), b1 = a1, a2 = o, b2 = o;
+        swap_halves(a0, b0);
+        swap_halves(a1, b1);
+        swap_halves(a2, b2);
+        const u64 p = ((u64)a1 << 32) | a0, q = ((u64)b1 << 32) | b0;
+        s = p + q;
+        o = a2 + b2 + (s < p ? 1u : 0u);
+    }
+}
+
+// columns beyond 64 (both operands far above one): two columns per lane, lane exchanges through the crossbar
+__device__ __forceinline__ u32 lane_mul_wide(const u32* xs, const u32* ys, int la, int lb, int ta, int tb, int WL, int LF) {
+    const int l = lane_id();
     const int kmin = max(LF - 2, la + lb), kmax = ta + tb;
     // column sums of columns kmin + l (h = 0) and kmin + 64 + l (h = 1) as lo / hi 32-bit halves
     u64 lo[2], hi[2];
@@ -360,26 +441,57 @@ __device__ u32 lane_mulfx(u32 a, u32 b, int t, int WL, int LF, u32* xs, u32* ys)
     // output word j = digit of column LF + j
     const int q = LF + l - kmin;
     const u32 w0 = lane_get(dig0, q & 63), w1 = lane_get(dig1, q & 63);
-    u32 w = (l >= WL || q < 0 || q > kmax + 2 - kmin) ? 0u : (q < 64 ? w0 : w1);
-    __builtin_amdgcn_wave_barrier();
-    return (sa ^ sb) ? lane_neg(w, WL) : w;
+    const u32 w = (l >= WL || q < 0 || q > kmax + 2 - kmin) ? 0u : (q < 64 ? w0 : w1);
+    return w;
+}
+
+// magnitude of mulfx(a, b, t): columns from max(LF - 2, la + lb) on of the truncated operands. U: terms per
+// lane and group of the half-wave form (2 U terms: 8 hold t <= 8, 16 hold t <= 16, 32 a number below
+// one of up to 32 words)
+template <int U>
+__device__ __forceinline__ u32 lane_mul(const Lane& Q, const LaneMag& a, const LaneMag& b, int t) {
+    const int l = lane_id(), ta = a.top, tb = b.top, LF = Q.LF;
+    const int la = (t && ta >= t) ? ta - t + 1 : 0, lb = (t && tb >= t) ? tb - t + 1 : 0;
+    wave_sync();                                         // earlier readers of the buffer are done
+    Q.buf[l] = a.m;
+    Q.buf[LANE_X + LANE_Y0 + l] = l >= lb ? b.m : 0u;
+    wave_sync();
+    // position q = column LF - 2 + q (columns below la + lb are empty), up to column ta + tb + 2
+    const int npos = ta + tb - LF + 5;
+    u64 s;
+    u32 o, dig;
+    if (__builtin_expect(npos <= 32, 1)) {
+        lane_columns<true, U>(Q, la, ta, s, o);
+        dig = lane_digits((u32)s, (u32)(s >> 32), o, 0xffffffffull);
+        dig = l < 32 ? dig : 0u;
+    } else if (npos <= 64) {
+        lane_columns<false, 16>(Q, la, ta, s, o);
+        dig = lane_digits((u32)s, (u32)(s >> 32), o, ~0ull);
+    } else {
+        return lane_mul_wide(Q.buf, Q.buf + LANE_X + LANE_Y0, la, lb, ta, tb, Q.WL, LF);
+    }
+    return lane_above(lane_above(dig)) & Q.in;           // output word j = digit of column LF + j
+}
+
+// mulfx(a, b, t) of two's complement lane numbers
+__device__ __forceinline__ u32 lane_mulfx(const Lane& Q, u32 a, u32 b, int t) {
+    const LaneMag x = lane_mag(Q, a), y = lane_mag(Q, b);
+    return lane_signed(Q, lane_mul<16>(Q, x, y, t), x.neg != y.neg);
 }
 
 // basecase.py:59-68 on a lane number, the same value in every lane
-__device__ double lane_to_double(u32 a, int WL, int LF) {
-    const bool s = (lane_get(a, WL - 1) >> 31) != 0;
-    const u32 m = s ? lane_neg(a, WL) : a;
-    const int t = lane_top(m, WL);
-    const u32 m0 = lane_get(m, t), m1 = lane_get(m, t >= 1 ? t - 1 : 0), m2 = lane_get(m, t >= 2 ? t - 2 : 0);
+__device__ __forceinline__ double lane_to_double(const LaneMag& a, int LF) {
+    const int t = a.top;
+    const u32 m0 = lane_read(a.m, t), m1 = lane_read(a.m, t >= 1 ? t - 1 : 0), m2 = lane_read(a.m, t >= 2 ? t - 2 : 0);
     double v = (double)m0;
     if (t >= 1) v = v * 4294967296.0 + (double)m1;
     if (t >= 2) v = v * 4294967296.0 + (double)m2;
     v = ldexp(v, 32 * (t - 2 > 0 ? t - 2 : 0) - 32 * LF);
-    return s ? -v : v;
+    return a.neg ? -v : v;
 }
 
 // basecase.py:69-78: the lane's word of the fixed-point value of v (0 for non-positive v)
-__device__ u32 lane_from_double(double v, int WL, int LF) {
+__device__ __forceinline__ u32 lane_from_double(double v, int WL, int LF) {
     const int l = lane_id();
     if (!(v > 0.0) || !isfinite(v) || l >= WL) return 0u;
     int e;
@@ -397,23 +509,35 @@ __device__ u32 lane_from_double(double v, int WL, int LF) {
     return k == 0 ? (u32)lo : k == 1 ? (u32)(lo >> 32) : k == 2 ? (u32)hi : k == 3 ? (u32)(hi >> 32) : 0u;
 }
 
-// d^-1/2 (basecase.py:145-156): double seed, Newton r <- r + r (1 - d r^2) / 2, precision doubling
-__device__ u32 lane_rsqrt(u32 d, int WL, int LF, u32* xs, u32* ys) {
-    const int l = lane_id();
-    u32 r = lane_from_double(1.0 / sqrt(lane_to_double(d, WL, LF)), WL, LF);
-    for (int bits = 100;; bits *= 2) {
-        int t = bits / 32 + 2;
-        if (t >= WL) t = 0;
-        u32 t1 = lane_mulfx(r, r, t, WL, LF, xs, ys);
-        u32 t2 = lane_mulfx(t1, d, t, WL, LF, xs, ys);
-        t1 = lane_add(l == LF ? 1u : 0u, ~t2, 1u, WL);            // one - t2
-        t2 = lane_mulfx(r, t1, t, WL, LF, xs, ys);
-        const u32 above = lane_get(t2, l < 63 ? l + 1 : 63);      // word l + 1
-        const u32 half = (l < WL - 1) ? ((t2 >> 1) | (above << 31)) : (u32)(((int)t2) >> 1);
-        r = lane_add(r, half, 0u, WL);                            // r += t2 >> 1 (arithmetic)
-        if (t == 0) break;
-    }
+// d^-1/2 (basecase.py:145-156): double seed, Newton steps r <- r + r (1 - d r^2) / 2 on t = bits / 32 + 2 words,
+// bits = 100, 200, 400, ... (all words once t >= WL)
+template <int U>
+__device__ __forceinline__ u32 lane_newton(const Lane& Q, const LaneMag& d, u32 r, int t) {
+    const int l = lane_id(), WL = Q.WL, LF = Q.LF;
+    const LaneMag R = lane_mag_pos(Q, r);
+    const LaneMag t1 = lane_mag_pos(Q, lane_mul<U>(Q, R, R, t));
+    const u32 t2 = lane_mul<U>(Q, t1, d, t);
+    // one - t2, t2 carrying the sign of its product
+    const bool t2neg = t1.neg != d.neg;
+    const LaneMag e = lane_mag(Q, lane_add(Q, l == LF ? 1u : 0u, (t2neg ? t2 : ~t2) & Q.in, t2neg ? 0u : 1u));
+    const u32 h = lane_signed(Q, lane_mul<U>(Q, R, e, t), R.neg != e.neg);
+    const u32 above = lane_above(h);                              // word l + 1
+    const u32 half = (l < WL - 1) ? ((h >> 1) | (above << 31)) : (u32)(((int)h) >> 1);
+    return lane_add(Q, r, half & Q.in, 0u);                       // r += h >> 1 (arithmetic)
+}
+// the seed and the steps on 5 and 8 words (bits = 100 and 200; WL >= 25)
+__device__ __forceinline__ u32 lane_rsqrt_begin(const Lane& Q, const LaneMag& d) {
+    u32 r = lane_from_double(1.0 / sqrt(lane_to_double(d, Q.LF)), Q.WL, Q.LF);
+    for (int t = 5; t <= 8; t += 3) r = lane_newton<4>(Q, d, r, t);
     return r;
+}
+__device__ __forceinline__ u32 lane_rsqrt_finish(const Lane& Q, const LaneMag& d, u32 r) {
+    r = lane_newton<8>(Q, d, r, 14);                              // bits = 400
+    for (int bits = 800;; bits *= 2) {
+        const int t = bits / 32 + 2 < Q.WL ? bits / 32 + 2 : 0;
+        r = lane_newton<16>(Q, d, r, t);
+        if (t == 0) return r;
+    }
 }
 
 // ---------------------------------------------------------------- the tile kernel
@@ -446,9 +570,11 @@ __global__ void __launch_bounds__(TT) k_tile_factor(u32* __restrict__ Wg, u32* _
         // pivot: d = A_kk, r = d^-1/2, A_kk = d r, RINV_k = r
         if (WL <= 64) {                                   // one word per lane on wave 0
             if (tid < 64) {
+                const Lane Q(WL, LF, (u32*)(P.col + 2 * (2 * WL + 4)));
                 const u32 d = tid < WL ? ent(W, k, k)[tid] : 0u;
-                const u32 r = lane_rsqrt(d, WL, LF, P.sx, P.sy);
-                const u32 dr = lane_mulfx(d, r, 0, WL, LF, P.sx, P.sy);
+                const LaneMag dm = lane_mag(Q, d);
+                const u32 r = lane_rsqrt_finish(Q, dm, lane_rsqrt_begin(Q, dm));
+                const u32 dr = lane_mulfx(Q, d, r, 0);
                 if (tid < WL) {
                     ent(W, k, k)[tid] = dr;
                     rinv[k * WL + tid] = r;
@@ -568,7 +694,7 @@ constexpr int TWAVES = TT / 64;
 // stride WS)
 __host__ __device__ inline i64 lds_factor_words(int BT, int WL, int nw) {
     const i64 WS = WL | 1;
-    return (i64)BT * (BT + 1) / 2 * WS + (i64)BT * WS + WL + 2 * BT + 128 * nw;
+    return (i64)BT * (BT + 1) / 2 * WS + (i64)BT * WS + WL + 2 * BT + LANE_LDS * nw;
 }
 
 // row i of the packed lower triangle starts at entry i (i + 1) / 2
@@ -583,16 +709,16 @@ __device__ __forceinline__ void tri_pair(int p, int& i, int& j) {
     j = p - r * (r + 1) / 2;
 }
 
-// A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`): x, y magnitudes with top words
+// (operands with words above N, which a factor of an SPD tile never has:) A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`): x, y magnitudes with top words
 // ta, tb, A a WL-word two's complement target. The column sums are formed four columns at a time:
 // x[i] is read once per block and the four operand words y[kb + c - i] sit in a window of registers
 // that shifts by one word per i, so a block costs two LDS reads per i instead of eight; the target
 // words of a block are read before its columns are summed. The column sums, the carry chain and the
 // target words equal those of mulfx_mag and its consumer (terms outside the tops are zero).
-__device__ __forceinline__ void trail_update(const u32* x, const u32* y, int ta, int tb, int WL, int LF, u32* A,
+__device__ __forceinline__ void trail_update_any(const u32* x, const u32* y, int ta, int tb, int WL, int LF, u32* A,
                                              bool add) {
     const int kmin = max(LF - 2, 0), kmax = ta + tb, kend = LF + WL;
-    u64 carry = 0, hprev = 0, cy = 0;  // product chain; carry of the addition
+    u64 carry = 0, cy = 0;             // carry into the next column; carry of the addition
     i64 br = 0;                          // borrow of the subtraction
     for (int kb = kmin; kb < kend; kb += 4) {
         u32 tw[4];
@@ -601,7 +727,8 @@ __device__ __forceinline__ void trail_update(const u32* x, const u32* y, int ta,
             const int j = kb + c - LF;
             tw[c] = (j >= 0 && j < WL) ? A[j] : 0u;
         }
-        u64 lo[4] = {0, 0, 0, 0}, hi[4] = {0, 0, 0, 0};
+        u64 acc[4] = {0, 0, 0, 0};
+        u32 ov[4] = {0, 0, 0, 0};
         if (kb <= kmax) {
             const int I0 = max(0, kb - tb), I1 = min(ta, kb + 3);
             u32 w[4];
@@ -620,12 +747,7 @@ __device__ __forceinline__ void trail_update(const u32* x, const u32* y, int ta,
                 }
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-#pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        const u64 p = (u64)xa[u] * w[c];
-                        lo[c] += (u32)p;
-                        hi[c] += p >> 32;
-                    }
+                    SDPV_MAC96_COLS4(acc, ov, xa[u], w);
                     w[3] = w[2];
                     w[2] = w[1];
                     w[1] = w[0];
@@ -639,9 +761,8 @@ __device__ __forceinline__ void trail_update(const u32* x, const u32* y, int ta,
             if (k >= kend) break;
             u32 wv = 0u;
             if (k <= kmax + 2) {
-                const u64 sm = lo[c] + hprev + carry;
-                carry = sm >> 32;
-                hprev = hi[c];
+                const u64 sm = acc[c] + carry;
+                carry = (sm >> 32) | ((u64)(ov[c] + (sm < carry ? 1u : 0u)) << 32);
                 wv = (u32)sm;
             }
             if (k >= LF) {
@@ -659,19 +780,87 @@ __device__ __forceinline__ void trail_update(const u32* x, const u32* y, int ta,
     }
 }
 
-// Pivot k: wave 0 computes r = d^-1/2 and d r (lane_rsqrt, lane_mulfx). Column scale: the waves
-// take the entries i > k in turn, L_ik = lane_mulfx(A_ik, r), and keep |L_ik|, its top word and its
-// sign for the trailing products. Trailing update over the pairs k < j <= i: wave 0 updates the
-// next diagonal entry and goes on to pivot k + 1 (look-ahead), the other waves update the
-// remaining pairs, one pair per thread while there are more than `lane_pairs`, else one per wave.
-// NT threads: 256 (one wave per SIMD), 512 or 1024 (two or four waves per SIMD: more instruction
-// streams per SIMD, and 448 or 960 threads for the trailing products).
-template <int NT>
+// acc + ov 2^64 = sum of x[i] y[K - i] over the static column K of two N-word magnitudes
+template <int N, int K>
+__device__ __forceinline__ void column_sum(const u32* x, const u32* y, u64& acc, u32& ov) {
+    constexpr int I0 = K - (N - 1) > 0 ? K - (N - 1) : 0, I1 = K < N - 1 ? K : N - 1, NT = I1 - I0 + 1;
+    acc = 0;
+    ov = 0;
+#pragma unroll
+    for (int q = 0; q < NT / 4; q++) {
+        const u32 yv[4] = {y[K - I0 - 4 * q], y[K - I0 - 4 * q - 1], y[K - I0 - 4 * q - 2], y[K - I0 - 4 * q - 3]};
+        SDPV_MAC96_CHAIN4(acc, ov, x + I0 + 4 * q, yv);
+    }
+#pragma unroll
+    for (int i = I0 + NT / 4 * 4; i <= I1; i++) SDPV_MAC96(acc, ov, x[i], y[K - i]);
+}
+template <int N, int K>
+struct TrailColumns {
+    // columns K and up: digit of column k into word k - LF of A
+    template <class Put>
+    static __device__ __forceinline__ void run(const u32* x, const u32* y, int LF, u64& carry, Put& put) {
+        if (K >= LF - 2) {                               // uniform: the first few columns only
+            u64 acc;
+            u32 ov;
+            column_sum<N, K>(x, y, acc, ov);
+            const u64 sm = acc + carry;
+            carry = (sm >> 32) | ((u64)(ov + (sm < carry ? 1u : 0u)) << 32);
+            if (K >= LF) put(K - LF, (u32)sm);
+        }
+        if constexpr (K < 2 * N - 2) TrailColumns<N, K + 1>::run(x, y, LF, carry, put);
+    }
+};
+
+// A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`) for magnitudes of at most N words: both
+// operands in registers, every column's terms at static indexes, so that a product is its N (N + 1) / 2
+// multiply-adds and 2 N LDS reads (6.5 thousand cycles at N = 24; reading the operands term by term from
+// LDS took 38 thousand, more than the pivot chain that these updates run beside).
+template <int N>
+__device__ __forceinline__ void trail_update(const u32* xs, const u32* ys, int ta, int tb, int WL, int LF, u32* A,
+                                             bool add) {
+    if (ta >= N || tb >= N) {
+        trail_update_any(xs, ys, ta, tb, WL, LF, A, add);
+        return;
+    }
+    u32 x[N], y[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        x[i] = xs[i];
+        y[i] = ys[i];
+    }
+    u64 carry = 0;
+    u32 c = add ? 0u : 1u;                               // A + w, or A + ~w + 1
+    const u32 flip = add ? 0u : ~0u;
+    auto put = [&](int j, u32 w) {
+        const u64 q = (u64)A[j] + (w ^ flip) + c;
+        A[j] = (u32)q;
+        c = (u32)(q >> 32);
+    };
+    constexpr int K0 = N > 8 ? N - 9 : 0;                // N - 8 < LF <= N (LF <= 8: N = 8)
+    TrailColumns<N, K0>::run(x, y, LF, carry, put);
+    for (int j = 2 * N - 1 - LF; j < WL; j++) {
+        put(j, (u32)carry);
+        carry >>= 32;
+    }
+}
+
+// Pivot k: wave 0 computes r = d^-1/2 and d r (lane_rsqrt, lane_mulfx). Column scale: the waves take the
+// entries i > k, L_ik = mulfx(A_ik, r), and keep |L_ik|, its top word and its sign for the trailing
+// products; wave 0 takes entry k + 1 and updates the next diagonal entry with it, the other waves take
+// the rest. Trailing update over the other pairs k < j <= i: wave 0 goes on to pivot k + 1 (look-ahead)
+// while the other waves update the pairs, one per thread. Wave 0 runs the pivot's first Newton steps
+// while the others scale, so a step is bound by wave 0's chain of products alone (18: one scale, one
+// update, 16 for the pivot). N: words that hold every |L_ik| < 1 (N >= LF).
+// 1024 threads (four waves per SIMD): 960 for the trailing products. One 32 x 32 tile at L = 24 on one
+// MI355X: 0.334 ms (0.795 ms with products out of line and trailing operands read term by term from
+// LDS); k_tile_inverse 0.088 ms (0.200 ms).
+constexpr int NT = 1024;
+template <int N>
 __global__ void __launch_bounds__(NT) k_tile_chol_lds(u32* __restrict__ Wg, u32* __restrict__ Rg, int BT, int WL,
-                                                     int LF, int lane_pairs) {
+                                                     int LF) {
     constexpr int NW = NT / 64;
     SDPV_DYNAMIC_LDS(u32, lds);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const i64 tile = blockIdx.x;
     const int WS = WL | 1;
     const int ne = BT * (BT + 1) / 2;
@@ -680,11 +869,11 @@ __global__ void __launch_bounds__(NT) k_tile_chol_lds(u32* __restrict__ Wg, u32*
     u32* RK = CL + BT * WS;        // WL: r of the pivot
     u32* SG = RK + WL;             // BT: sign of L_ik
     u32* TP = SG + BT;             // BT: top word of |L_ik|
-    u32* PX = TP + BT + 128 * wave;  // 64 + 64 per wave: lane_mulfx operands
-    u32* PY = PX + 64;
+    u32* PB = TP + BT + LANE_LDS * wave;  // the wave's lane_mulfx operands
     u32* W = Wg + tile * BT * BT * WL;
     auto te = [&](int i, int j) { return T + (i64)(tri_base(i) + j) * WS; };
     const int total = BT * BT * WL;
+    const Lane Q(WL, LF, PB);
     // the lower triangle into LDS, 16 independent loads per thread in flight
     for (int base = tid; base < total; base += 16 * NT) {
         u32 v[16];
@@ -703,69 +892,70 @@ __global__ void __launch_bounds__(NT) k_tile_chol_lds(u32* __restrict__ Wg, u32*
         }
     }
     __syncthreads();
-    // pivot k on wave 0, from the (updated) diagonal entry d held one word per lane:
-    // r = d^-1/2, A_kk = mulfx(d, r), RINV_k = r
-    auto pivot = [&](int k, u32 d) {
-        const u32 r = lane_rsqrt(d, WL, LF, PX, PY);
-        const u32 dr = lane_mulfx(d, r, 0, WL, LF, PX, PY);
+    // pivot k on wave 0, from the (updated) diagonal entry d held one word per lane: r = d^-1/2,
+    // A_kk = mulfx(d, r), RINV_k = r; r0: the root after its first steps
+    auto pivot = [&](int k, const LaneMag& d, u32 r0) {
+        const u32 r = lane_rsqrt_finish(Q, d, r0);
+        const LaneMag rm = lane_mag(Q, r);
+        const u32 dr = lane_signed(Q, lane_mul<16>(Q, d, rm, 0), d.neg != rm.neg);
         if (lane < WL) {
             te(k, k)[lane] = dr;
             RK[lane] = r;
             Rg[(tile * BT + k) * WL + lane] = r;
         }
     };
-    if (wave == 0) pivot(0, lane < WL ? te(0, 0)[lane] : 0u);
+    if (wave == 0) {
+        const LaneMag d = lane_mag(Q, lane < WL ? te(0, 0)[lane] : 0u);
+        pivot(0, d, lane_rsqrt_begin(Q, d));
+    }
     __syncthreads();
     for (int k = 0; k < BT; k++) {
-        // column scale, entry i on wave (i - k - 1) mod NW: L_ik = mulfx(A_ik, r)
-        {
-            const u32 r = lane < WL ? RK[lane] : 0u;
-            for (int i = k + 1 + wave; i < BT; i += NW) {
-                u32* a = te(i, k);
-                const u32 lv = lane_mulfx(lane < WL ? a[lane] : 0u, r, 0, WL, LF, PX, PY);
-                const bool neg = (lane_get(lv, WL - 1) >> 31) != 0;
-                const u32 mag = neg ? lane_neg(lv, WL) : lv;
-                const int top = lane_top(mag, WL);
-                if (lane < WL) {
-                    a[lane] = lv;
-                    CL[(i64)i * WS + lane] = mag;
-                }
-                if (lane == 0) {
-                    SG[i] = neg;
-                    TP[i] = top;
-                }
+        // column scale: entry k + 1 on wave 0, which also updates the next diagonal entry (pair 0 of the
+        // trailing update); the other entries on the other waves in turn
+        const LaneMag rk = lane_mag(Q, lane < WL ? RK[lane] : 0u);
+        auto scale = [&](int i) {
+            u32* a = te(i, k);
+            const LaneMag x = lane_mag(Q, lane < WL ? a[lane] : 0u);
+            const u32 w = lane_mul<16>(Q, x, rk, 0);
+            const bool neg = x.neg != rk.neg;
+            const u32 lv = lane_signed(Q, w, neg);
+            LaneMag v{w, lane_top(w), neg};
+            if (v.top == WL - 1) v = lane_mag(Q, lv);    // the top bit of an overflowed product is a sign
+            if (lane < WL) {
+                a[lane] = lv;
+                CL[(i64)i * WS + lane] = v.m;
             }
+            if (lane == 0) {
+                SG[i] = v.neg;
+                TP[i] = v.top;
+            }
+            return v;
+        };
+        LaneMag dnext{0u, 0, false};
+        u32 rnext = 0u;
+        if (wave == 0) {
+            if (k + 1 < BT) {
+                const LaneMag v = scale(k + 1);
+                u32* dk = te(k + 1, k + 1);
+                dnext = lane_mag(Q, lane_add(Q, lane < WL ? dk[lane] : 0u, ~lane_mul<16>(Q, v, v, 0) & Q.in, 1u));
+                rnext = lane_rsqrt_begin(Q, dnext);
+            }
+        } else {
+            for (int i = k + 1 + wave; i < BT; i += NW - 1) scale(i);
         }
         __syncthreads();
         if (k == BT - 1) break;
-        // trailing update over the lower pairs k < j <= i: A_ij -= L_ik L_jk. Pair 0, the next
-        // diagonal entry, on wave 0, which then computes pivot k + 1 while the other waves update the
-        // other pairs (one per wave while there are at most `lane_pairs`, else one per thread)
+        // trailing update over the lower pairs k < j <= i (all but pair 0): A_ij -= L_ik L_jk, while wave 0
+        // finishes pivot k + 1
         const int m = BT - k - 1, npairs = m * (m + 1) / 2;
         if (wave == 0) {
-            const int r = k + 1;
-            const u32 x = lane < WL ? te(r, k)[lane] : 0u;
-            const u32 prod = lane_mulfx(x, x, 0, WL, LF, PX, PY);
-            const u32 d = lane_add(lane < WL ? te(r, r)[lane] : 0u, ~prod, 1u, WL);
-            if (lane < WL) te(r, r)[lane] = d;
-            pivot(r, d);
-        } else if (npairs - 1 <= lane_pairs) {
-            for (int p = wave; p < npairs; p += NW - 1) {
-                int ii, jj;
-                tri_pair(p, ii, jj);
-                const int r = k + 1 + ii, c = k + 1 + jj;
-                const u32 x = lane < WL ? te(r, k)[lane] : 0u, y = lane < WL ? te(c, k)[lane] : 0u;
-                const u32 prod = lane_mulfx(x, y, 0, WL, LF, PX, PY);
-                u32* aij = te(r, c);
-                const u32 nv = lane_add(lane < WL ? aij[lane] : 0u, ~prod, 1u, WL);
-                if (lane < WL) aij[lane] = nv;
-            }
+            pivot(k + 1, dnext, rnext);
         } else {
             for (int p = 1 + tid - 64; p < npairs; p += NT - 64) {
                 int ii, jj;
                 tri_pair(p, ii, jj);
                 const int r = k + 1 + ii, c = k + 1 + jj;
-                trail_update(CL + (i64)r * WS, CL + (i64)c * WS, TP[r], TP[c], WL, LF, te(r, c), SG[r] ^ SG[c]);
+                trail_update<N>(CL + (i64)r * WS, CL + (i64)c * WS, TP[r], TP[c], WL, LF, te(r, c), SG[r] != SG[c]);
             }
         }
         __syncthreads();
@@ -779,39 +969,38 @@ __global__ void __launch_bounds__(NT) k_tile_chol_lds(u32* __restrict__ Wg, u32*
 
 // words of k_tile_inverse's LDS for BT, WL and nw waves; the row prefetch takes BT WL <= 8 threads
 __host__ __device__ inline i64 lds_inverse_words(int BT, int WL, int nw) {
-    return 4 * (i64)BT * WL + (i64)nw * WL + 128 * nw;
+    return 4 * (i64)BT * WL + 2 * (i64)nw * WL + LANE_LDS * nw;
 }
 constexpr int INV_PRE = 8;  // words of the next row each thread prefetches
 
 // Column k of X = L^-1 for one tile (the recurrences of k_tile_factor's inverse):
 // x_kk = rinv_k; for i > k, x_ik = -mulfx(sum_{j=k}^{i-1} mulfx(l_ij, x_jk), rinv_i), every product
 // truncated, the sum exact (modulo 2^(32 WL)). Step i: the NT / 64 waves take the products j = k..i-1
-// in turn, one lane_mulfx each, and add them into a running lane sum; wave 0 adds the waves' sums
-// and finishes x_ik with one lane_mulfx. Row i + 1 of L is loaded while step i computes.
-// Grid (nb, BT), NT threads. X entries above the diagonal are written as zeros.
-template <int NT>
-__global__ void __launch_bounds__(NT) k_tile_inverse(const u32* __restrict__ Wg, const u32* __restrict__ Rg,
+// in turn and add them on the lanes, carries left pending; wave 0 adds the waves' sums, propagates the
+// carries once and finishes x_ik with one more product. Row i + 1 of L is loaded while step i computes.
+// Grid (nb, BT), INV_NT threads. X entries above the diagonal are written as zeros.
+constexpr int INV_NT = 512;
+__global__ void __launch_bounds__(INV_NT) k_tile_inverse(const u32* __restrict__ Wg, const u32* __restrict__ Rg,
                                                     u32* __restrict__ Xg, int BT, int WL, int LF) {
-    constexpr int NW = NT / 64;
+    constexpr int NW = INV_NT / 64;
     SDPV_DYNAMIC_LDS(u32, lds);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const i64 tile = blockIdx.x;
     const int k = blockIdx.y;
     u32* XT = lds;                      // BT x WL: x_jk
     u32* RI = XT + BT * WL;             // BT x WL: rinv
     u32* LR = RI + BT * WL;             // 2 x BT x WL: rows of L (slot j holds l_ij), double buffered
-    u32* PART = LR + 2 * BT * WL;       // NW x WL: the waves' partial sums
-    u32* PX = PART + NW * WL + 128 * wave;
-    u32* PY = PX + 64;
+    u32* PART = LR + 2 * BT * WL;       // NW x 2 WL: the waves' partial sums (low and high halves of 64 bits)
+    const Lane Q(WL, LF, PART + 2 * NW * WL + LANE_LDS * wave);
     const u32* W = Wg + tile * BT * BT * WL;
     const u32* R = Rg + tile * BT * WL;
     u32* X = Xg + tile * BT * BT * WL;
-    for (int idx = tid; idx < BT * WL; idx += NT) RI[idx] = R[idx];
+    for (int idx = tid; idx < BT * WL; idx += INV_NT) RI[idx] = R[idx];
     for (int i = 0; i < k; i++)
-        for (int q = tid; q < WL; q += NT) X[((i64)i * BT + k) * WL + q] = 0u;
+        for (int q = tid; q < WL; q += INV_NT) X[((i64)i * BT + k) * WL + q] = 0u;
     // row k + 1 into buffer 0 (entries j = k..k, at slot j)
     if (k + 1 < BT)
-        for (int idx = tid; idx < WL; idx += NT) LR[(i64)k * WL + idx] = W[((i64)(k + 1) * BT + k) * WL + idx];
+        for (int idx = tid; idx < WL; idx += INV_NT) LR[(i64)k * WL + idx] = W[((i64)(k + 1) * BT + k) * WL + idx];
     __syncthreads();
     if (wave == 0 && lane < WL) {       // x_kk = r_k
         const u32 r = RI[k * WL + lane];
@@ -828,27 +1017,36 @@ __global__ void __launch_bounds__(NT) k_tile_inverse(const u32* __restrict__ Wg,
         const u32* src = W + ((i64)(i + 1) * BT + k) * WL;
 #pragma unroll
         for (int u = 0; u < INV_PRE; u++) {
-            const int idx = tid + u * NT;
+            const int idx = tid + u * INV_NT;
             pre[u] = idx < nw ? src[idx] : 0u;
         }
-        // this wave's products, summed exactly
-        u32 acc = 0u;
+        // this wave's products, summed exactly: words of two's complement numbers in 64 bits per lane, the
+        // carries left for the end (a negative product adds its complement and one)
+        u64 acc = 0;
         for (int j = k + wave; j < i; j += NW) {
-            const u32 lij = lane < WL ? cur[j * WL + lane] : 0u;
-            const u32 xjk = lane < WL ? XT[j * WL + lane] : 0u;
-            acc = lane_add(acc, lane_mulfx(lij, xjk, 0, WL, LF, PX, PY), 0u, WL);
+            const LaneMag lij = lane_mag(Q, lane < WL ? cur[j * WL + lane] : 0u);
+            const LaneMag xjk = lane_mag(Q, lane < WL ? XT[j * WL + lane] : 0u);
+            const u32 w = lane_mul<16>(Q, lij, xjk, 0);
+            acc += lij.neg != xjk.neg ? (u64)(~w & Q.in) + (lane == 0 ? 1u : 0u) : (u64)w;
         }
-        if (lane < WL) PART[wave * WL + lane] = acc;
+        if (lane < WL) {
+            PART[2 * wave * WL + lane] = (u32)acc;
+            PART[(2 * wave + 1) * WL + lane] = (u32)(acc >> 32);
+        }
 #pragma unroll
         for (int u = 0; u < INV_PRE; u++) {
-            const int idx = tid + u * NT;
+            const int idx = tid + u * INV_NT;
             if (idx < nw) nxt[k * WL + idx] = pre[u];
         }
         __syncthreads();
         if (wave == 0) {
-            u32 sum = lane < WL ? PART[lane] : 0u;
-            for (int w = 1; w < NW; w++) sum = lane_add(sum, lane < WL ? PART[w * WL + lane] : 0u, 0u, WL);
-            const u32 x = lane_neg(lane_mulfx(sum, lane < WL ? RI[i * WL + lane] : 0u, 0, WL, LF, PX, PY), WL);
+            u64 part = 0;                // at most BT words below 2^33 in all
+            for (int w = 0; w < NW; w++)
+                if (lane < WL)
+                    part += ((u64)PART[(2 * w + 1) * WL + lane] << 32) + PART[2 * w * WL + lane];
+            const LaneMag sum = lane_mag(Q, lane_digits((u32)part, (u32)(part >> 32), 0u, ~0ull) & Q.in);
+            const LaneMag ri = lane_mag(Q, lane < WL ? RI[i * WL + lane] : 0u);
+            const u32 x = lane_signed(Q, lane_mul<16>(Q, sum, ri, 0), sum.neg == ri.neg);
             if (lane < WL) {
                 X[((i64)i * BT + k) * WL + lane] = x;
                 XT[i * WL + lane] = x;
@@ -924,35 +1122,17 @@ __global__ void __launch_bounds__(256) k_tile_narrow(const u32* __restrict__ W, 
 
 inline unsigned nblk(i64 n, int tpb) { return (unsigned)((n + tpb - 1) / tpb); }
 
-// trailing updates with at most this many pairs run one pair per wave (SDPV_TILE_LANE_PAIRS)
-inline int tile_lane_pairs() {
-    static const int v = [] {
-        const char* e = getenv("SDPV_TILE_LANE_PAIRS");
-        return e ? atoi(e) : 32;
-    }();
-    return v;
-}
-
-// threads per (tile, column) of the inverse: 512 unless SDPV_INV_THREADS is 256 or 1024
-inline int inverse_threads() {
-    static const int v = [] {
-        const char* e = getenv("SDPV_INV_THREADS");
-        const int t = e ? atoi(e) : 512;
-        return (t == 256 || t == 1024) ? t : 512;
-    }();
-    return v;
-}
-
-// threads of the LDS-resident factorisation: 1024 unless SDPV_TILE_THREADS is 256 or 512. Measured
-// at L = 24: chol(Q) of N = 3000 in 0.241 s with 256 threads, 0.203 s with 512 and 0.197 s with 1024
-// (all with the 512-thread inverse; 0.210 s with 512 and the 256-thread inverse).
-inline int tile_threads() {
-    static const int v = [] {
-        const char* e = getenv("SDPV_TILE_THREADS");
-        const int t = e ? atoi(e) : 1024;
-        return (t == 256 || t == 512) ? t : 1024;
-    }();
-    return v;
+// the factorisation for magnitudes of N words
+template <int N>
+int launch_factor(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, size_t lds, hipStream_t st) {
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<N>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        attr = true;
+    }
+    hipLaunchKernelGGL(k_tile_chol_lds<N>, dim3((unsigned)nb), dim3(NT), lds, st, W, RI, BT, WL, LF);
+    SDPV_TRY_LAUNCH();
+    return SDPV_OK;
 }
 
 }  // namespace
@@ -965,7 +1145,8 @@ int sdpv_tile_chol(const int32_t* A, int64_t L, int64_t nb, int64_t BT, int32_t*
     if (nb == 0) return SDPV_OK;
     if (!A || !Lout || !Xw || !work) return SDPV_EARG;
     const int WL = (int)L + 24;
-    const size_t lds = (size_t)2 * WL * TT * 4 + (size_t)(6 * WL + BT * WL + 2) * 4 + (size_t)2 * (2 * WL + 4) * 8;
+    const size_t lds = (size_t)2 * WL * TT * 4 + (size_t)(6 * WL + BT * WL + 2) * 4 + (size_t)2 * (2 * WL + 4) * 8 +
+                       (WL <= 64 ? LANE_LDS * 4 : 0);
     if (lds > 160 * 1024) return SDPV_ESIZE;
     hipStream_t st = as_stream(stream);
     const i64 n = nb * BT * BT;
@@ -978,39 +1159,22 @@ int sdpv_tile_chol(const int32_t* A, int64_t L, int64_t nb, int64_t BT, int32_t*
     static bool attr = false;
     if (!attr) {
         (void)hipFuncSetAttribute((const void*)k_tile_factor, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
-        (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<512>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
-        (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<1024>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
         attr = true;
     }
-    const int nt = tile_threads();
-    const size_t lds_f = (size_t)lds_factor_words((int)BT, WL, nt / 64) * 4;
-    const int ni = inverse_threads();
-    const size_t lds_i = (size_t)lds_inverse_words((int)BT, WL, ni / 64) * 4;
-    if (WL <= 64 && lds_f <= 160 * 1024 && BT * WL <= INV_PRE * 256) {
+    const size_t lds_f = (size_t)lds_factor_words((int)BT, WL, NT / 64) * 4;
+    const size_t lds_i = (size_t)lds_inverse_words((int)BT, WL, INV_NT / 64) * 4;
+    if (WL <= 64 && lds_f <= 160 * 1024 && BT * WL <= INV_PRE * INV_NT) {
         // the tile stays in LDS; the inverse one workgroup per column
-        if (nt == 1024)
-            hipLaunchKernelGGL(k_tile_chol_lds<1024>, dim3((unsigned)nb), dim3(1024), lds_f, st, W, RI, (int)BT, WL,
-                               (int)L, tile_lane_pairs());
-        else if (nt == 512)
-            hipLaunchKernelGGL(k_tile_chol_lds<512>, dim3((unsigned)nb), dim3(512), lds_f, st, W, RI, (int)BT, WL,
-                               (int)L, tile_lane_pairs());
-        else
-            hipLaunchKernelGGL(k_tile_chol_lds<256>, dim3((unsigned)nb), dim3(256), lds_f, st, W, RI, (int)BT, WL,
-                               (int)L, tile_lane_pairs());
-        SDPV_TRY_LAUNCH();
-        if (ni == 1024)
-            hipLaunchKernelGGL(k_tile_inverse<1024>, dim3((unsigned)nb, (unsigned)BT), dim3(1024), lds_i, st, W, RI,
-                               X, (int)BT, WL, (int)L);
-        else if (ni == 512)
-            hipLaunchKernelGGL(k_tile_inverse<512>, dim3((unsigned)nb, (unsigned)BT), dim3(512), lds_i, st, W, RI, X,
-                               (int)BT, WL, (int)L);
-        else
-            hipLaunchKernelGGL(k_tile_inverse<256>, dim3((unsigned)nb, (unsigned)BT), dim3(256), lds_i, st, W, RI, X,
-                               (int)BT, WL, (int)L);
+        const int rc = L <= 8 ? launch_factor<8>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
+                     : L <= 16 ? launch_factor<16>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
+                     : L <= 24 ? launch_factor<24>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
+                     : L <= 28 ? launch_factor<28>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
+                     : L <= 32 ? launch_factor<32>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
+                     : L <= 36 ? launch_factor<36>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
+                               : launch_factor<40>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st);
+        if (rc != SDPV_OK) return rc;
+        hipLaunchKernelGGL(k_tile_inverse, dim3((unsigned)nb, (unsigned)BT), dim3(INV_NT), lds_i, st, W, RI, X,
+                           (int)BT, WL, (int)L);
         SDPV_TRY_LAUNCH();
     } else {
         hipLaunchKernelGGL(k_tile_factor, dim3((unsigned)nb), dim3(TT), lds, st, W, X, S, RI, (int)BT, WL, (int)L);

@@ -31,6 +31,45 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 #define SDPV_WAIT_VMCNT(n) \
     __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
 #endif
+// Four multiply-adds into 96-bit accumulators acc + ov 2^64: v_mad_u64_u32 with its carry out taken by one
+// addition (the compiler forms the product with a zero addend and adds it in 64 bits twice). The four
+// multiplies go first, so that three instructions lie between a carry's write and its read (a VALU read of
+// an SGPR that a VALU wrote needs two wait states). CHAIN4: four terms a[u] b[u] of one sum; COLS4: one
+// factor x times y[u] into four sums; MAC96: one term alone. SETTLE(v, w): the wait states that a lane move of v or w needs after
+// such a block (the compiler does not see the block's instructions).
+#ifndef SDPV_MAC96_CHAIN4
+#define SDPV_MAC96_CHAIN4(acc, ov, a, b)                                                          \
+    do {                                                                                          \
+        u64 m0_, m1_, m2_, m3_;                                                                   \
+        asm("v_mad_u64_u32 %0, %2, %6, %10, %0\n\tv_mad_u64_u32 %0, %3, %7, %11, %0\n\t"          \
+            "v_mad_u64_u32 %0, %4, %8, %12, %0\n\tv_mad_u64_u32 %0, %5, %9, %13, %0\n\t"          \
+            "v_addc_co_u32 %1, %2, 0, %1, %2\n\tv_addc_co_u32 %1, %3, 0, %1, %3\n\t"              \
+            "v_addc_co_u32 %1, %4, 0, %1, %4\n\tv_addc_co_u32 %1, %5, 0, %1, %5"                  \
+            : "+v"(acc), "+v"(ov), "=&s"(m0_), "=&s"(m1_), "=&s"(m2_), "=&s"(m3_)                 \
+            : "v"((a)[0]), "v"((a)[1]), "v"((a)[2]), "v"((a)[3]), "v"((b)[0]), "v"((b)[1]),       \
+              "v"((b)[2]), "v"((b)[3]));                                                          \
+    } while (0)
+#define SDPV_MAC96_COLS4(acc, ov, x, y)                                                           \
+    do {                                                                                          \
+        u64 m0_, m1_, m2_, m3_;                                                                   \
+        asm("v_mad_u64_u32 %0, %8, %12, %13, %0\n\tv_mad_u64_u32 %1, %9, %12, %14, %1\n\t"        \
+            "v_mad_u64_u32 %2, %10, %12, %15, %2\n\tv_mad_u64_u32 %3, %11, %12, %16, %3\n\t"      \
+            "v_addc_co_u32 %4, %8, 0, %4, %8\n\tv_addc_co_u32 %5, %9, 0, %5, %9\n\t"              \
+            "v_addc_co_u32 %6, %10, 0, %6, %10\n\tv_addc_co_u32 %7, %11, 0, %7, %11"              \
+            : "+v"((acc)[0]), "+v"((acc)[1]), "+v"((acc)[2]), "+v"((acc)[3]), "+v"((ov)[0]),      \
+              "+v"((ov)[1]), "+v"((ov)[2]), "+v"((ov)[3]), "=&s"(m0_), "=&s"(m1_), "=&s"(m2_),    \
+              "=&s"(m3_)                                                                          \
+            : "v"(x), "v"((y)[0]), "v"((y)[1]), "v"((y)[2]), "v"((y)[3]));                        \
+    } while (0)
+#define SDPV_MAC96(acc, ov, a, b)                                                                 \
+    do {                                                                                          \
+        u64 m0_;                                                                                  \
+        asm("v_mad_u64_u32 %0, %2, %3, %4, %0\n\ts_nop 1\n\tv_addc_co_u32 %1, %2, 0, %1, %2"       \
+            : "+v"(acc), "+v"(ov), "=&s"(m0_)                                                     \
+            : "v"(a), "v"(b));                                                                    \
+    } while (0)
+#define SDPV_SETTLE(v, w) asm("s_nop 1" : "+v"(v), "+v"(w))
+#endif
 #define SDPV_TRY_LAUNCH()                                   \
     do {                                                    \
         hipError_t err__ = hipGetLastError();               \
@@ -52,6 +91,15 @@ __device__ __forceinline__ void swap_halves(u32& x, u32& y) {
     const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
     x = r[0];
     y = r[1];
+}
+
+// The value of the lane below (lane 0: zero) and of the lane above (lane 63: zero) of the wave: one
+// data-parallel move each, no LDS crossbar.
+__device__ __forceinline__ u32 lane_below(u32 v) {
+    return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xf, 0xf, true);   // wave_shr:1
+}
+__device__ __forceinline__ u32 lane_above(u32 v) {
+    return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);   // wave_shl:1
 }
 
 __device__ __forceinline__ int clz32(u32 x) { return __clz((int)x); }

@@ -88,9 +88,31 @@ inline emu_u2 __builtin_amdgcn_permlane32_swap(unsigned x, unsigned y, bool, boo
     const unsigned tx = (unsigned)emu_shfl_xor64((long long)x, 32), ty = (unsigned)emu_shfl_xor64((long long)y, 32);
     return (threadIdx.x & 63) < 32 ? emu_u2{{x, tx}} : emu_u2{{ty, y}};
 }
+// wave-wide moves by one lane (0x138: from the lane below, 0x130: from the lane above; lanes without a
+// source take `old`) and reads of one lane
+inline int __builtin_amdgcn_update_dpp(int old, int v, int ctrl, int, int, bool bound) {
+    const int l = (int)(threadIdx.x & 63), src = ctrl == 0x138 ? l - 1 : l + 1;
+    if (ctrl != 0x138 && ctrl != 0x130) abort();
+    const int r = (int)emu_shfl_idx64(v, src & 63);
+    return (src < 0 || src > 63) ? (bound ? 0 : old) : r;
+}
+inline int __builtin_amdgcn_readlane(int v, int src) { return (int)emu_shfl_idx64(v, src); }
+inline void emu_mac96(uint64_t& acc, uint32_t& ov, uint32_t a, uint32_t b) {
+    const unsigned __int128 p = (unsigned __int128)acc + (uint64_t)a * b;
+    acc = (uint64_t)p;
+    ov += (uint32_t)(p >> 64);
+}
+#define SDPV_MAC96(acc, ov, a, b) emu_mac96((acc), (ov), (a), (b))
+#define SDPV_MAC96_CHAIN4(acc, ov, a, b) \
+    for (int emu_u = 0; emu_u < 4; emu_u++) emu_mac96((acc), (ov), (a)[emu_u], (b)[emu_u])
+#define SDPV_MAC96_COLS4(acc, ov, x, y) \
+    for (int emu_u = 0; emu_u < 4; emu_u++) emu_mac96((acc)[emu_u], (ov)[emu_u], (x), (y)[emu_u])
+#define SDPV_SETTLE(v, w) ((void)(v), (void)(w))
 void emu_wave_barrier();
 unsigned long long emu_ballot(int pred);
 #define __ballot(p) emu_ballot((int)(p))
+#define __builtin_amdgcn_ballot_w64(p) emu_ballot((int)(p))
+#define __builtin_amdgcn_inverse_ballot_w64(m) ((((unsigned long long)(m)) >> (threadIdx.x & 63)) & 1)
 inline unsigned __builtin_amdgcn_perm(unsigned s0, unsigned s1, unsigned sel) {
     unsigned long long v = ((unsigned long long)s0 << 32) | s1;   // bytes 0-3 from s1, 4-7 from s0
     unsigned r = 0;
