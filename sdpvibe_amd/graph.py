@@ -6,6 +6,8 @@ C ABI and never synchronises with the host, so a whole call such as mpf.gemm can
 and replayed: the replay re-runs the same kernels on the same buffers with no host work and no
 launch gaps. Inputs are updated in place (copy_ into the captured tensors) between replays.
 """
+import gc
+
 import torch
 
 
@@ -23,8 +25,16 @@ class Captured:
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            self.out = fn(*args)
+        # no cyclic garbage collection while capturing: it may destroy another object's graph (a solver that
+        # went out of use), whose destructor synchronises the device, which a capture forbids
+        collecting = gc.isenabled()
+        gc.disable()
+        try:
+            with torch.cuda.graph(self.graph):
+                self.out = fn(*args)
+        finally:
+            if collecting:
+                gc.enable()
 
     def replay(self):
         self.graph.replay()
