@@ -78,8 +78,8 @@ int sdpv_badd_align(const int32_t* A, const int32_t* Bm, const int64_t* EA, cons
  * operands (limb u of A[b, i, k] at A[u * planeA + b * ldAb + i * ldAr + k * ldAk], likewise B),
  * written exactly as NW >= 2L + 2 words W[w * E + e] (E = nb * M * N), with its bit length (of ~S
  * when S < 0) in bitlen[e]: the words and bit lengths that sdpv_rns_crt's word mode returns for the
- * same product. K beyond 256 is split over waves, whose column sums go through `work`
- * (sdpv_exact_dot_work(...) int64 entries; 0 when K <= 256). No counterpart in the reference, which
+ * same product. K is split into slices whose sums go through `work` (sdpv_exact_dot_work(...) int64
+ * entries, 0 when there is one slice of at most 32 rows). No counterpart in the reference, which
  * always goes through residues: the direct path for products with one or two right-hand-side
  * columns (triangular solves with one vector), where the residue path's fixed costs dominate.
  * L <= 63. */
@@ -109,6 +109,46 @@ int sdpv_mpf_add(const int32_t* A, const int64_t* eA, const int32_t* Bm, const i
  * Replaces mpf.normalize / mpf_norm (sdpvibe/mpf.py:307-313, :127-140). */
 int sdpv_mpf_norm(const int32_t* X, const int64_t* eI, int64_t LI, int32_t* O, int64_t* eO,
                   int64_t L, int64_t n, void* stream);
+
+/* The same exact products with the operands rounded on the way in and the result on the way out.
+ * eA / eB non-null: entry (b, i, k) of A is first rounded to its row exponent, shift_round by
+ * EA[b * M + i] - eA[entry] (zero entries, e == SDPV_EZ, to zero), entry (b, j, k) of B by
+ * EB[b * N + j] - eB[entry]; null: the limbs as they are. K <= 2^17, L <= 63. Output limb w of entry
+ * (b, i, j) goes to out[w * plane + b * ob + i * oi + j * oj]. The exponent of a product is
+ * e0 + ea[b * lea] + eb[b * N + j] (null arrays count as 0). mode:
+ *   SDPV_NARROW_NORMALIZE  normalised entries (as sdpv_rns_crt's NORMALIZE), exponents
+ *                          EA + EB + shift in oute at the same offset;
+ *   SDPV_NARROW_FIXED      rounded to the exponent oexp;
+ *   SDPV_NARROW_COL        every column (b, j) rounded to 32 L - 32 bits below its largest bit length; with
+ *                          X (limbs at X[w * planeX + b * xb + i * xi + j * xj], column exponents
+ *                          eX (nb, N)) the result is X + sgn * product, both rounded to one above the larger
+ *                          exponent as sdpv_badd_align does. Column exponents in oute (nb, N);
+ *   SDPV_NARROW_ACC        the exact 2L + 2 words added to out[e * (2L + 2) + w], e = (b M + i) N + j (plane
+ *                          and strides unused); sdpv_narrow_result normalises such sums.
+ * flag: optional, set when a FIXED or COL rounding overflows. work: sdpv_exact_dot_work(...) int64
+ * entries. Replaces, for a few columns, the residue path under mpf.gemm, batched.bgemm_nt and badd
+ * (sdpvibe/mpf.py:401-452, sdpvibe/batched.py:56-79, 165-231). */
+#define SDPV_NARROW_NORMALIZE 1
+#define SDPV_NARROW_FIXED 2
+#define SDPV_NARROW_COL 3
+#define SDPV_NARROW_ACC 4
+int sdpv_narrow(const int32_t* A, const int64_t* eA, const int64_t* EA, int64_t planeA, int64_t ldAb,
+                int64_t ldAr, int64_t ldAk, const int32_t* B, const int64_t* eB, const int64_t* EB,
+                int64_t planeB, int64_t ldBb, int64_t ldBr, int64_t ldBk, int64_t L, int64_t nb, int64_t M,
+                int64_t N, int64_t K, int32_t mode, int32_t* out, int64_t plane, int64_t ob, int64_t oi,
+                int64_t oj, int64_t* oute, int64_t e0, const int64_t* ea, int64_t lea, const int64_t* eb,
+                int64_t oexp, const int32_t* X, int64_t planeX, int64_t xb, int64_t xi, int64_t xj,
+                const int64_t* eX, int32_t sgn, int32_t* flag, int64_t* work, int64_t nwork, void* stream);
+int sdpv_narrow_result(const int32_t* acc, int64_t L, int64_t nb, int64_t M, int64_t N, const int64_t* EA,
+                       const int64_t* EB, int32_t* out, int64_t plane, int64_t ob, int64_t oi, int64_t oj,
+                       int64_t* oute, void* stream);
+
+/* [P1; P2] with one exponent per (block, column): P1 (L, nb, R1, C) and P2 (L, nb, R2, C) with column
+ * exponents e1, e2 (nb, C), both rounded (shift_round) to EO = max(e1, e2) and written into one
+ * (L, nb, R1 + R2, C) array. flag: optional int32, set when a rounding overflows. */
+int sdpv_stack_common(const int32_t* P1, const int64_t* e1, const int32_t* P2, const int64_t* e2, int32_t* out,
+                      int64_t* EO, int64_t L, int64_t nb, int64_t R1, int64_t R2, int64_t C, int32_t* flag,
+                      void* stream);
 
 /* ---------------------------------------------------------------- exact RNS GEMM */
 

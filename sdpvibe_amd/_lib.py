@@ -25,6 +25,10 @@ SIGNATURES = {
     "sdpv_exact_dot_work": ([_I64, _I64, _I64, _I64, _I64], _I64),
     "sdpv_exact_dot": ([_P, _I64, _I64, _I64, _I64, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P,
                         _I64, _P, _P, _I64, _P], _I32),
+    "sdpv_narrow": ([_P] * 3 + [_I64] * 4 + [_P] * 3 + [_I64] * 4 + [_I64] * 5 + [_I32, _P] + [_I64] * 4 + [_P, _I64, _P, _I64,
+                     _P, _I64, _P] + [_I64] * 4 + [_P, _I32, _P, _P, _I64, _P], _I32),
+    "sdpv_narrow_result": ([_P, _I64, _I64, _I64, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P], _I32),
+    "sdpv_stack_common": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P], _I32),
     "sdpv_mpf_top": ([_P, _P, _I64, _I64, _P, _P], _I32),
     "sdpv_mpf_mul": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I32, _P], _I32),
     "sdpv_mpf_add": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I32, _P], _I32),

@@ -11,7 +11,7 @@ array instead of being concatenated level by level.
 """
 import torch
 
-from ._lib import call, lib, ptr, ptr_strided, stream
+from ._lib import call, lib, ptr, stream
 from .limbops import _errbuf, add_same, shift_round
 from .mpmat import ctx, headroom_bits, residue_gemm
 from .rns import dev
@@ -130,13 +130,18 @@ def bgemm_nt(A, Bt, out_exp="col", kc=4096, bt_rowexp=None, bt_cache=None):
     assert nb == nb2 and K == K2
     L = A.L
     R = ctx(L)
+    eB = Bt.exp if bt_rowexp is None else bt_rowexp
+    if _narrow(M, N, K, L):
+        C = _narrow_product(A, Bt, eB, out_exp if isinstance(out_exp, int) else "col")
+        if out_exp == "mat":
+            C = brescale(C, C.exp.amax(1, keepdim=True).expand(nb, N).contiguous())
+        return C
     eA = A.exp if isinstance(A.exp, int) else A.exp[:, 0]
     cache = {}
-    if not _narrow(M, N, K, L):
-        Al, Bl = A.limbs, Bt.limbs                  # views are read through their strides
-        same = Al.data_ptr() == Bl.data_ptr() and Al.stride() == Bl.stride() and Al.shape == Bl.shape
-        fa = _residue_desc(R, Al, nb, M, K)
-        fb = _residue_desc(R, Bl, nb, N, K)
+    Al, Bl = A.limbs, Bt.limbs                      # views are read through their strides
+    same = Al.data_ptr() == Bl.data_ptr() and Al.stride() == Bl.stride() and Al.shape == Bl.shape
+    fa = _residue_desc(R, Al, nb, M, K)
+    fb = _residue_desc(R, Bl, nb, N, K)
 
     def fa0(k0, kc_, kp, j0, jw):
         cache["a"] = fa(k0, kc_, kp, None, None)
@@ -152,9 +157,8 @@ def bgemm_nt(A, Bt, out_exp="col", kc=4096, bt_rowexp=None, bt_cache=None):
             bt_cache[key] = fb(k0, kc_, kp, j0, jw)
         return bt_cache[key]
 
-    eB = Bt.exp if bt_rowexp is None else bt_rowexp
     out = torch.empty((L, nb, M, N), dtype=torch.int32, device=dev)
-    if isinstance(out_exp, int) and not _narrow(M, N, K, L):
+    if isinstance(out_exp, int):
         # a fixed output exponent: the reconstruction rounds by per-(block, column) shifts alone
         s = _fixed_shift(eA, eB, out_exp, nb, N, bt_cache)
         for j0, jw, acc in residue_gemm(R, fa0, fb0, nb, M, N, K):
@@ -169,64 +173,70 @@ def bgemm_nt(A, Bt, out_exp="col", kc=4096, bt_rowexp=None, bt_cache=None):
         if eB_t.dim() == 1:
             eB_t = eB_t[:, None].expand(nb, N)
         e_in = (eA_t[:, None] + eB_t).contiguous()
-    exps = None if isinstance(out_exp, int) else torch.empty((nb, N), dtype=torch.int64, device=dev)
-    if _narrow(M, N, K, L):
-        W, bl = _exact_narrow(A.limbs, Bt.limbs, nb, M, N, K, L)
-        _round_exact(W, bl, nb, M, N, e_in, out_exp, L, out, exps)
-    else:
-        for j0, jw, acc in residue_gemm(R, fa0, fb0, nb, M, N, K):
-            _bcrt_round_panel(R, acc, nb, M, N, j0, jw, e_in, out_exp, L, out, exps)
-    if isinstance(out_exp, int):
-        return BMP(out, out_exp)
+    exps = torch.empty((nb, N), dtype=torch.int64, device=dev)
+    for j0, jw, acc in residue_gemm(R, fa0, fb0, nb, M, N, K):
+        _bcrt_round_panel(R, acc, nb, M, N, j0, jw, e_in, out_exp, L, out, exps)
     C = BMP(out, exps)
     if out_exp == "mat":
         C = brescale(C, exps.amax(1, keepdim=True).expand(nb, N).contiguous())
     return C
 
 
-# products with at most NARROW right-hand-side columns and at most NARROW_MK rows times inner length
-# are formed directly (sdpv_exact_dot); larger ones go through residues, which are faster there
-# (one MI355X, L = 24, one column, M x K: direct 0.084 / 0.104 / 0.106 / 0.164 ms against residues
-# 0.135 / 0.134 / 0.132 / 0.135 ms at 32 x 32, 188 x 188, 32 x 1504, 375 x 375)
+# products with at most NARROW right-hand-side columns and at most NARROW_MK rows times inner length are
+# formed directly (sdpv_narrow): the matrix is read once and multiplied as bytes, where the residue path
+# reduces each of its entries modulo every prime. One MI355X, L = 24, one column: 60 blocks of 162 x 3000
+# in 1.55 ms against 5.83 ms; 32 x 32 in 0.022 ms against 0.135 ms
 NARROW = 2
-NARROW_MK = 65536
+NARROW_MK = 1 << 40
+NARROW_K = 1 << 17                             # inner dimension of one direct product
 
 
 def _narrow(M, N, K, L):
-    return N <= NARROW and M * K <= NARROW_MK and L <= 63
+    return N <= NARROW and M * K <= NARROW_MK and K <= NARROW_K and L <= 63
 
 
-def _exact_narrow(Al, Bl, nb, M, N, K, L):
-    """the exact products of (L, nb, M, K) and (L, nb, N, K) limb tensors (views with unit stride
-    along k are read in place) as 2L + 2 words per entry (entry (b*M + i)*N + j) and bit lengths:
-    what the reconstruction's word mode gives for the same product"""
-    Al = Al if Al.stride(-1) == 1 else Al.contiguous()
-    Bl = Bl if Bl.stride(-1) == 1 else Bl.contiguous()
-    NW, E = 2 * L + 2, nb * M * N
-    W = torch.empty((NW, E), dtype=torch.int32, device=Al.device)
-    bl = torch.empty((E,), dtype=torch.int64, device=Al.device)
-    nwork = int(lib().sdpv_exact_dot_work(L, nb, M, N, K))
-    work = torch.empty((max(nwork, 1),), dtype=torch.int64, device=Al.device)
+def flat_view(X):
+    """the storage of a view with non-negative strides from its first entry to its last, as a contiguous
+    1-d tensor (for entry points that take base pointer and strides)"""
+    if X.numel() == 0:
+        return X.reshape(-1)
+    return torch.as_strided(X, (sum((n - 1) * s for n, s in zip(X.shape, X.stride())) + 1,), (1,))
+
+
+def narrow_work(L, nb, M, N, K, device):
+    """scratch of sdpv_narrow for this shape: (tensor, int64 entries)"""
+    n = int(lib().sdpv_exact_dot_work(L, nb, M, N, K))
+    return torch.empty((max(n, 1),), dtype=torch.int64, device=device), n
+
+
+def _narrow_product(A, Bt, eB, out_exp, plus=None, sgn=1):
+    """A Bt^T with few rows of Bt as one direct product, rounded to the int out_exp or per (block,
+    column) ('col'); plus: a BMP X (possibly a view), the result is then badd(X, A Bt^T, sgn, 'align')"""
+    nb, M, K = A.shape
+    N, L = Bt.shape[1], A.L
+    Al, Bl = A.limbs, Bt.limbs
     sa, sb = Al.stride(), Bl.stride()
-    call("sdpv_exact_dot", ptr_strided(Al), sa[0], sa[1], sa[2], sa[3], ptr_strided(Bl), sb[0], sb[1], sb[2], sb[3],
-         L, nb, M, N, K, ptr(W), NW, ptr(bl), ptr(work), nwork, stream())
-    return W, bl
-
-
-def _round_exact(W, bl, nb, M, N, e_in, out_exp, L, out, exps):
-    """the roundings of _bcrt_round_panel on exact words: a fixed output exponent, or per
-    (block, column) headroom_bits(L) below the column's largest bit length"""
-    if isinstance(out_exp, int):
-        if isinstance(e_in, int):
-            s = torch.full((nb * M * N,), out_exp - e_in, dtype=torch.int64, device=dev)
-        else:
-            s = (out_exp - e_in)[:, None, :].expand(nb, M, N).reshape(-1).contiguous()
+    out = torch.empty((L, nb, M, N), dtype=torch.int32, device=Al.device)
+    e0, ea, lea, eb = 0, None, 0, None
+    if isinstance(A.exp, int):
+        e0 += A.exp
     else:
-        ein = e_in if torch.is_tensor(e_in) else torch.full((nb, N), e_in, dtype=torch.int64, device=dev)
-        sj = bl.view(nb, M, N).amax(1) - headroom_bits(L)
-        exps[:, :] = ein + sj
-        s = sj[:, None, :].expand(nb, M, N).reshape(-1).contiguous()
-    shift_round(W, s, L, out=out.view(L, nb * M * N))
+        ea = A.exp.contiguous()                # (nb, C), read at column 0
+        lea = ea.shape[1]
+    if isinstance(eB, int):
+        e0 += eB
+    else:
+        eb = (eB[:, None].expand(nb, N) if eB.dim() == 1 else eB).contiguous()
+    fixed = isinstance(out_exp, int)
+    exps = None if fixed else torch.empty((nb, N), dtype=torch.int64, device=Al.device)
+    X, sx, eX = None, (0, 0, 0, 0), None
+    if plus is not None:
+        X, sx, eX = flat_view(plus.limbs), plus.limbs.stride(), plus.expt().contiguous()
+    work, nwork = narrow_work(L, nb, M, N, K, Al.device)
+    call("sdpv_narrow", ptr(flat_view(Al)), None, None, *sa, ptr(flat_view(Bl)), None, None, *sb, L, nb, M, N, K,
+         2 if fixed else 3, ptr(out), nb * M * N, M * N, N, 1, ptr(exps), e0, ptr(ea), lea, ptr(eb),
+         out_exp if fixed else 0, ptr(X), *sx, ptr(eX), sgn, ptr(_errbuf()), ptr(work), nwork, stream())
+    return BMP(out, out_exp if fixed else exps)
 
 
 def _fixed_shift(eA, eB, out_exp, nb, N, cache=None):
@@ -403,8 +413,23 @@ def _apply_tile(X, Lm, B, refine):
 
 def _stack_common(P1, P2):
     """[P1; P2] with one exponent per (block, column): both parts re-rounded to the larger"""
-    ee = torch.maximum(P1.expt(), P2.expt())
-    return BMP(torch.cat([brescale(P1, ee, share_exp=True).limbs, brescale(P2, ee, share_exp=True).limbs], 2), ee)
+    nb, R1, C = P1.shape
+    R2, L = P2.shape[1], P1.L
+    out = torch.empty((L, nb, R1 + R2, C), dtype=torch.int32, device=P1.limbs.device)
+    ee = torch.empty((nb, C), dtype=torch.int64, device=P1.limbs.device)
+    m1, e1, m2, e2 = (x.contiguous() for x in (P1.limbs, P1.expt(), P2.limbs, P2.expt()))
+    call("sdpv_stack_common", ptr(m1), ptr(e1), ptr(m2), ptr(e2), ptr(out), ptr(ee), L, nb, R1, R2, C, ptr(_errbuf()),
+         stream())
+    return BMP(out, ee)
+
+
+def _minus_product(X, A, P):
+    """badd(X, A P, -1, 'align'): rows X of a right-hand side less a block of the factor times the part
+    already solved; one direct product with few columns"""
+    nb, M, K = A.shape
+    if _narrow(M, P.shape[2], K, A.L):
+        return _narrow_product(A, _as_rows(P), P.expt(), "col", plus=X, sgn=-1)
+    return badd(X, bgemm_nt(A, _as_rows(P), out_exp="col", bt_rowexp=P.expt()), -1, out_exp="align")
 
 
 def _view(A, rows, cols, transpose=False):
@@ -426,14 +451,12 @@ def _left_solve(node, Lf, B, tiles, refine, upper):
     head, tail = slice(None, k), slice(k, None)
     if not upper:
         P1 = _left_solve(node.head, _view(Lf, head, head), _rows(B, 0, k), tiles, refine, upper)
-        coupled = bgemm_nt(_view(Lf, tail, head), _as_rows(P1), out_exp="col", bt_rowexp=P1.expt())
-        P2 = _left_solve(node.tail, _view(Lf, tail, tail), badd(_rows(B, k), coupled, -1, out_exp="align"), tiles,
+        P2 = _left_solve(node.tail, _view(Lf, tail, tail), _minus_product(_rows(B, k), _view(Lf, tail, head), P1), tiles,
                          refine, upper)
     else:
         P2 = _left_solve(node.tail, _view(Lf, tail, tail), _rows(B, k), tiles, refine, upper)
-        coupled = bgemm_nt(_view(Lf, tail, head, transpose=True), _as_rows(P2), out_exp="col", bt_rowexp=P2.expt())
-        P1 = _left_solve(node.head, _view(Lf, head, head), badd(_rows(B, 0, k), coupled, -1, out_exp="align"), tiles,
-                         refine, upper)
+        P1 = _left_solve(node.head, _view(Lf, head, head),
+                         _minus_product(_rows(B, 0, k), _view(Lf, tail, head, transpose=True), P2), tiles, refine, upper)
     return _stack_common(P1, P2)
 
 

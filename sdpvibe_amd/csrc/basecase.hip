@@ -277,9 +277,7 @@ __device__ void wave_rsqrt(const Pivot& P) {
 // once per product, and the lane lookahead and the products are always inlined (out of line their LDS
 // operands turn into flat accesses). The product took 2300 cycles out of line with its lane exchanges
 // through the LDS crossbar.
-__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ u32 lane_get(u32 v, int src) { return (u32)__shfl((int)v, src, 64); }
-__device__ __forceinline__ u32 lane_read(u32 v, int src) { return (u32)__builtin_amdgcn_readlane((int)v, src); }
 __device__ __forceinline__ u64 lane_get64(u64 v, int src) {
     return ((u64)lane_get((u32)(v >> 32), src) << 32) | lane_get((u32)v, src);
 }
@@ -289,9 +287,6 @@ __device__ __forceinline__ u64 from_below64(u64 v) {
     const u64 r = lane_get64(v, l > 0 ? l - 1 : 0);
     return l > 0 ? r : 0;
 }
-__device__ __forceinline__ u64 ballot64(bool p) { return __builtin_amdgcn_ballot_w64(p); }
-// 1 in the lanes of the mask m (uniform)
-__device__ __forceinline__ u32 mask_bit(u64 m) { return __builtin_amdgcn_inverse_ballot_w64(m) ? 1u : 0u; }
 
 // LDS words of one wave's products: the left magnitude with zeros above, the right one with zeros on both
 // sides (column c reads word c - i for every term i). Terms are read in groups that reach up to 32 past the

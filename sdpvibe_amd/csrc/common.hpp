@@ -101,6 +101,12 @@ __device__ __forceinline__ u32 lane_below(u32 v) {
 __device__ __forceinline__ u32 lane_above(u32 v) {
     return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);   // wave_shl:1
 }
+__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+// the value of lane src (uniform)
+__device__ __forceinline__ u32 lane_read(u32 v, int src) { return (u32)__builtin_amdgcn_readlane((int)v, src); }
+__device__ __forceinline__ u64 ballot64(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+// 1 in the lanes of the mask m (uniform)
+__device__ __forceinline__ u32 mask_bit(u64 m) { return __builtin_amdgcn_inverse_ballot_w64(m) ? 1u : 0u; }
 
 __device__ __forceinline__ int clz32(u32 x) { return __clz((int)x); }
 

@@ -101,6 +101,24 @@ __global__ void __launch_bounds__(TPB) k_badd_align(const i32* __restrict__ A, c
     if ((e / cols) % rows == 0) EO[col] = ex;
 }
 
+// both parts of a stacked solve re-rounded to their columns' larger exponent and joined, one pass (a
+// rounding each, a broadcast shift per entry and a concatenation took seven launches)
+__global__ void __launch_bounds__(TPB) k_stack_common(const i32* __restrict__ P1, const i64* __restrict__ E1,
+                                                      const i32* __restrict__ P2, const i64* __restrict__ E2,
+                                                      i32* __restrict__ O, i64* __restrict__ EO, int L, i64 nb, i64 R1,
+                                                      i64 R2, i64 C, i32* __restrict__ flag) {
+    const i64 e = blockIdx.x * (i64)TPB + threadIdx.x, R = R1 + R2, n = nb * R * C;
+    if (e >= n) return;
+    const i64 c = e % C, r = e / C % R, b = e / (C * R), col = b * C + c;
+    const i64 ea = E1[col], eb = E2[col], ex = ea > eb ? ea : eb;
+    const bool up = r < R1;
+    const i64 n1 = nb * R1 * C, n2 = nb * R2 * C;
+    const PlaneSrc src = up ? PlaneSrc{P1 + (b * R1 + r) * C + c, n1} : PlaneSrc{P2 + (b * R2 + r - R1) * C + c, n2};
+    const int bad = shr_round_batched(src, L, ex - (up ? ea : eb), L, [&](int k, u32 w) { O[(i64)k * n + e] = (i32)w; });
+    if (bad && flag) atomicOr(flag, 1);
+    if (r == 0) EO[col] = ex;
+}
+
 // ------------------------------------------------------------------ mpf_norm (mpf.py:127-140)
 __global__ void __launch_bounds__(TPB) k_mpf_norm(const i32* __restrict__ X, const i64* __restrict__ eI, int LI,
                                                   i32* __restrict__ O, i64* __restrict__ eO, int L, i64 n) {
@@ -453,6 +471,19 @@ int sdpv_badd_align(const int32_t* A, const int32_t* Bm, const int64_t* EA, cons
     if (!A || !Bm || !EA || !EB || !out || !EO) return SDPV_EARG;
     hipLaunchKernelGGL(k_badd_align, dim3(nblocks(entries, TPB)), dim3(TPB), 0, as_stream(stream), A, Bm, EA, EB,
                        out, EO, (int)L, entries, (i64)rows, (i64)cols, (int)(sgn < 0));
+    SDPV_TRY_LAUNCH();
+    return SDPV_OK;
+}
+
+int sdpv_stack_common(const int32_t* P1, const int64_t* e1, const int32_t* P2, const int64_t* e2, int32_t* out,
+                      int64_t* EO, int64_t L, int64_t nb, int64_t R1, int64_t R2, int64_t C, int32_t* flag,
+                      void* stream) {
+    if (L < 1 || nb < 0 || R1 < 1 || R2 < 1 || C < 0) return SDPV_EARG;
+    const i64 n = nb * (R1 + R2) * C;
+    if (n == 0) return SDPV_OK;
+    if (!P1 || !P2 || !e1 || !e2 || !out || !EO) return SDPV_EARG;
+    hipLaunchKernelGGL(k_stack_common, dim3(nblocks(n, TPB)), dim3(TPB), 0, as_stream(stream), P1, e1, P2, e2, out, EO,
+                       (int)L, (i64)nb, (i64)R1, (i64)R2, (i64)C, flag);
     SDPV_TRY_LAUNCH();
     return SDPV_OK;
 }

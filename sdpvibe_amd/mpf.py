@@ -15,6 +15,7 @@ import mpmath as mp
 import numpy as np
 import torch
 
+from . import batched as _batched
 from ._lib import call, ptr, stream
 from .limbops import bitlen_words, shift_round
 from .mpmat import RES_BUDGET, ctx, residue_gemm
@@ -370,6 +371,16 @@ def gemm(A, B, transA=False, transB=False):
     if nb * M * N == 0:
         return MPF(out_m, out_e)
 
+    if _batched._narrow(max(M, N), min(M, N), K, L):
+        # one side has few rows: the direct product, the other side read once as it is stored
+        work, nwork = _batched.narrow_work(L, nb, max(M, N), min(M, N), K, out_m.device)
+        opA = (ptr(Am), ptr(Ae), ptr(EA), Ae.numel(), aldb, aldr, aldk)
+        opB = (ptr(Bm), ptr(Be), ptr(EB), Be.numel(), bldb, bldr, bldk)
+        first, second, oi, oj = (opA, opB, N, 1) if N <= M else (opB, opA, 1, N)
+        call("sdpv_narrow", *first, *second, L, nb, max(M, N), min(M, N), K, 1, ptr(out_m), nb * M * N, M * N, oi, oj,
+             ptr(out_e), 0, None, 0, None, 0, None, 0, 0, 0, 0, None, 1, None, ptr(work), nwork, stream())
+        return MPF(out_m, out_e)
+
     def fa(k0, kc, kp, j0, jw):
         Rh = torch.empty((R.n, kp // 16, nb * M, 16), dtype=torch.int8, device=dev)
         Rl = torch.empty_like(Rh)
@@ -414,7 +425,12 @@ class KSum:
         self.M, self.N = EA.numel(), EB.numel()
         self.R = ctx(L)
         self.K = 0
-        self.acc = torch.zeros((self.R.n, self.M, self.N), dtype=torch.int16, device=dev)
+        # few columns: the exact words of every entry's sum (direct products), else its residues
+        self.direct = _batched._narrow(self.M, self.N, 0, L)
+        if self.direct:
+            self.acc = torch.zeros((self.M * self.N, 2 * L + 2), dtype=torch.int32, device=dev)
+        else:
+            self.acc = torch.zeros((self.R.n, self.M, self.N), dtype=torch.int16, device=dev)
 
     def add(self, A, B):
         R, L, M, N = self.R, self.L, self.M, self.N
@@ -424,6 +440,14 @@ class KSum:
         if self.K + K > R.kmax:
             raise ValueError(f"KSum: inner dimension {self.K + K} exceeds the RNS bound {R.kmax}")
         Am, Ae, Bm, Be = A.m.contiguous(), A.e.contiguous(), B.m.contiguous(), B.e.contiguous()
+        if self.direct:                          # K is within sdpv_narrow's bound: it is the RNS bound above
+            if K and M and N:
+                work, nwork = _batched.narrow_work(L, 1, M, N, K, Am.device)
+                call("sdpv_narrow", ptr(Am), ptr(Ae), ptr(self.EA), K * M, K * M, 1, M, ptr(Bm), ptr(Be), ptr(self.EB),
+                     K * N, K * N, 1, N, L, 1, M, N, K, 4, ptr(self.acc), 0, 0, 0, 0, None, 0, None, 0, None, 0, None, 0, 0, 0,
+                     0, None, 1, None, ptr(work), nwork, stream())
+            self.K += K
+            return
         per_k = 2 * R.n * (M + N) * 2
         kc = max(64, min(KMAX_LAUNCH, RES_BUDGET // max(per_k, 1) // 64 * 64))
         for k0 in range(0, K, kc):
@@ -445,8 +469,12 @@ class KSum:
         L, M, N = self.L, self.M, self.N
         out_m = torch.empty((L, 1, M, N), dtype=torch.int32, device=dev)
         out_e = torch.empty((1, M, N), dtype=torch.int64, device=dev)
-        self.R.crt(self.acc, M, N, 0, N, 1, outm=out_m, oute=out_e, L=L, plane=M * N, ldo=N, jo=0, Mb=M,
-                   erow=self.EA, ecol=self.EB, scaled=True)
+        if self.direct:
+            call("sdpv_narrow_result", ptr(self.acc), L, 1, M, N, ptr(self.EA), ptr(self.EB), ptr(out_m), M * N, M * N, N, 1,
+                 ptr(out_e), stream())
+        else:
+            self.R.crt(self.acc, M, N, 0, N, 1, outm=out_m, oute=out_e, L=L, plane=M * N, ldo=N, jo=0, Mb=M,
+                       erow=self.EA, ecol=self.EB, scaled=True)
         return MPF(out_m[:, 0], out_e[0])
 
 

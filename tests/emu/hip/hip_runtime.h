@@ -50,6 +50,10 @@ inline long long max(long long a, long long b) { return a > b ? a : b; }
 inline long long min(long long a, long long b) { return a < b ? a : b; }
 inline int __clz(int x) { return x == 0 ? 32 : __builtin_clz((unsigned)x); }
 inline int atomicOr(int* p, int v) { return __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }
+inline int atomicAdd(int* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+inline unsigned __builtin_amdgcn_alignbyte(unsigned hi, unsigned lo, unsigned sh) {
+    return (unsigned)((((unsigned long long)hi << 32) | lo) >> (8 * (sh & 3)));
+}
 inline long long atomicMax(long long* p, long long v) {
     long long cur = __atomic_load_n(p, __ATOMIC_SEQ_CST);
     while (cur < v && !__atomic_compare_exchange_n(p, &cur, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST)) {
