@@ -303,6 +303,20 @@ __device__ __forceinline__ void split_centred(int r, int m, int& hi, int& lo) {
     hi = (r - lo) >> 7;
 }
 
+// acc + ov 2^64 = sum of x[i] y[K - i] over the static column K of two N-word magnitudes
+template <int N, int K>
+__device__ __forceinline__ void column_sum(const u32* x, const u32* y, u64& acc, u32& ov) {
+    constexpr int I0 = K - (N - 1) > 0 ? K - (N - 1) : 0, I1 = K < N - 1 ? K : N - 1, NT = I1 - I0 + 1;
+    acc = 0;
+    ov = 0;
+#pragma unroll
+    for (int q = 0; q < NT / 4; q++) {
+        const u32 yv[4] = {y[K - I0 - 4 * q], y[K - I0 - 4 * q - 1], y[K - I0 - 4 * q - 2], y[K - I0 - 4 * q - 3]};
+        SDPV_MAC96_CHAIN4(acc, ov, x + I0 + 4 * q, yv);
+    }
+#pragma unroll
+    for (int i = I0 + NT / 4 * 4; i <= I1; i++) SDPV_MAC96(acc, ov, x[i], y[K - i]);
+}
 // Bytewise a + b of packed int8 lanes (no carries between bytes); exact when each byte sum
 // stays in [-128, 127].
 __device__ __forceinline__ u32 add_bytes(u32 a, u32 b) {

@@ -139,7 +139,293 @@ __global__ void __launch_bounds__(TPB) k_mpf_norm(const i32* __restrict__ X, con
     eO[i] = eI[i] + s;
 }
 
-// ------------------------------------------------------------------ mpf_mul (mpf.py:58-89)
+// ------------------------------------------------------------------ products and sums in registers
+// Up to 40 limbs both operands of an entry live in registers, in arrays of N >= L words with static indexes
+// (N = 8, 16, 24, 28, 32, 36 or 40). Bound: reading two operands and writing one; a product's N^2
+// multiply-adds take about as long.
+
+// magnitude of the two's complement words x (zero above the sign's word), its sign returned
+template <int N>
+__device__ __forceinline__ bool to_magnitude(u32* x, u32 top) {
+    const bool neg = (top >> 31) != 0;
+    const u32 f = neg ? ~0u : 0u;
+    u32 c = neg ? 1u : 0u;
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        const u64 t = (u64)(x[w] ^ f) + c;
+        x[w] = (u32)t;
+        c = (u32)(t >> 32);
+    }
+    return neg;
+}
+
+// words of a product from column K on into p[K - (N - 1)] for K >= N - 1 (the lower ones carry only)
+template <int N, int K>
+struct MulColumns {
+    static __device__ __forceinline__ void run(const u32* x, const u32* y, u64& carry, u32* p) {
+        u64 acc;
+        u32 ov;
+        column_sum<N, K>(x, y, acc, ov);
+        const u64 sm = acc + carry;
+        carry = (sm >> 32) | ((u64)(ov + (sm < carry ? 1u : 0u)) << 32);
+        if (K >= N - 1) p[K >= N - 1 ? K - (N - 1) : 0] = (u32)sm;
+        if constexpr (K < 2 * N - 2) MulColumns<N, K + 1>::run(x, y, carry, p);
+        else p[N] = (u32)carry;
+    }
+};
+
+// any product (operands that are not normalised): columns from memory, once for the length, once rounded
+__device__ void mul_any(const PlaneSrc& xa, const PlaneSrc& xb, int L, i64 n, i64 i, i32* O, i64* eO, i64 e) {
+    MagView<PlaneSrc> ma(xa, L), mb(xb, L);
+    int bl = 0, s = 0;
+    i64 q1 = 0;
+    u32 prev = 0, c = 0;
+    NegStream ng(ma.neg != mb.neg);
+    for (int pass = 0; pass < 2; pass++) {
+        u64 carry = 0, hprev = 0;
+        for (int k = 0; k < 2 * L + 1; k++) {
+            u64 lo = 0, hi = 0;
+            const int first = k - L + 1 > 0 ? k - L + 1 : 0, last = k < L - 1 ? k : L - 1;
+            for (int x = first; x <= last; x++) {
+                const u64 pr = (u64)ma(x) * mb(k - x);
+                lo += (u32)pr;
+                hi += pr >> 32;
+            }
+            const u64 sum = lo + hprev + carry;
+            const u32 w = (u32)sum;
+            carry = sum >> 32;
+            hprev = hi;
+            if (pass == 0) {
+                if (w) bl = 32 * k + 32 - clz32(w);
+                continue;
+            }
+            if (s > 0) {                                  // word k of the product completes output word k - 1 - q1
+                if (k == q1) c = (w >> ((s - 1) & 31)) & 1u;
+                if (k > q1 && k - 1 - q1 < L) {
+                    const u64 d = ((((u64)w << 32) | prev) >> (((s - 1) & 31) + 1)) & 0xffffffffull;
+                    const u64 t = d + c;
+                    c = (u32)(t >> 32);
+                    O[(k - 1 - q1) * n + i] = (i32)ng((u32)t);
+                }
+            } else {                                      // left shift by whole words and bits: words below stay zero
+                const int t = -s, q = t >> 5, r = t & 31;
+                if (k == 0)
+                    for (int z = 0; z < q && z < L; z++) O[(i64)z * n + i] = (i32)ng(0u);
+                if (k + q < L) O[(i64)(k + q) * n + i] = (i32)ng(r ? (w << r) | (prev >> (32 - r)) : w);
+            }
+            prev = w;
+        }
+        s = bl - (32 * L - 2);
+        q1 = s > 0 ? (s - 1) >> 5 : 0;
+    }
+    eO[i] = e + s;
+}
+
+// one entry per thread. Limbs sit in the upper L of N words, so the product of two normalised entries has
+// its rounded words at static places whatever L is. 787 320 products at L = 24 on one MI355X:
+// 0.061 ms, 4.0 TB/s (operands in LDS slices, word by word: 0.511 ms).
+template <int N>
+__global__ void __launch_bounds__(256) k_mul_regs(const i32* __restrict__ A, const i64* __restrict__ eA,
+                                                  const i32* __restrict__ Bm, const i64* __restrict__ eB,
+                                                  i32* __restrict__ O, i64* __restrict__ eO, int L, i64 n, int bscalar) {
+    const i64 i = blockIdx.x * (i64)256 + threadIdx.x;
+    if (i >= n) return;
+    const i64 ib = bscalar ? 0 : i, nb = bscalar ? 1 : n;
+    const int d = N - L;
+    u32 x[N], y[N];
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        x[w] = w >= d ? (u32)A[(i64)(w - d) * n + i] : 0u;
+        y[w] = w >= d ? (u32)Bm[(i64)(w - d) * nb + ib] : 0u;
+    }
+    const i64 e = eA[i] + eB[ib];
+    const bool neg = to_magnitude<N>(x, x[N - 1]) != to_magnitude<N>(y, y[N - 1]);
+    u32 za = 0, zb = 0;
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        za |= x[w];
+        zb |= y[w];
+    }
+    if (za == 0u || zb == 0u) {
+        for (int k = 0; k < L; k++) O[(i64)k * n + i] = 0;
+        eO[i] = EZV;
+        return;
+    }
+    u32 p[N + 1];                                         // words N - 1 .. 2N - 1 of the product
+    u64 carry = 0;
+    MulColumns<N, 0>::run(x, y, carry, p);
+    // bit length from the two top words; the shift to 32 L - 2 bits must start in word 2N - L - 1
+    const int bl = 32 * (2 * L - 2) + (p[N] ? 64 - clz32(p[N]) : 32 - clz32(p[N - 1]));
+    const int s = bl - (32 * L - 2);
+    if ((p[N] | p[N - 1]) == 0u || (s - 1) >> 5 != L - 1) {
+        mul_any(PlaneSrc{A + i, n}, PlaneSrc{Bm + ib, nb}, L, n, i, O, eO, e);
+        return;
+    }
+    const int r = (s - 1) & 31, q = N - L;                // p[q]: the word with the rounding bit
+    u32 c = 0, nc = neg ? 1u : 0u;
+    const u32 f = neg ? ~0u : 0u;
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        if (w == q) c = (p[w] >> r) & 1u;
+        const u64 t = (((((u64)p[w + 1] << 32) | p[w]) >> r >> 1) & 0xffffffffull) + c;
+        c = (u32)(t >> 32);
+        if (w >= q) {
+            const u64 u = (u64)((u32)t ^ f) + nc;
+            nc = (u32)(u >> 32);
+            O[(i64)(w - q) * n + i] = (i32)(u32)u;
+        }
+    }
+    eO[i] = e + s;
+}
+
+// x >>= 32 q words in registers (0 <= q < 64), words moved in steps that some lane of the wave needs
+template <int N>
+__device__ __forceinline__ void words_down(u32* x, int q) {
+#pragma unroll
+    for (int st = 1; st < 64; st <<= 1) {
+        if (st < N ? ballot64(q & st) != 0 : false) {
+#pragma unroll
+            for (int w = 0; w < N; w++) x[w] = (q & st) ? (w + st < N ? x[w + st] : 0u) : x[w];
+        } else if (st >= N) {
+#pragma unroll
+            for (int w = 0; w < N; w++) x[w] = (q & st) ? 0u : x[w];
+        }
+    }
+}
+template <int N>
+__device__ __forceinline__ void words_up(u32* x, int q) {
+#pragma unroll
+    for (int st = 1; st < 64; st <<= 1) {
+        if (st < N ? ballot64(q & st) != 0 : false) {
+#pragma unroll
+            for (int w = N - 1; w >= 0; w--) x[w] = (q & st) ? (w >= st ? x[w - st] : 0u) : x[w];
+        } else if (st >= N) {
+#pragma unroll
+            for (int w = 0; w < N; w++) x[w] = (q & st) ? 0u : x[w];
+        }
+    }
+}
+// x <- round_half_up(x / 2^s), s >= 1 (x, N words, unsigned); lanes with s < 1 keep x
+template <int N>
+__device__ __forceinline__ void round_down(u32* x, i64 s) {
+    const bool on = s >= 1;
+    const int t = on ? (int)(s > 32 * N + 1 ? 32 * N + 1 : s) - 1 : 0, r = t & 31;
+    words_down<N>(x, t >> 5);
+    u32 c = (x[0] >> r) & 1u;
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        const u64 v = (((((u64)(w + 1 < N ? x[w + 1] : 0u) << 32) | x[w]) >> r >> 1) & 0xffffffffull) + c;
+        c = (u32)(v >> 32);
+        x[w] = on ? (u32)v : x[w];
+    }
+}
+
+// A + sgn B (mpf.py:92-124): the operand with the larger exponent one word up, the other rounded to the same
+// place, magnitudes added or subtracted, the result normalised. 787 320 sums at L = 24 on one
+// MI355X: 0.079 ms, 3.1 TB/s (operands read word by word at every use, sums in LDS: 0.344 ms).
+template <int N>
+__global__ void __launch_bounds__(256) k_add_regs(const i32* __restrict__ A, const i64* __restrict__ eA,
+                                                  const i32* __restrict__ Bm, const i64* __restrict__ eB,
+                                                  i32* __restrict__ O, i64* __restrict__ eO, int L, i64 n, int sgn) {
+    constexpr int W = N + 2;
+    const i64 i0 = blockIdx.x * (i64)256 + threadIdx.x, i = i0 < n ? i0 : n - 1;   // every lane takes part in ballots
+    u32 x[W], y[W];                                       // one word up
+    x[0] = y[0] = x[W - 1] = y[W - 1] = 0u;
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        x[w + 1] = w < L ? (u32)A[(i64)w * n + i] : 0u;
+        y[w + 1] = w < L ? (u32)Bm[(i64)w * n + i] : 0u;
+    }
+    i64 ea = eA[i], eb = eB[i];
+    auto magnitude = [&](u32* v) {                        // of the L words from v[1] on
+        u32 top = 0;
+#pragma unroll
+        for (int w = 1; w <= N; w++) top = w == L ? v[w] : top;
+        const bool neg = (top >> 31) != 0;
+        const u32 f = neg ? ~0u : 0u;
+        u32 c = neg ? 1u : 0u;
+#pragma unroll
+        for (int w = 1; w <= N; w++) {
+            const u64 t = (u64)(w <= L ? v[w] ^ f : 0u) + c;
+            v[w] = w <= L ? (u32)t : 0u;
+            c = (u32)(t >> 32);
+        }
+        return neg;
+    };
+    bool na = magnitude(x), nbg = magnitude(y) != (sgn < 0);
+    u32 za = 0, zb = 0;
+#pragma unroll
+    for (int w = 1; w <= N; w++) {
+        za |= x[w];
+        zb |= y[w];
+    }
+    if (za == 0u) ea = EZV;
+    if (zb == 0u) eb = EZV;
+    const bool zero = ea == EZV && eb == EZV;
+    if (ea == EZV || eb == EZV) {                         // a zero operand adds nothing
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            x[w] = ea == EZV ? 0u : x[w];
+            y[w] = eb == EZV ? 0u : y[w];
+        }
+    }
+    const bool sw = eb > ea;                              // x: the larger exponent
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+        const u32 t = x[w];
+        x[w] = sw ? y[w] : t;
+        y[w] = sw ? t : y[w];
+    }
+    const bool nx = sw ? nbg : na, ny = sw ? na : nbg;
+    const i64 et = (sw ? eb : ea) - 32, dist = sw ? eb - ea : ea - eb;
+    round_down<W>(y, dist);
+    // magnitudes: x + y, or x - y with the sign of the larger
+    const bool sub = nx != ny;
+    const u32 fy = sub ? ~0u : 0u;
+    u32 c = sub ? 1u : 0u;
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+        const u64 t = (u64)x[w] + (y[w] ^ fy) + c;
+        x[w] = (u32)t;
+        c = (u32)(t >> 32);
+    }
+    const bool flip = sub && c == 0u;                     // y was larger
+    const bool neg = nx != flip;
+    if (ballot64(flip)) {
+        const u32 ff = flip ? ~0u : 0u;
+        c = flip ? 1u : 0u;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const u64 t = (u64)(x[w] ^ ff) + c;
+            x[w] = (u32)t;
+            c = (u32)(t >> 32);
+        }
+    }
+    int bl = 0;
+#pragma unroll
+    for (int w = 0; w < W; w++) bl = x[w] ? 32 * w + 32 - clz32(x[w]) : bl;
+    const int s = bl == 0 ? 0 : bl - (32 * L - 2);
+    if (ballot64(s < 0)) {                                // cancellation: left
+        const int t = s < 0 ? -s : 0, r = t & 31;
+        words_up<W>(x, t >> 5);
+#pragma unroll
+        for (int w = W - 1; w >= 0; w--) x[w] = (u32)(((((u64)x[w] << 32) | (w > 0 ? x[w - 1] : 0u)) << r) >> 32);
+    }
+    round_down<W>(x, s);
+    if (i0 >= n) return;
+    const bool none = zero || bl == 0;
+    const u32 f = neg ? ~0u : 0u;
+    c = neg ? 1u : 0u;
+#pragma unroll
+    for (int w = 0; w < N; w++) {
+        const u64 t = (u64)(x[w] ^ f) + c;
+        c = (u32)(t >> 32);
+        if (w < L) O[(i64)w * n + i] = none ? 0 : (i32)(u32)t;
+    }
+    eO[i] = none ? EZV : et + s;
+}
+
+// ------------------------------------------------------------------ mpf_mul (mpf.py:58-89), more than 40 limbs
 // Magnitudes staged in per-thread LDS slices; product scanning over runtime L.
 constexpr int MUL_TPB = 64;
 __global__ void __launch_bounds__(MUL_TPB) k_mpf_mul(const i32* __restrict__ A, const i64* __restrict__ eA,
@@ -189,7 +475,7 @@ __global__ void __launch_bounds__(MUL_TPB) k_mpf_mul(const i32* __restrict__ A, 
     eO[i] = eA[i] + eB[ib] + s;
 }
 
-// ------------------------------------------------------------------ mpf_add (mpf.py:92-124)
+// ------------------------------------------------------------------ mpf_add (mpf.py:92-124), more than 40 limbs
 constexpr int ADD_TPB = 64;
 __global__ void __launch_bounds__(ADD_TPB) k_mpf_add(const i32* __restrict__ A, const i64* __restrict__ eA,
                                                      const i32* __restrict__ Bm, const i64* __restrict__ eB,
@@ -505,6 +791,15 @@ int sdpv_mpf_mul(const int32_t* A, const int64_t* eA, const int32_t* Bm, const i
     if (L > 128) return SDPV_ESIZE;
     if (n == 0) return SDPV_OK;
     if (!A || !eA || !Bm || !eB || !O || !eO) return SDPV_EARG;
+#define SDPV_MUL(N)                                                                                              \
+    if (L <= N) {                                                                                                \
+        hipLaunchKernelGGL(k_mul_regs<N>, dim3(nblocks(n, 256)), dim3(256), 0, as_stream(stream), A, eA, Bm, eB, O, \
+                           eO, (int)L, (i64)n, (int)(bscalar != 0));                                             \
+        SDPV_TRY_LAUNCH();                                                                                       \
+        return SDPV_OK;                                                                                          \
+    }
+    SDPV_MUL(8) SDPV_MUL(16) SDPV_MUL(24) SDPV_MUL(28) SDPV_MUL(32) SDPV_MUL(36) SDPV_MUL(40)
+#undef SDPV_MUL
     const size_t lds = (size_t)4 * L * MUL_TPB * sizeof(u32);
     hipLaunchKernelGGL(k_mpf_mul, dim3(nblocks(n, MUL_TPB)), dim3(MUL_TPB), lds, as_stream(stream), A, eA, Bm, eB,
                        O, eO, (int)L, (i64)n, (int)(bscalar != 0));
@@ -518,6 +813,15 @@ int sdpv_mpf_add(const int32_t* A, const int64_t* eA, const int32_t* Bm, const i
     if (L > 256) return SDPV_ESIZE;
     if (n == 0) return SDPV_OK;
     if (!A || !eA || !Bm || !eB || !O || !eO) return SDPV_EARG;
+#define SDPV_ADD(N)                                                                                              \
+    if (L <= N) {                                                                                                \
+        hipLaunchKernelGGL(k_add_regs<N>, dim3(nblocks(n, 256)), dim3(256), 0, as_stream(stream), A, eA, Bm, eB, O, \
+                           eO, (int)L, (i64)n, (int)sgn);                                                        \
+        SDPV_TRY_LAUNCH();                                                                                       \
+        return SDPV_OK;                                                                                          \
+    }
+    SDPV_ADD(8) SDPV_ADD(16) SDPV_ADD(24) SDPV_ADD(28) SDPV_ADD(32) SDPV_ADD(36) SDPV_ADD(40)
+#undef SDPV_ADD
     const size_t lds = (size_t)(L + 2) * ADD_TPB * sizeof(u32);
     hipLaunchKernelGGL(k_mpf_add, dim3(nblocks(n, ADD_TPB)), dim3(ADD_TPB), lds, as_stream(stream), A, eA, Bm, eB,
                        O, eO, (int)L, (i64)n, (int)sgn);
