@@ -171,7 +171,8 @@ int sdpv_row_exp(const int32_t* X, const int64_t* e, int64_t L, int64_t plane, i
  * s = 0 for every entry when e == NULL) from L to Lout limbs, then reduced modulo the primes
  * g0 .. g0+G-1 to the centred residue r = 128*hi + lo (lo in [-64, 63]).
  * Rh, Rl: (G, kp/16, nb*rows, 16) int8, chunk-major: byte k of row r of prime g at
- * ((g*(kp/16) + k/16)*nb*rows + r)*16 + k%16; columns kc <= k < kp hold residue 0.
+ * ((g*(kp/16) + k/16)*nb*rows + r)*16 + k%16; columns kc <= k < kp hold residue 0
+ * (kp a multiple of 32).
  * Tables (built by the caller for Lout): Thi/Tlo (npad, NBp) int8 with NBp = 32*ceil(4 Lout/32),
  * T = 128*Thi + Tlo the centred 256^j mod m; C1 (n,) int32 = 128 * sum_{j < 4 Lout - 1} T_j mod m
  * (the bias of every byte but the top one, which enters signed); mods (n,) int32, minv (n,)
@@ -195,7 +196,7 @@ int sdpv_rns_split(const int32_t* X, const int64_t* e, const int64_t* Erow, int6
  *   acc[(g0+gi)*ld_g + (b*M + i)*N + j] = s_g * (sum_k a[gi, b*M+i, k] * b[gi, b*N+j, k]) mod m_g
  * (g = g0+gi) stored as int16 in [0, m), or centred with SDPV_GEMM_CENTRED.
  * Ah/Al: (G, kp/16, nb*M, 16), Bh/Bl: (G, kp/16, nb*N, 16) int8, chunk-major as written by
- * sdpv_rns_split, kp a multiple of 64, kp <= 65536.
+ * sdpv_rns_split, kp a multiple of 64 (of 32 for config -1, 2, 3, 12 and 13), kp <= 65536.
  * kcoef: (n, 3) int32 = (16256, 128, -127) * s_g mod m: ra*rb = 16256*HH + 128*SS - 127*LL.
  * s_g = 1 gives the residues of the product; s_g = (M/m_g)^-1 mod m_g with SDPV_GEMM_CENTRED
  * gives the CRT coefficients that sdpv_rns_crt takes with SDPV_CRT_SCALED.

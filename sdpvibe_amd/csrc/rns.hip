@@ -870,7 +870,7 @@ int sdpv_rns_split(const int32_t* X, const int64_t* e, const int64_t* Erow, int6
                    const int32_t* mods, const double* minv, int64_t g0, int64_t G, int8_t* Rh,
                    int8_t* Rl, int32_t* flag, void* stream) {
     if (L < 1 || Lout < 1 || nb < 0 || rows < 0 || kc < 0 || kp < kc || G < 0 || g0 < 0) return SDPV_EARG;
-    if (kp % 64 != 0 || NBp != 32 * ((4 * Lout + 31) / 32)) return SDPV_EARG;
+    if (kp % 32 != 0 || NBp != 32 * ((4 * Lout + 31) / 32)) return SDPV_EARG;
     if (Lout > 128 || L > 128) return SDPV_ESIZE;
     const i64 nrows = nb * rows;
     if (nrows == 0 || kp == 0 || G == 0) return SDPV_OK;
@@ -920,7 +920,10 @@ int sdpv_rns_gemm(const int8_t* Ah, const int8_t* Al, const int8_t* Bh, const in
                   const double* minv, const int32_t* kcoef, int64_t g0, int32_t mode, int32_t config, void* stream) {
     if (G < 0 || nb < 0 || M < 0 || N < 0 || kp < 0 || g0 < 0 || (mode & ~7)) return SDPV_EARG;
     if (config < -1 || config > 13) return SDPV_EARG;
-    if (kp % 64 != 0 || kp > 65536) return SDPV_ESIZE;
+    if (kp % 32 != 0 || kp > 65536) return SDPV_ESIZE;
+    // an odd multiple of 32 takes the tiles that have 32-byte stages
+    const bool half = kp % 64 != 0;
+    if (half && !(config == -1 || config == 2 || config == 3 || config == 12 || config == 13)) return SDPV_ESIZE;
     if (nb * M > (1LL << 26) || nb * N > (1LL << 26)) return SDPV_ESIZE;   // 32-bit offsets in a stage
     // the syrk mode skips tiles above the diagonal by tile index: square tiles only
     if ((mode & SDPV_GEMM_SYRK_LOWER) &&
@@ -932,14 +935,20 @@ int sdpv_rns_gemm(const int8_t* Ah, const int8_t* Al, const int8_t* Bh, const in
     if (kp == 0) return SDPV_EARG;
     if (config == -1) {
         const i64 mn = M < N ? M : N;  // syrk: square tiles of 128 / 64 / 32 by N, as the reference
-        config = mn >= 128 ? 6 : (mn >= 64 ? 2 : 3);   // 128x128 four-product tile: the fastest
+        config = mn >= 128 && !half ? 6 : (mn >= 64 ? 2 : 3);   // 128x128 four-product tile: the fastest
     }
     const int g = (int)G, b = (int)nb, q0 = (int)g0;
     switch (config) {
         case 0: return launch_gemm<2, 2, 2, 2, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
         case 1: return launch_gemm<2, 2, 2, 2, 3, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
-        case 2: return launch_gemm<2, 2, 1, 1, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
-        case 3: return launch_gemm<1, 1, 1, 1, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
+        case 2:
+            if (half)
+                return launch_gemm<2, 2, 1, 1, 2, 0, 32>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
+            return launch_gemm<2, 2, 1, 1, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
+        case 3:
+            if (half)
+                return launch_gemm<1, 1, 1, 1, 2, 0, 32>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
+            return launch_gemm<1, 1, 1, 1, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
         case 4: return launch_gemm<4, 2, 2, 2, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
         case 5: return launch_gemm<2, 4, 2, 2, 2, 0>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);
         case 6: return launch_gemm<2, 2, 2, 2, 2, 1>(Ah, Al, Bh, Bl, g, b, M, N, kp, acc, ld_g, mods, minv, kcoef, q0, mode, st);

@@ -204,7 +204,7 @@ def residue_gemm(R, A_desc, B_desc, nb, M, N, K, acc_rows_budget=None):
             acc.zero_()
         for k0 in range(0, K, kc):
             kk = min(kc, K - k0)
-            kp = R.kp(kk)
+            kp = R.kp_product(kk)
             Ah, Al = A_desc(k0, kk, kp, j0, jw)
             Bh, Bl = B_desc(k0, kk, kp, j0, jw)
             R.product(Ah, Al, Bh, Bl, acc, nb, M, jw, nb * M * jw, accumulate=not first, scaled=True)

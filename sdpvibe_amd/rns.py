@@ -67,6 +67,7 @@ def gemm_config(M, N, K):
 
 # ------------------------------------------------------------------ product tile autotuner
 GEMM_CONFIGS = tuple(range(14))   # see sdpv_rns_gemm: tile shapes, stages, three or four products, epilogue
+HALF_CONFIGS = (2, 3, 12, 13)     # those that take an inner dimension padded to a multiple of 32
 _tuned = {}
 TUNE = os.environ.get("SDPV_TUNE", "1") != "0"
 # SDPV_GEMM_CONFIG=<c> pins every tuned product to configuration c (measurements of one tile shape)
@@ -92,15 +93,16 @@ def tuned_config(R, nb, M, N, kp):
     tuning is off or the product is small"""
     if not TUNE or nb * M * N * kp < (1 << 24):
         return -1
+    half = kp % RNS.KPAD != 0                # multiples of 32 only: the tiles with 32-byte stages
     if FORCED is not None:
-        return FORCED
-    key = (R.L, _bucket(nb), _bucket(M), _bucket(N), _bucket(kp))
+        return FORCED if not half or FORCED in HALF_CONFIGS else -1
+    key = (R.L, _bucket(nb), _bucket(M), _bucket(N), kp if half else _bucket(kp))
     if key not in _tuned:
-        _tuned[key] = _measure(R, nb, M, N, kp)
+        _tuned[key] = _measure(R, nb, M, N, kp, HALF_CONFIGS if half else GEMM_CONFIGS)
     return _tuned[key]
 
 
-def _measure(R, nb, M, N, kp, reps=3):
+def _measure(R, nb, M, N, kp, configs, reps=3):
     # every prime when the scratch operands stay small (the launch's wave count decides between tiles)
     G = R.n if R.n * nb * (2 * kp * (M + N) + 2 * M * N) <= (1 << 29) else min(R.n, 32)
     dev_ = R.m32.device
@@ -113,11 +115,11 @@ def _measure(R, nb, M, N, kp, reps=3):
     st = torch.cuda.current_stream()
     launch = lambda cfg: call("sdpv_rns_gemm", ptr(Ah), ptr(Al), ptr(Bh), ptr(Bl), G, nb, M, N, kp, ptr(acc),
                               nb * M * N, ptr(R.m32), ptr(R.minv), ptr(R.kcoef), 0, 0, cfg, stream())
-    for cfg in GEMM_CONFIGS:                          # warm every configuration (attributes, clocks)
+    for cfg in configs:                               # warm every configuration (attributes, clocks)
         launch(cfg)
     best_t = {}
     for _ in range(2):                                # two passes, the faster of each: clock drift
-        for cfg in GEMM_CONFIGS:
+        for cfg in configs:
             ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             ev0.record(st)
             for _ in range(reps):
@@ -126,7 +128,7 @@ def _measure(R, nb, M, N, kp, reps=3):
             ev1.synchronize()
             t = ev0.elapsed_time(ev1)
             best_t[cfg] = min(t, best_t.get(cfg, t))
-    return min(GEMM_CONFIGS, key=lambda c: best_t[c])
+    return min(configs, key=lambda c: best_t[c])
 
 
 def row_major(R):
@@ -197,6 +199,12 @@ class RNS:
     def kp(self, kc):
         return -(-kc // self.KPAD) * self.KPAD
 
+    def kp_product(self, kc):
+        """padded inner dimension of an internal product: to a multiple of 32 for a short one (a tile of 32
+        pays for no zero half: splitting and multiplying 32 x 32 leaves padded to 64 took twice the
+        work), of 64 otherwise, where the padding weighs little and every product tile applies"""
+        return -(-kc // 32) * 32 if kc <= 96 else self.kp(kc)
+
     def residues(self, X, k0, kc, g0=0, G=None):
         """X: (L, rows, K) int32 limb planes. Residues of X[:, :, k0:k0+kc] modulo primes
         g0..g0+G as (G, rows, kp) int8 hi / lo (128*hi + lo = centred residue), inner dimension
@@ -219,7 +227,7 @@ class RNS:
         G = self.n - g0 if G is None else G
         # host-side extent checks: the kernel trusts these sizes
         nrows = nb * rows
-        if not (0 <= g0 and g0 + G <= self.n and kp % self.KPAD == 0 and 0 <= kc <= kp):
+        if not (0 <= g0 and g0 + G <= self.n and kp % 32 == 0 and 0 <= kc <= kp):
             raise ValueError("split: prime range or padded width out of range")
         for Rx in (Rh, Rl):
             if tuple(Rx.shape) != (G, kp // 16, nrows, 16) or not Rx.is_contiguous() or Rx.dtype != torch.int8:
