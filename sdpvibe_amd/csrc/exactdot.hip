@@ -284,52 +284,6 @@ __device__ __forceinline__ i64 round_shift(const Operand& X, i64 row, i64 off) {
     return e == EZV ? (i64)1 << 30 : X.E[row] - e;
 }
 
-// x (NW words, L of them given, the others the sign) <- the words of round_half_up(x / 2^s), s >= 0 per lane, and
-// `ext` the word that extends them. The rounding bit is added first; then every word is a funnel shift of two
-// neighbours, and whole words move by 1 and 2 in registers and by multiples of 4 through the lane's 16-byte
-// aligned slot (aligned accesses have no bank conflicts; only when some lane of the wave needs it).
-template <int NW>
-__device__ __forceinline__ void round_words(u32* x, int L, i64 s, u32& ext, v4i* slot) {
-    ext = 0;
-#pragma unroll
-    for (int w = 0; w < NW; w++)
-        if (w == L - 1) ext = (x[w] >> 31) ? ~0u : 0u;
-#pragma unroll
-    for (int w = NW - 8 > 0 ? NW - 8 : 0; w < NW; w++)
-        if (w >= L) x[w] = ext;
-    const int sc = s > 32 * NW ? 32 * NW : (int)s, hb = sc - 1;
-    const u32 half = sc > 0 ? 1u << (hb & 31) : 0u;
-    const int hw = hb >> 5;
-    u32 c = 0;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-        const u64 t = (u64)x[w] + (w == hw ? half : 0u) + c;
-        x[w] = (u32)t;
-        c = (u32)(t >> 32);
-    }
-    ext += c;
-    const int r = sc & 31, q = sc >> 5;
-#pragma unroll
-    for (int w = 0; w < NW; w++) x[w] = (u32)((((u64)(w + 1 < NW ? x[w + 1] : ext) << 32) | x[w]) >> r);
-#pragma unroll
-    for (int w = 0; w < NW; w++) x[w] = (q & 1) ? (w + 1 < NW ? x[w + 1] : ext) : x[w];
-#pragma unroll
-    for (int w = 0; w < NW; w++) x[w] = (q & 2) ? (w + 2 < NW ? x[w + 2] : ext) : x[w];
-    if (ballot64(q >= 4)) {
-        const int q4 = q >> 2;
-#pragma unroll
-        for (int g = 0; g < NW / 4; g++)
-            slot[g] = v4i{(int)x[4 * g], (int)x[4 * g + 1], (int)x[4 * g + 2], (int)x[4 * g + 3]};
-#pragma unroll
-        for (int g = 0; g < NW / 4; g++) {
-            const bool in = g + q4 < NW / 4;
-            const v4i v = slot[in ? g + q4 : 0];
-#pragma unroll
-            for (int u = 0; u < 4; u++) x[4 * g + u] = in ? (u32)v[u] : ext;
-        }
-    }
-}
-
 // KM: the entries' threads run along k (contiguous) instead of rows
 template <int KS, bool KM>
 __global__ void __launch_bounds__(Geo<KS>::NT, KS <= 3 ? 2 : 1) k_narrow(Operand A, Operand B, Dims D, Result R, i64* __restrict__ part,

@@ -72,8 +72,12 @@ __device__ __forceinline__ u32 pack4(int a, int b, int c, int d) {  // low bytes
 }
 
 // table chunks of 32 bytes: KSC = NBp / 32 (0: any, read from NBp); up to three chunks the kernel
-// fits 128 VGPRs, four workgroups per CU
-template <int KSC>
+// fits 128 VGPRs, four workgroups per CU. SMALL (KSC 1..4): small launches, whose time is one chain of
+// dependent steps: the prime blocks are shared out over grid.y (each workgroup repeats phase 1) and the limbs
+// rounded in registers. The splits of chol(Q) at N = 3000, mostly of 32 to 1504 rows of 32 entries: 12.8 us on
+// average before, 7.4 now. For large launches this form measured equal or slower (60 x 192 x 3000: 0.50
+// against 0.47 ms).
+template <int KSC, bool SMALL>
 __global__ void __launch_bounds__(256, (KSC >= 1 && KSC <= 3) ? 4 : 1) k_rns_split(
     const i32* __restrict__ X, const i64* __restrict__ e, const i64* __restrict__ Erow, int L, int Lout, i64 plane,
     i64 nb, i64 rows, i64 ldb, i64 ldr, i64 ldk, i64 k0, i64 kc, i64 kp, const int8_t* __restrict__ Thi,
@@ -121,7 +125,7 @@ __global__ void __launch_bounds__(256, (KSC >= 1 && KSC <= 3) ? 4 : 1) k_rns_spl
         o.c1 = C1[g];
     };
     PB cur, nxt;
-    load_pb(0, cur);                                    // first block's tables: in flight during phase 1
+    load_pb(SMALL ? blockIdx.y : 0, cur);                           // first block's tables: in flight during phase 1
 
     // ---- phase 1: thread t -> entry (r, k) of the tile
     {
@@ -138,70 +142,105 @@ __global__ void __launch_bounds__(256, (KSC >= 1 && KSC <= 3) ? 4 : 1) k_rns_spl
         const i64 off = valid ? (Rc / rows) * ldb + (Rc % rows) * ldr + (k0 + kg) * ldk : 0;
         const i64 ex = e ? e[off] : 0;                  // exponents first: their latency overlaps the limbs'
         const i64 er = e ? Erow[Rc] : 0;
-        if (stage) {
+        if constexpr (SMALL) {
+            // the entry in registers: all limbs requested at once, rounded there (round_words), the bytes
+            // written as aligned 16-byte groups
+            constexpr int NW = 8 * (KSC >= 1 ? KSC : 1);
+            u32 x[NW];
             const i32* px = X + off;
-            for (int w0 = 0; w0 < L; w0 += 32) {         // independent loads, up to 32 in flight
-                u32 v[32];
 #pragma unroll
-                for (int u = 0; u < 32; u++) {
-                    v[u] = (u32)*px;                    // words past L - 1 re-read word L - 1
-                    if (w0 + u + 1 < L) px += plane;
-                }
-                if (stage == 2) {                       // 16-byte row: L rounded up to 4 words fits
-#pragma unroll
-                    for (int q = 0; q < 8; q++)
-                        if (w0 + 4 * q < L) {
-                            v4i g4;
-                            g4[0] = (int)v[4 * q]; g4[1] = (int)v[4 * q + 1];
-                            g4[2] = (int)v[4 * q + 2]; g4[3] = (int)v[4 * q + 3];
-                            *(v4i*)(raw + w0 + 4 * q) = g4;
-                        }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 32; u++)
-                        if (w0 + u < L) raw[w0 + u] = v[u];
-                }
+            for (int w = 0; w < NW; w++) {
+                x[w] = (u32)*px;                        // words past L - 1 re-read word L - 1
+                if (w + 1 < L) px += plane;
             }
-        }
-        // words leave in groups of four (16-byte LDS writes: conflict-free at this row stride)
-        u32 b0 = 0x80808080u, b1 = 0x80808080u, b2 = 0x80808080u, b3 = 0x80808080u;
-        auto flush4 = [&](int w4) {
-            v4i q4;
-            q4[0] = (int)b0; q4[1] = (int)b1; q4[2] = (int)b2; q4[3] = (int)b3;
-            *(v4i*)(row + 4 * w4) = q4;
-            b0 = b1 = b2 = b3 = 0x80808080u;
-        };
-        auto put = [&](int wi, u32 v) {                 // bias every byte but the top one
-            const u32 x = v ^ (wi == Lout - 1 ? 0x00808080u : 0x80808080u);
-            switch (wi & 3) {
-                case 0: b0 = x; break;
-                case 1: b1 = x; break;
-                case 2: b2 = x; break;
-                default: b3 = x; flush4(wi >> 2);
-            }
-        };
-        if (valid) {
             i64 s = 0;
             if (e) s = (ex == EZV) ? (i64)(1 << 30) : er - ex;
-            // In place (stage 2), output word k is written after every read of source words <= k
-            // when s >= 0 (the reads of a batch of 8 precede its writes, and later batches read
-            // words >= k + 8). A left shift (s < 0) reads below k, so it re-reads the limbs from
-            // global memory instead.
-            const bool lds_src = stage == 1 || (stage == 2 && s >= 0);
-            const int bad = lds_src ? shr_round_batched(LdsStrided{raw, 1}, L, s, Lout, put)
-                                    : shr_round_batched(PlaneSrc{X + off, plane}, L, s, Lout, put);
-            if (bad && flag) atomicOr(flag, 1);
+            if (e || L < Lout) {
+                if (s < 0) {                            // beyond the row's reference: a left shift
+                    (void)shr_round_batched(PlaneSrc{X + off, plane}, L, s, Lout, [&](int k2, u32 v) { row[k2] = v; });
+#pragma unroll
+                    for (int w = 0; w < NW; w++) x[w] = w < Lout ? row[w] : 0u;
+                }
+                u32 ext;
+                round_words<NW>(x, s < 0 ? Lout : L, s < 0 ? 0 : s, ext, (v4i*)row);
+            }
+#pragma unroll
+            for (int g4 = 0; g4 < NW / 4; g4++) {
+                u32 y[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {           // bias every byte but the top one; biased zeros above
+                    const int w = 4 * g4 + u;
+                    y[u] = (valid && w < Lout ? x[w] : 0u) ^ (w == Lout - 1 ? 0x00808080u : 0x80808080u);
+                }
+                ((v4i*)row)[g4] = v4i{(int)y[0], (int)y[1], (int)y[2], (int)y[3]};
+            }
         } else {
-            for (int wi = 0; wi < Lout; wi++) put(wi, 0u);  // zero entry
+            if (stage) {
+                const i32* px = X + off;
+                for (int w0 = 0; w0 < L; w0 += 32) {         // independent loads, up to 32 in flight
+                    u32 v[32];
+#pragma unroll
+                    for (int u = 0; u < 32; u++) {
+                        v[u] = (u32)*px;                    // words past L - 1 re-read word L - 1
+                        if (w0 + u + 1 < L) px += plane;
+                    }
+                    if (stage == 2) {                       // 16-byte row: L rounded up to 4 words fits
+#pragma unroll
+                        for (int q = 0; q < 8; q++)
+                            if (w0 + 4 * q < L) {
+                                v4i g4;
+                                g4[0] = (int)v[4 * q]; g4[1] = (int)v[4 * q + 1];
+                                g4[2] = (int)v[4 * q + 2]; g4[3] = (int)v[4 * q + 3];
+                                *(v4i*)(raw + w0 + 4 * q) = g4;
+                            }
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 32; u++)
+                            if (w0 + u < L) raw[w0 + u] = v[u];
+                    }
+                }
+            }
+            // words leave in groups of four (16-byte LDS writes: conflict-free at this row stride)
+            u32 b0 = 0x80808080u, b1 = 0x80808080u, b2 = 0x80808080u, b3 = 0x80808080u;
+            auto flush4 = [&](int w4) {
+                v4i q4;
+                q4[0] = (int)b0; q4[1] = (int)b1; q4[2] = (int)b2; q4[3] = (int)b3;
+                *(v4i*)(row + 4 * w4) = q4;
+                b0 = b1 = b2 = b3 = 0x80808080u;
+            };
+            auto put = [&](int wi, u32 v) {                 // bias every byte but the top one
+                const u32 x = v ^ (wi == Lout - 1 ? 0x00808080u : 0x80808080u);
+                switch (wi & 3) {
+                    case 0: b0 = x; break;
+                    case 1: b1 = x; break;
+                    case 2: b2 = x; break;
+                    default: b3 = x; flush4(wi >> 2);
+                }
+            };
+            if (valid) {
+                i64 s = 0;
+                if (e) s = (ex == EZV) ? (i64)(1 << 30) : er - ex;
+                // In place (stage 2), output word k is written after every read of source words <= k
+                // when s >= 0 (the reads of a batch of 8 precede its writes, and later batches read
+                // words >= k + 8). A left shift (s < 0) reads below k, so it re-reads the limbs from
+                // global memory instead.
+                const bool lds_src = stage == 1 || (stage == 2 && s >= 0);
+                const int bad = lds_src ? shr_round_batched(LdsStrided{raw, 1}, L, s, Lout, put)
+                                        : shr_round_batched(PlaneSrc{X + off, plane}, L, s, Lout, put);
+                if (bad && flag) atomicOr(flag, 1);
+            } else {
+                for (int wi = 0; wi < Lout; wi++) put(wi, 0u);  // zero entry
+            }
+            if (Lout & 3) flush4(Lout >> 2);                  // last partial group (zero bytes beyond)
+            for (int w4 = (Lout + 3) / 4; w4 < NBp / 16; w4++) flush4(w4);
         }
-        if (Lout & 3) flush4(Lout >> 2);                  // last partial group (zero bytes beyond)
-        for (int w4 = (Lout + 3) / 4; w4 < NBp / 16; w4++) flush4(w4);
     }
     __syncthreads();
 
     // ---- phase 2: wave w owns slots 64w .. 64w + 63 (rows 4w .. 4w + 3 of the tile)
-    for (int pb = 0; pb < nPB; pb++) {
-        if (pb + 1 < nPB) load_pb(pb + 1, nxt);        // next block's table chunks in flight
+    const int pstep = SMALL ? (int)gridDim.y : 1;
+    for (int pb = SMALL ? blockIdx.y : 0; pb < nPB; pb += pstep) {
+        if (pb + pstep < nPB) load_pb(pb + pstep, nxt);   // next block's table chunks in flight
         const int pr = pb * 32 + l32;
         const bool pok = pr < G;
         const int g = g0 + (pok ? pr : 0);
@@ -889,26 +928,35 @@ int sdpv_rns_split(const int32_t* X, const int64_t* e, const int64_t* Erow, int6
     else if (lds + stage_bytes <= 160 * 1024) stage = 1;
     if (stage == 1) lds += stage_bytes;
     if (lds > 160 * 1024) return SDPV_ESIZE;
-    static bool attr_set[5] = {false, false, false, false, false};
     const int ks = NBp / 32 <= 4 ? (int)(NBp / 32) : 0;
-#define SDPV_SPLIT_LAUNCH(KSC)                                                                                 \
+    // at most 512 workgroups (two per CU): the small form, up to 1024 with the prime blocks shared out; a caller
+    // that wants overflows flagged takes the staged form
+    const i64 npb = (G + 31) / 32;
+    const bool small = grid <= 512 && ks && L <= 8 * ks && L >= 8 * (ks - 1) && !flag;
+    const unsigned gy = (unsigned)(!small ? 1 : (1024 / grid < npb ? 1024 / grid : npb));
+    static bool attr_set[10] = {};
+#define SDPV_SPLIT_LAUNCH(KSC, SM)                                                                             \
     do {                                                                                                       \
-        if (!attr_set[KSC]) {                                                                                  \
-            (void)hipFuncSetAttribute((const void*)k_rns_split<KSC>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                      160 * 1024);                                                             \
-            attr_set[KSC] = true;                                                                              \
+        if (!attr_set[KSC + 5 * SM]) {                                                                         \
+            (void)hipFuncSetAttribute((const void*)k_rns_split<KSC, SM>,                                       \
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                 \
+            attr_set[KSC + 5 * SM] = true;                                                                     \
         }                                                                                                      \
-        hipLaunchKernelGGL((k_rns_split<KSC>), dim3((unsigned)grid), dim3(256), lds, as_stream(stream), X, e,   \
+        hipLaunchKernelGGL((k_rns_split<KSC, SM>), dim3((unsigned)grid, gy), dim3(256), lds, as_stream(stream), X, e, \
                            Erow, (int)L, (int)Lout, (i64)plane, (i64)nb, (i64)rows, (i64)ldb, (i64)ldr, (i64)ldk, \
                            (i64)k0, (i64)kc, (i64)kp, Thi, Tlo, (int)NBp, C1, mods, minv, (int)g0, (int)G, Rh, Rl, \
                            flag, ntiles_k, stage);                                                             \
     } while (0)
-    switch (ks) {
-        case 1: SDPV_SPLIT_LAUNCH(1); break;
-        case 2: SDPV_SPLIT_LAUNCH(2); break;
-        case 3: SDPV_SPLIT_LAUNCH(3); break;
-        case 4: SDPV_SPLIT_LAUNCH(4); break;
-        default: SDPV_SPLIT_LAUNCH(0); break;
+    switch (small ? ks + 5 : ks) {
+        case 1: SDPV_SPLIT_LAUNCH(1, false); break;
+        case 2: SDPV_SPLIT_LAUNCH(2, false); break;
+        case 3: SDPV_SPLIT_LAUNCH(3, false); break;
+        case 4: SDPV_SPLIT_LAUNCH(4, false); break;
+        case 6: SDPV_SPLIT_LAUNCH(1, true); break;
+        case 7: SDPV_SPLIT_LAUNCH(2, true); break;
+        case 8: SDPV_SPLIT_LAUNCH(3, true); break;
+        case 9: SDPV_SPLIT_LAUNCH(4, true); break;
+        default: SDPV_SPLIT_LAUNCH(0, false); break;
     }
 #undef SDPV_SPLIT_LAUNCH
     SDPV_TRY_LAUNCH();
