@@ -321,6 +321,19 @@ int64_t sdpv_encode_bigfloats(const int32_t* in, const int64_t* exps, int64_t n,
 
 /* ---------------------------------------------------------------- diagnostics */
 
+/* sdpv_rns_crt in its ROUND mode on a scaled accumulator, into a block of a larger array: limb k of entry
+ * (i, jj), i < rows, jj < w, goes to outm[k * plane + (i / Mb) * ob + (i % Mb) * ldo + jo + jj]. The shift is
+ * scol[(i / Mb) * cld + jo + jj], or s0 everywhere when scol is null. With X the result is
+ * X + sgn * round(value) modulo 2^(32 L) (sgn +1 or -1), X read at
+ * X[k * xplane + (i / Mb) * xb + (i % Mb) * xld + jj]; X may be the output itself. Replaces the product's
+ * rounding and the exact addition that follows it in the Cholesky recursion
+ * (sdpvibe/batched.py:165-231, sdpvibe/limbops.py:188-193). */
+int sdpv_rns_crt_fixed(const int16_t* acc, int64_t n, int64_t ld_g, int64_t rows, int64_t N, int64_t j0,
+                       int64_t w, const int32_t* mods, const double* minv, const int32_t* inv, const int8_t* Ct,
+                       int64_t E, int64_t npad, int32_t* outm, int64_t L, int64_t plane, int64_t ldo, int64_t jo,
+                       int64_t ob, int64_t Mb, int64_t s0, const int64_t* scol, int64_t cld, const int32_t* X,
+                       int64_t xplane, int64_t xld, int64_t xb, int32_t sgn, int32_t* flag, void* stream);
+
 /* D = A * B through one wave of v_mfma_i32_32x32x32_i8 using the same fragment mapping as the
  * GEMM kernels. A: (32, 32) int8 row-major, B: (32, 32) int8 row-major (k, n), D: (32, 32) int32.
  * No counterpart in the reference: a self-test of the matrix-core operand layout. */

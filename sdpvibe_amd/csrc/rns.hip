@@ -603,6 +603,101 @@ int launch_gemm(const int8_t* Ah, const int8_t* Al, const int8_t* Bh, const int8
 // Phase 3 (lane = entry): words -> W + bitlen (mode 0), normalised MPF limbs (1), or a
 //   fixed-exponent rounding (2).
 
+// where a reconstruction goes: limbs outm + k * plane + (i / Mb) * ob + (i % Mb) * ldo + jo + jj of entry (i, jj)
+// (exponents at the same offset); with X (fixed exponent) the result is X + sgn * value modulo 2^(32 L), X laid
+// out likewise at its own strides
+struct CrtOut {
+    i64 plane, ldo, jo, ob;
+    const i32* X;
+    i64 xplane, xld, xb;
+    i64 cld;                                            // entries of ecol and scol per block of Mb rows
+    i64 s0;                                             // shift when scol is null
+    int sgn;
+};
+
+// phase 3 (lane = entry; reads only its own LDS row, in batches of independent reads): words -> limbs of entry
+// (ib, jj) of block bi, row i overall; xl: the addend's limbs in LDS (xl[64 k]), or null to read them in place
+__device__ __forceinline__ void crt_emit(const u32* wrow, int NW, int mode, i64 i, i64 bi, i64 ib, i64 jj, int L,
+                                         const u32* xl, i32* __restrict__ outm, i64* __restrict__ oute, const CrtOut& R,
+                                         const i64* __restrict__ erow, const i64* __restrict__ ecol,
+                                         const i64* __restrict__ scol, i32* __restrict__ flag) {
+    const i64 plane = R.plane, o = bi * R.ob + ib * R.ldo + R.jo + jj;
+    const i64 cidx = bi * R.cld + R.jo + jj;            // of ecol and scol
+    const u32 ext = (wrow[NW - 1] >> 31) ? 0xffffffffu : 0u;   // sign extension word
+    const LdsWords src{wrow};
+    // word t of the value's two's complement: zero below 0, the sign extension above NW - 1
+    auto wd = [&](int t) -> u32 {
+        const u32 v = wrow[t < 0 ? 0 : (t >= NW ? NW - 1 : t)];
+        return t < 0 ? 0u : (t >= NW ? ext : v);
+    };
+    i64 sv;                                           // shift: out = (v + rounding) / 2^sv
+    u32 c = 0;                                        // rounding carry into bit sv
+    if (mode == SDPV_CRT_NORMALIZE) {
+        // bit length of |v|: top word T of v ^ ext; for v < 0 also the lowest nonzero word z, as
+        // |v| = ~v above z, -v_z at z (mpf.py normalize via bitlen of the magnitude)
+        const bool neg = ext != 0u;
+        int T = -1;
+        u32 wT = 0;
+        for (int b = NW - 1; b >= 0 && T < 0; b -= 8) {
+            u32 x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = (b - u >= 0) ? wd(b - u) ^ ext : 0u;
+#pragma unroll
+            for (int u = 7; u >= 0; u--)
+                if (x[u] != 0u) { T = b - u; wT = x[u]; }
+        }
+        int z = -1;
+        u32 vz = 0;
+        if (neg) {
+            for (int b = 0; b < NW && z < 0; b += 8) {
+                u32 x[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) x[u] = wd(b + u);
+#pragma unroll
+                for (int u = 7; u >= 0; u--)
+                    if (x[u] != 0u && b + u < NW) { z = b + u; vz = x[u]; }
+            }
+        }
+        int bl;
+        if (!neg) bl = T < 0 ? 0 : 32 * T + 32 - clz32(wT);
+        else bl = T > z ? 32 * T + 32 - clz32(wT) : 32 * z + 32 - clz32(0u - vz);
+        if (bl == 0) {
+            for (int k = 0; k < L; k++) outm[(i64)k * plane + o] = 0;
+            oute[o] = EZV;
+            return;
+        }
+        sv = bl - (32 * L - 2);
+        if (sv > 0) {
+            // -round_half_up(|v| / 2^sv) = floor((v + 2^(sv-1) - 1) / 2^sv) for v < 0: the carry into
+            // bit sv needs bit sv-1 and, for v < 0, a nonzero bit below it
+            const u32 rb = (wd((int)((sv - 1) >> 5)) >> (int)((sv - 1) & 31)) & 1u;
+            const bool sticky = !neg || 32 * (i64)z + __builtin_ctz(vz) < sv - 1;
+            c = (rb && sticky) ? 1u : 0u;
+        }
+        const i64 ein = (erow ? erow[i] : 0) + (ecol ? ecol[cidx] : 0);
+        oute[o] = ein + sv;
+        (void)shift_words(src, NW, ext, sv, c, L, [&](int k, u32 v) { outm[(i64)k * plane + o] = (i32)v; });
+    } else {
+        // round_half_up(v / 2^s) = floor((v + 2^(s-1)) / 2^s) (limbops._shift_round_kernel)
+        const i64 sh = scol ? scol[cidx] : R.s0;
+        int bad;
+        if (R.X) {
+            const i32* x = R.X + bi * R.xb + ib * R.xld + jj;
+            const u32 f = R.sgn < 0 ? ~0u : 0u;
+            u32 c1 = R.sgn < 0 ? 1u : 0u;
+            bad = shr_round_batched(src, NW, sh, L, [&](int k, u32 v) {
+                const u32 xk = xl ? xl[64 * k] : (u32)x[(i64)k * R.xplane];
+                const u64 t = (u64)xk + (v ^ f) + c1;
+                c1 = (u32)(t >> 32);
+                outm[(i64)k * plane + o] = (i32)(u32)t;
+            });
+        } else {
+            bad = shr_round_batched(src, NW, sh, L, [&](int k, u32 v) { outm[(i64)k * plane + o] = (i32)v; });
+        }
+        if (bad && flag) atomicOr(flag, 1);
+    }
+}
+
 // NDB > 0 (modes 1, 2 with that many digit blocks): the words of an entry stay in registers
 // during phase 2 and move into the then unused byte rows afterwards, so a wave needs only the
 // byte rows of LDS (more waves per CU); NDB = 0: words in their own LDS rows, digit blocks
@@ -612,7 +707,7 @@ __global__ void __launch_bounds__(64) k_rns_crt(
     const int16_t* __restrict__ acc, int n, i64 ld_g, i64 rows, i64 N, i64 j0, i64 w, const i32* __restrict__ mods,
     const double* __restrict__ minv, const i32* __restrict__ inv, const int8_t* __restrict__ Ct, int E, int npad,
     int mode, i32* __restrict__ W, i64* __restrict__ bitlen, i32* __restrict__ outm, i64* __restrict__ oute, int L,
-    i64 plane, i64 ldo, i64 jo, i64 Mb, const i64* __restrict__ erow, const i64* __restrict__ ecol,
+    CrtOut R, i64 Mb, const i64* __restrict__ erow, const i64* __restrict__ ecol,
     const i64* __restrict__ scol, i32* __restrict__ flag) {
     SDPV_DYNAMIC_LDS(unsigned char, smem);
     const int YS = npad + 16;                         // bytes per entry row (multiple of 16)
@@ -810,9 +905,8 @@ __global__ void __launch_bounds__(64) k_rns_crt(
         }
     }
 
-    // ---- phase 3 (lane = entry; reads only its own LDS row, in batches of independent reads)
+    // ---- phase 3
     if (!qok) return;
-    const i64 i = q / w, jj = q % w;
     if (mode == SDPV_CRT_WORDS) {
         const bool neg = (lastw >> 31) != 0;
         const int last = neg ? last1 : last0;
@@ -820,67 +914,170 @@ __global__ void __launch_bounds__(64) k_rns_crt(
         bitlen[q] = last >= 0 ? 32 * (i64)last + 32 - clz32(top) : 0;
         return;
     }
-    const i64 o = i * ldo + jo + jj;
-    const i64 cidx = (i / Mb) * ldo + jo + jj;
-    const u32 ext = (wrow[NW - 1] >> 31) ? 0xffffffffu : 0u;   // sign extension word
-    const LdsWords src{wrow};
-    // word t of the value's two's complement: zero below 0, the sign extension above NW - 1
-    auto wd = [&](int t) -> u32 {
-        const u32 v = wrow[t < 0 ? 0 : (t >= NW ? NW - 1 : t)];
-        return t < 0 ? 0u : (t >= NW ? ext : v);
+    const i64 i = q / w, bi = i / Mb;
+    crt_emit(wrow, NW, mode, i, bi, i - bi * Mb, q - i * w, L, nullptr, outm, oute, R, erow, ecol, scol, flag);
+}
+
+// The same reconstruction with four waves for the 64 entries, for launches too small to fill the device (scaled
+// input): a launch then takes one chain of dependent steps, which is a quarter as long here. Each wave takes
+// a quarter of the primes in phase 1 (all its loads at once) and every fourth digit block in phase 2, whose
+// 64-bit word partials meet in LDS; wave 0 carries and rounds. The reconstructions of chol(Q) at N = 3000,
+// L = 24: 17.2 us on average before, 13.4 now (15.6 with the addend, whose own pass took 9.3).
+__global__ void __launch_bounds__(256) k_rns_crt4(
+    const int16_t* __restrict__ acc, int n, i64 ld_g, i64 rows, i64 N, i64 j0, i64 w, const double* __restrict__ minv,
+    const int8_t* __restrict__ Ct, int E, int npad, int mode, i32* __restrict__ W, i64* __restrict__ bitlen,
+    i32* __restrict__ outm, i64* __restrict__ oute, int L, CrtOut R, i64 Mb, const i64* __restrict__ erow,
+    const i64* __restrict__ ecol, const i64* __restrict__ scol, i32* __restrict__ flag) {
+    SDPV_DYNAMIC_LDS(unsigned char, smem);
+    const int YS = npad + 16, NW = E / 4, nDB = (E + 31) / 32, nK = npad / 32;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int8_t* Yh = (int8_t*)smem;                       // [64][YS]
+    int8_t* Yl = Yh + 64 * YS;                        // [64][YS]
+    u64* part = (u64*)(smem + 128 * YS);              // [8 nDB][64] word partials
+    double* sums = (double*)(part + 512 * nDB);       // [4][64] partial sums of y_g / m_g
+    u32* wrow = (u32*)smem + (size_t)lane * (NW + 1);   // wave 0's words, over the byte rows
+    u32* xl = (u32*)(sums + 256) + lane;              // [L][64] limbs of the addend
+    const u32 Bq = rows * w, q = blockIdx.x * 64 + lane;   // at most 65536 entries: 32-bit divisions
+    const bool qok = q < Bq;
+    const u32 i = qok ? q / (u32)w : 0u, jj = qok ? q - i * (u32)w : 0u, bi = i / (u32)Mb;
+    const u32 boff = (u32)((i * N + j0 + jj) * 2);
+
+    // this wave's share of the addend's limbs (every fourth)
+    const i32* px = R.X ? R.X + bi * R.xb + (i - bi * Mb) * R.xld + jj : nullptr;
+    u32 xv[8];
+    if (px) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) xv[u] = (u32)px[(i64)(4 * u + wave < L ? 4 * u + wave : 0) * R.xplane];
+    }
+    // the first four chunks of this wave's first digit block: in flight during phase 1
+    auto load_ct = [&](int db, v4i (&c)[4]) {
+        const int8_t* crow = Ct + (i64)((db < nDB ? db : 0) * 32 + l32) * npad + 16 * half;
+#pragma unroll
+        for (int k = 0; k < 4; k++) c[k] = k < nK ? *(const v4i*)(crow + 32 * k) : zero4();
     };
-    i64 sv;                                           // shift: out = (v + rounding) / 2^sv
-    u32 c = 0;                                        // rounding carry into bit sv
-    if (mode == SDPV_CRT_NORMALIZE) {
-        // bit length of |v|: top word T of v ^ ext; for v < 0 also the lowest nonzero word z, as
-        // |v| = ~v above z, -v_z at z (mpf.py normalize via bitlen of the magnitude)
-        const bool neg = ext != 0u;
-        int T = -1;
-        u32 wT = 0;
-        for (int b = NW - 1; b >= 0 && T < 0; b -= 8) {
-            u32 x[8];
+    v4i c0[4], c1[4];
+    load_ct(wave, c0);
+
+    // ---- phase 1: groups of 16 primes, group index = wave mod 4, two groups in flight
+    double sp[2] = {0.0, 0.0};
+    for (int gc = 16 * wave; gc < npad; gc += 128) {
+        int a[32];
 #pragma unroll
-            for (int u = 0; u < 8; u++) x[u] = (b - u >= 0) ? wd(b - u) ^ ext : 0u;
-#pragma unroll
-            for (int u = 7; u >= 0; u--)
-                if (x[u] != 0u) { T = b - u; wT = x[u]; }
+        for (int u = 0; u < 32; u++) {
+            const int g = gc + u + (u >= 16 ? 48 : 0);
+            a[u] = g < n ? *(const int16_t*)((const char*)(acc + (i64)g * ld_g) + boff) : 0;
         }
-        int z = -1;
-        u32 vz = 0;
-        if (neg) {
-            for (int b = 0; b < NW && z < 0; b += 8) {
-                u32 x[8];
 #pragma unroll
-                for (int u = 0; u < 8; u++) x[u] = wd(b + u);
+        for (int h = 0; h < 2; h++) {
+            const int g0 = gc + 64 * h;
+            if (g0 >= npad) break;
+            int hi[16], lo[16];
 #pragma unroll
-                for (int u = 7; u >= 0; u--)
-                    if (x[u] != 0u && b + u < NW) { z = b + u; vz = x[u]; }
+            for (int u = 0; u < 16; u++) {
+                const int x = a[16 * h + u];
+                sp[u & 1] = fma((double)x, minv[g0 + u < n ? g0 + u : n - 1], sp[u & 1]);
+                hi[u] = (x + 64) >> 7;
+                lo[u] = x - (hi[u] << 7);
+            }
+            v4i vh, vl;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                vh[c] = (int)pack4(hi[4 * c], hi[4 * c + 1], hi[4 * c + 2], hi[4 * c + 3]);
+                vl[c] = (int)pack4(lo[4 * c], lo[4 * c + 1], lo[4 * c + 2], lo[4 * c + 3]);
+            }
+            *(v4i*)(Yh + (size_t)lane * YS + g0) = vh;
+            *(v4i*)(Yl + (size_t)lane * YS + g0) = vl;
+        }
+    }
+    sums[wave * 64 + lane] = sp[0] + sp[1];
+    if (px) {
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (4 * u + wave < L) xl[64 * (4 * u + wave)] = xv[u];
+        for (int k = 32 + wave; k < L; k += 4) xl[64 * k] = (u32)px[(i64)k * R.xplane];
+    }
+    __syncthreads();
+    if (wave == 0) {                                  // column n: -k
+        const int nk = -(int)rint((sums[lane] + sums[64 + lane]) + (sums[128 + lane] + sums[192 + lane]));
+        const int kl = ((nk + 64) & 127) - 64;
+        Yh[(size_t)lane * YS + n] = (int8_t)((nk - kl) >> 7);
+        Yl[(size_t)lane * YS + n] = (int8_t)kl;
+    }
+    __syncthreads();
+
+    // ---- phase 2: digit blocks wave, wave + 4, ...
+    const int8_t* y0h = Yh + (size_t)l32 * YS + 16 * half;
+    const int8_t* y0l = Yl + (size_t)l32 * YS + 16 * half;
+    for (int db = wave; db < nDB; db += 4) {
+        load_ct(db + 4, c1);
+        v16i z[4] = {zero16(), zero16(), zero16(), zero16()};
+        auto step = [&](v4i c, int kb) {
+            const int o = kb * 32;
+            z[0] = mfma(c, *(const v4i*)(y0h + o), z[0]);
+            z[1] = mfma(c, *(const v4i*)(y0l + o), z[1]);
+            z[2] = mfma(c, *(const v4i*)(y0h + 32 * YS + o), z[2]);
+            z[3] = mfma(c, *(const v4i*)(y0l + 32 * YS + o), z[3]);
+        };
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++)
+            if (kb < nK) step(c0[kb], kb);
+        const int8_t* crow = Ct + (i64)(db * 32 + l32) * npad + 16 * half;
+        for (int kb = 4; kb < nK; kb++) step(*(const v4i*)(crow + 32 * kb), kb);
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) c0[kb] = c1[kb];
+        // word partials sum_u Z_u 256^u: even words in the lower lane half, odd ones in the upper
+#pragma unroll
+        for (int wq = 0; wq < 4; wq++) {
+            i64 v0 = 0, v1 = 0;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                v0 += (i64)(128 * z[0][4 * wq + u] + z[1][4 * wq + u]) << (8 * u);
+                v1 += (i64)(128 * z[2][4 * wq + u] + z[3][4 * wq + u]) << (8 * u);
+            }
+            u64* p = part + (size_t)(db * 8 + 2 * wq + half) * 64 + l32;
+            p[0] = (u64)v0;
+            p[32] = (u64)v1;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+
+    // ---- carries and phase 3 on wave 0, lane = entry
+    i64 carry = 0;
+    int last0 = -1, last1 = -1;
+    u32 w0 = 0, w1 = 0, lastw = 0;
+    for (int t = 0; t < NW; t += 8) {
+        u64 p[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) p[u] = part[(size_t)(t + u) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            if (t + u < NW) {
+                const i64 v = carry + (i64)p[u];
+                carry = v >> 32;
+                const u32 x = (u32)v;
+                if (mode == SDPV_CRT_WORDS) {
+                    if (qok) W[(i64)(t + u) * Bq + q] = (i32)x;
+                    if (x != 0u) { last0 = t + u; w0 = x; }
+                    if (x != 0xffffffffu) { last1 = t + u; w1 = ~x; }
+                    lastw = x;
+                } else {
+                    wrow[t + u] = x;
+                }
             }
         }
-        int bl;
-        if (!neg) bl = T < 0 ? 0 : 32 * T + 32 - clz32(wT);
-        else bl = T > z ? 32 * T + 32 - clz32(wT) : 32 * z + 32 - clz32(0u - vz);
-        if (bl == 0) {
-            for (int k = 0; k < L; k++) outm[(i64)k * plane + o] = 0;
-            oute[o] = EZV;
-            return;
-        }
-        sv = bl - (32 * L - 2);
-        if (sv > 0) {
-            // -round_half_up(|v| / 2^sv) = floor((v + 2^(sv-1) - 1) / 2^sv) for v < 0: the carry into
-            // bit sv needs bit sv-1 and, for v < 0, a nonzero bit below it
-            const u32 rb = (wd((int)((sv - 1) >> 5)) >> (int)((sv - 1) & 31)) & 1u;
-            const bool sticky = !neg || 32 * (i64)z + __builtin_ctz(vz) < sv - 1;
-            c = (rb && sticky) ? 1u : 0u;
-        }
-        const i64 ein = (erow ? erow[i] : 0) + (ecol ? ecol[cidx] : 0);
-        oute[o] = ein + sv;
-        (void)shift_words(src, NW, ext, sv, c, L, [&](int k, u32 v) { outm[(i64)k * plane + o] = (i32)v; });
-    } else {
-        // round_half_up(v / 2^s) = floor((v + 2^(s-1)) / 2^s) (limbops._shift_round_kernel)
-        const int bad = shr_round_batched(src, NW, scol[cidx], L, [&](int k, u32 v) { outm[(i64)k * plane + o] = (i32)v; });
-        if (bad && flag) atomicOr(flag, 1);
     }
+    // ---- phase 3
+    if (!qok) return;
+    if (mode == SDPV_CRT_WORDS) {
+        const bool neg = (lastw >> 31) != 0;
+        const int last = neg ? last1 : last0;
+        const u32 top = neg ? w1 : w0;
+        bitlen[q] = last >= 0 ? 32 * (i64)last + 32 - clz32(top) : 0;
+        return;
+    }
+    crt_emit(wrow, NW, mode, i, bi, i - bi * Mb, jj, L, xl, outm, oute, R, erow, ecol, scol, flag);
 }
 
 // ================================================================== MFMA layout self-test
@@ -895,6 +1092,72 @@ __global__ void __launch_bounds__(64) k_mfma_selftest(const int8_t* A, const int
     }
     v16i d = mfma(fa, fb, zero16());
     for (int j = 0; j < 16; j++) D[(8 * (j >> 2) + 4 * hsel + (j & 3)) * 32 + l32] = d[j];
+}
+
+int crt_run(const int16_t* acc, i64 n, i64 ld_g, i64 rows, i64 N, i64 j0, i64 w, const i32* mods, const double* minv,
+            const i32* inv, const int8_t* Ct, i64 E, i64 npad, int mode, i32* W, i64* bitlen, i32* outm, i64* oute, i64 L,
+            const CrtOut& R, i64 Mb, const i64* erow, const i64* ecol, const i64* scol, i32* flag, hipStream_t st) {
+    if (n < 1 || rows < 0 || N < 0 || j0 < 0 || w < 0 || E < 4 || E % 4 != 0 || npad <= n || npad % 32 != 0)
+        return SDPV_EARG;
+    const int omode = mode & ~SDPV_CRT_SCALED;
+    if (omode < 0 || omode > 2) return SDPV_EARG;
+    const i64 Bq = rows * w;
+    if (Bq == 0) return SDPV_OK;
+    if (!acc || !mods || !minv || !inv || !Ct) return SDPV_EARG;
+    if (omode == SDPV_CRT_WORDS && (!W || !bitlen)) return SDPV_EARG;
+    if (omode != SDPV_CRT_WORDS && (!outm || L < 1 || Mb < 1)) return SDPV_EARG;
+    if (omode == SDPV_CRT_NORMALIZE && !oute) return SDPV_EARG;
+    if (npad > 1024) return SDPV_ESIZE;  // digit sums 128*Zh + Zl stay within int32
+    if ((rows - 1) * N + j0 + w > ld_g || ld_g >= (1LL << 31)) return SDPV_ESIZE;  // 32-bit plane offsets
+    const i64 NW = E / 4;
+    const int ndb = (int)((E + 31) / 32);
+    const bool scaled = (mode & SDPV_CRT_SCALED) != 0;
+    // register-held words: scaled input, limb output, 5..8 digit blocks (about L = 16..31; more
+    // words would cost the wave count that the smaller LDS gains)
+    const int reg = (scaled && omode != SDPV_CRT_WORDS && ndb >= 5 && ndb <= 8) ? ndb : 0;
+    const size_t ybytes = (size_t)128 * (npad + 16), wbytes = (size_t)256 * (NW + 1);
+    const size_t lds = omode == SDPV_CRT_WORDS ? ybytes : (reg ? (ybytes > wbytes ? ybytes : wbytes) : ybytes + wbytes);
+    if (lds > 160 * 1024) return SDPV_ESIZE;
+    const i64 grid = (Bq + 63) / 64;
+    if (grid > 0x7fffffffLL) return SDPV_ESIZE;
+    // four waves per 64 entries up to 1024 workgroups (four per CU; more of them fill the device as single waves,
+    // which need a third of the LDS)
+    const size_t lds4 = ybytes + (size_t)4096 * ndb + 2048 + (R.X ? 256 * (size_t)L : 0);
+    if (scaled && grid <= 1024 && lds4 <= 80 * 1024 && wbytes <= ybytes) {
+        static bool attr4 = false;
+        if (!attr4) {
+            (void)hipFuncSetAttribute((const void*)k_rns_crt4, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            attr4 = true;
+        }
+        const i64 mb = Mb < 1 ? 1 : (Mb < rows ? Mb : rows);
+        hipLaunchKernelGGL(k_rns_crt4, dim3((unsigned)grid), dim3(256), lds4, st, acc, (int)n, ld_g, rows, N, j0, w, minv,
+                           Ct, (int)E, (int)npad, omode, W, bitlen, outm, oute, (int)L, R, mb, erow, ecol, scol, flag);
+        SDPV_TRY_LAUNCH();
+        return SDPV_OK;
+    }
+#define SDPV_CRT_LAUNCH(SC, ND)                                                                                \
+    do {                                                                                                       \
+        static bool attr = false;                                                                              \
+        if (!attr) {                                                                                           \
+            (void)hipFuncSetAttribute((const void*)k_rns_crt<SC, ND>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                      160 * 1024);                                                             \
+            attr = true;                                                                                       \
+        }                                                                                                      \
+        hipLaunchKernelGGL((k_rns_crt<SC, ND>), dim3((unsigned)grid), dim3(64), lds, st, acc, (int)n, (i64)ld_g, \
+                           (i64)rows, (i64)N, (i64)j0, (i64)w, mods, minv, inv, Ct, (int)E, (int)npad, omode, W,  \
+                           bitlen, outm, oute, (int)L, R, (i64)Mb, erow, ecol, scol, flag);                     \
+    } while (0)
+    if (!scaled) SDPV_CRT_LAUNCH(false, 0);
+    else switch (reg) {
+        case 5: SDPV_CRT_LAUNCH(true, 5); break;
+        case 6: SDPV_CRT_LAUNCH(true, 6); break;
+        case 7: SDPV_CRT_LAUNCH(true, 7); break;
+        case 8: SDPV_CRT_LAUNCH(true, 8); break;
+        default: SDPV_CRT_LAUNCH(true, 0); break;
+    }
+#undef SDPV_CRT_LAUNCH
+    SDPV_TRY_LAUNCH();
+    return SDPV_OK;
 }
 
 inline unsigned nblk(i64 n, int tpb) { return (unsigned)((n + tpb - 1) / tpb); }
@@ -1016,55 +1279,21 @@ int sdpv_rns_crt(const int16_t* acc, int64_t n, int64_t ld_g, int64_t rows, int6
                  int64_t npad, int32_t mode, int32_t* W, int64_t* bitlen, int32_t* outm, int64_t* oute, int64_t L,
                  int64_t plane, int64_t ldo, int64_t jo, int64_t Mb, const int64_t* erow, const int64_t* ecol,
                  const int64_t* scol, int32_t* flag, void* stream) {
-    if (n < 1 || rows < 0 || N < 0 || j0 < 0 || w < 0 || E < 4 || E % 4 != 0 || npad <= n || npad % 32 != 0)
-        return SDPV_EARG;
-    const int omode = mode & ~SDPV_CRT_SCALED;
-    if (omode < 0 || omode > 2) return SDPV_EARG;
-    const i64 Bq = rows * w;
-    if (Bq == 0) return SDPV_OK;
-    if (!acc || !mods || !minv || !inv || !Ct) return SDPV_EARG;
-    if (omode == SDPV_CRT_WORDS && (!W || !bitlen)) return SDPV_EARG;
-    if (omode != SDPV_CRT_WORDS && (!outm || L < 1 || Mb < 1)) return SDPV_EARG;
-    if (omode == SDPV_CRT_NORMALIZE && !oute) return SDPV_EARG;
-    if (omode == SDPV_CRT_ROUND && !scol) return SDPV_EARG;
-    if (npad > 1024) return SDPV_ESIZE;  // digit sums 128*Zh + Zl stay within int32
-    if ((rows - 1) * N + j0 + w > ld_g || ld_g >= (1LL << 31)) return SDPV_ESIZE;  // 32-bit plane offsets
-    const i64 NW = E / 4;
-    const int ndb = (int)((E + 31) / 32);
-    const bool scaled = (mode & SDPV_CRT_SCALED) != 0;
-    // register-held words: scaled input, limb output, 5..8 digit blocks (about L = 16..31; more
-    // words would cost the wave count that the smaller LDS gains)
-    const int reg = (scaled && omode != SDPV_CRT_WORDS && ndb >= 5 && ndb <= 8) ? ndb : 0;
-    const size_t ybytes = (size_t)128 * (npad + 16), wbytes = (size_t)256 * (NW + 1);
-    const size_t lds = omode == SDPV_CRT_WORDS ? ybytes : (reg ? (ybytes > wbytes ? ybytes : wbytes) : ybytes + wbytes);
-    if (lds > 160 * 1024) return SDPV_ESIZE;
-    const i64 grid = (Bq + 63) / 64;
-    if (grid > 0x7fffffffLL) return SDPV_ESIZE;
-    hipStream_t st = as_stream(stream);
-#define SDPV_CRT_LAUNCH(SC, ND)                                                                                \
-    do {                                                                                                       \
-        static bool attr = false;                                                                              \
-        if (!attr) {                                                                                           \
-            (void)hipFuncSetAttribute((const void*)k_rns_crt<SC, ND>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                      160 * 1024);                                                             \
-            attr = true;                                                                                       \
-        }                                                                                                      \
-        hipLaunchKernelGGL((k_rns_crt<SC, ND>), dim3((unsigned)grid), dim3(64), lds, st, acc, (int)n, (i64)ld_g, \
-                           (i64)rows, (i64)N, (i64)j0, (i64)w, mods, minv, inv, Ct, (int)E, (int)npad, omode, W,  \
-                           bitlen, outm, oute, (int)L, (i64)plane, (i64)ldo, (i64)jo, (i64)Mb, erow, ecol, scol,  \
-                           flag);                                                                              \
-    } while (0)
-    if (!scaled) SDPV_CRT_LAUNCH(false, 0);
-    else switch (reg) {
-        case 5: SDPV_CRT_LAUNCH(true, 5); break;
-        case 6: SDPV_CRT_LAUNCH(true, 6); break;
-        case 7: SDPV_CRT_LAUNCH(true, 7); break;
-        case 8: SDPV_CRT_LAUNCH(true, 8); break;
-        default: SDPV_CRT_LAUNCH(true, 0); break;
-    }
-#undef SDPV_CRT_LAUNCH
-    SDPV_TRY_LAUNCH();
-    return SDPV_OK;
+    if ((mode & ~SDPV_CRT_SCALED) == SDPV_CRT_ROUND && rows * w != 0 && !scol) return SDPV_EARG;
+    const CrtOut R{plane, ldo, jo, Mb * ldo, nullptr, 0, 0, 0, ldo, 0, 1};
+    return crt_run(acc, n, ld_g, rows, N, j0, w, mods, minv, inv, Ct, E, npad, mode, W, bitlen, outm, oute, L, R, Mb, erow,
+                   ecol, scol, flag, as_stream(stream));
+}
+
+int sdpv_rns_crt_fixed(const int16_t* acc, int64_t n, int64_t ld_g, int64_t rows, int64_t N, int64_t j0, int64_t w,
+                       const int32_t* mods, const double* minv, const int32_t* inv, const int8_t* Ct, int64_t E,
+                       int64_t npad, int32_t* outm, int64_t L, int64_t plane, int64_t ldo, int64_t jo, int64_t ob,
+                       int64_t Mb, int64_t s0, const int64_t* scol, int64_t cld, const int32_t* X, int64_t xplane,
+                       int64_t xld, int64_t xb, int32_t sgn, int32_t* flag, void* stream) {
+    if (sgn != 1 && sgn != -1) return SDPV_EARG;
+    const CrtOut R{plane, ldo, jo, ob, X, xplane, xld, xb, cld, s0, sgn};
+    return crt_run(acc, n, ld_g, rows, N, j0, w, mods, minv, inv, Ct, E, npad, SDPV_CRT_ROUND | SDPV_CRT_SCALED, nullptr,
+                   nullptr, outm, nullptr, L, R, Mb, nullptr, nullptr, scol, flag, as_stream(stream));
 }
 
 int sdpv_mfma_selftest(const int8_t* A, const int8_t* B, int32_t* D, void* stream) {

@@ -24,7 +24,7 @@ import os
 import numpy as np
 import torch
 
-from ._lib import call, ptr, stream
+from ._lib import call, ptr, ptr_strided, stream
 
 dev = "cuda"
 PMAX = 16257       # largest modulus with centred residues |r| <= 8128: h + l stays in int8
@@ -298,6 +298,23 @@ class RNS:
              ptr(self.inv32), ptr(self.Ct), self.E, self.npad, mode | (4 if scaled else 0), ptr(W), ptr(bitlen),
              ptr(outm), ptr(oute), L or self.L, plane, ldo, jo, Mb, ptr(erow), ptr(ecol), ptr(scol),
              ptr(flag), stream())
+
+    def crt_fixed(self, acc, nb, M, w, out, j0, s0, scol=None, plus=None, sgn=1, flag=None):
+        """columns j0..j0+w of out (L, nb, M, N), a view with unit column stride, from a scaled accumulator
+        (n, nb * M, w): round(value / 2^s) for each column's shift s (scol (nb * N,), or the int s0), or
+        plus + sgn * that modulo 2^(32 L) (plus: limbs laid out like out; it may be out itself)"""
+        L, N = out.shape[0], out.shape[3]
+        if acc.numel() < self.n * nb * M * w or not acc.is_contiguous() or j0 + w > N:
+            raise ValueError("crt: block exceeds the residue accumulator")
+        if (tuple(out.shape[1:3]) != (nb, M) or out.stride(3) != 1 or (scol is not None and scol.numel() < nb * N)
+                or (plus is not None and (plus.shape != out.shape or plus.stride(3) != 1))):
+            raise ValueError("crt: limb arrays of another shape or column stride")
+        op, ob, ld, _ = out.stride()
+        xp, xb, xld, _ = (0, 0, 0, 0) if plus is None else plus.stride()
+        x = None if plus is None else ptr_strided(plus[:, :, :, j0:])
+        call("sdpv_rns_crt_fixed", ptr(acc), self.n, nb * M * w, nb * M, w, 0, w, ptr(self.m32), ptr(self.minv),
+             ptr(self.inv32), ptr(self.Ct), self.E, self.npad, ptr_strided(out), L, op, ld, j0, ob, M, s0, ptr(scol), N,
+             x, xp, xld, xb, sgn, ptr(flag), stream())
 
     def crt_block(self, acc, N, j0, w, rows, scaled=False):
         """acc: (n, rows_total, N) int16 residues in [0, m) (scaled: the product's CRT coefficients);
