@@ -261,6 +261,14 @@ int sdpv_rns_crt(const int16_t* acc, int64_t n, int64_t ld_g, int64_t rows, int6
 int sdpv_tile_chol(const int32_t* A, int64_t L, int64_t nb, int64_t BT, int32_t* Lout, int32_t* Xw,
                    uint32_t* work, int32_t* flag, void* stream);
 
+/* sdpv_tile_chol with the inverse rounded in the same call: X (L, nb, BT, BT) to hb bits below the largest entry
+ * of its tile, Xe (nb, BT) that exponent, repeated; A read in place, limb k of entry (b, i, j) at
+ * A[k * plane + b * ldb + i * ldr + j]. work: nb * (BT * (3 * BT + 1) * (L + 24) + 1) words.
+ * Replaces batched.bchol_tile (sdpvibe/batched.py:243-257). */
+int sdpv_tile_chol_inv(const int32_t* A, int64_t plane, int64_t ldb, int64_t ldr, int64_t L, int64_t nb,
+                       int64_t BT, int32_t* Lout, int32_t* X, int64_t* Xe, int64_t hb, uint32_t* work,
+                       int32_t* flag, void* stream);
+
 /* Forward substitution L y = v with one factored tile, in place, for nvec vectors.
  * Lw: (BT, BT, WL) wide factor, RINV: (BT, WL) pivot reciprocals (both from sdpv_tile_chol's work),
  * V: (nvec, BT, WL) wide fixed-point vectors (F = 32 LF fractional bits). BT <= 32.

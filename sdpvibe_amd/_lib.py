@@ -43,6 +43,7 @@ SIGNATURES = {
     "sdpv_rns_crt_fixed": ([_P] + [_I64] * 6 + [_P] * 4 + [_I64] * 2 + [_P] + [_I64] * 7 + [_P, _I64, _P] + [_I64] * 3 + [_I32, _P, _P],
                            _I32),
     "sdpv_tile_chol": ([_P, _I64, _I64, _I64, _P, _P, _P, _P, _P], _I32),
+    "sdpv_tile_chol_inv": ([_P] + [_I64] * 6 + [_P] * 3 + [_I64] + [_P] * 3, _I32),
     "sdpv_tile_trsv": ([_P, _P, _P, _I64, _I64, _I64, _I64, _P], _I32),
     "sdpv_mpf_to_double": ([_P, _P, _I64, _I64, _P, _I64, _P, _P], _I32),
     "sdpv_mpf_from_double": ([_P, _I64, _I64, _P, _P, _P], _I32),

@@ -7,7 +7,7 @@ be tiny and their reciprocals (and X = L^-1) large, hence the integer words.
 """
 import torch
 
-from ._lib import call, ptr, stream
+from ._lib import call, ptr, ptr_strided, stream
 from .limbops import _errbuf, bitlen_words, shift_round
 from .mpmat import MP, headroom_bits, rescale
 
@@ -27,6 +27,21 @@ def tile_factor(limbs, BT):
     work = torch.empty((nb * BT * (3 * BT + 1) * WL,), dtype=torch.int32, device=A.device)
     call("sdpv_tile_chol", ptr(A), L, nb, BT, ptr(Lout), ptr(Xw), ptr(work), ptr(_errbuf()), stream())
     return Lout, Xw, work
+
+
+def tile_factor_inverse(limbs, BT, hb):
+    """limbs as for tile_factor, any view -> (Lout, X (L, nb, BT, BT) rounded to hb bits below the largest
+    entry of its tile, its exponents (nb, BT))"""
+    L, nb = limbs.shape[0], limbs.shape[1]
+    if limbs.stride(3) != 1:
+        limbs = limbs.contiguous()
+    Lout = torch.empty((L, nb, BT, BT), dtype=torch.int32, device=limbs.device)
+    X = torch.empty_like(Lout)
+    Xe = torch.empty((nb, BT), dtype=torch.int64, device=limbs.device)
+    work = torch.empty((nb * (BT * (3 * BT + 1) * (L + LI) + 1),), dtype=torch.int32, device=limbs.device)
+    call("sdpv_tile_chol_inv", ptr_strided(limbs), *limbs.stride()[:3], L, nb, BT, ptr(Lout), ptr(X), ptr(Xe), hb,
+         ptr(work), ptr(_errbuf()), stream())
+    return Lout, X, Xe
 
 
 class Tile:

@@ -301,20 +301,15 @@ class BTile:
 def bchol_tile(A, LI=24, threads=256):
     """factor and invert the bt x bt tiles A (nb, bt, bt) (fixed point at -(32L - 40)) on the GPU:
     (L as a BMP, BTile) with X rounded to headroom_bits(L) below its largest entry, per block"""
-    from .basecase import tile_factor
-    from .limbops import bitlen_words
+    from .basecase import tile_factor_inverse
     nb, b, _ = A.shape
     L = A.L
     if A.exp != -(32 * L - 40):
         raise ValueError("tiles enter at the fixed-point exponent")
-    Fb = 32 * L
-    Lw, Xw, _ = tile_factor(A.limbs, b)
-    top = bitlen_words(Xw.reshape(L + LI, -1)).view(nb, b * b).amax(1) - Fb
+    Lw, X, Xe = tile_factor_inverse(A.limbs, b, headroom_bits(L))
     tile = BTile()
     tile.res = None
-    tile.Lmp = BMP(Lw, A.exp)
-    wide = BMP(Xw, torch.full((nb, b), -Fb, dtype=torch.int64, device=Xw.device))
-    tile.X = brescale(wide, (top - headroom_bits(L)).unsqueeze(1).expand(nb, b).contiguous(), L)
+    tile.Lmp, tile.X = BMP(Lw, A.exp), BMP(X, Xe)
     return tile.Lmp, tile
 
 

@@ -54,6 +54,12 @@ inline int atomicAdd(int* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_S
 inline unsigned __builtin_amdgcn_alignbyte(unsigned hi, unsigned lo, unsigned sh) {
     return (unsigned)((((unsigned long long)hi << 32) | lo) >> (8 * (sh & 3)));
 }
+inline int atomicMax(int* p, int v) {
+    int cur = __atomic_load_n(p, __ATOMIC_SEQ_CST);
+    while (cur < v && !__atomic_compare_exchange_n(p, &cur, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST)) {
+    }
+    return cur;
+}
 inline long long atomicMax(long long* p, long long v) {
     long long cur = __atomic_load_n(p, __ATOMIC_SEQ_CST);
     while (cur < v && !__atomic_compare_exchange_n(p, &cur, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST)) {
