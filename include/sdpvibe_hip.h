@@ -143,6 +143,19 @@ int sdpv_narrow_result(const int32_t* acc, int64_t L, int64_t nb, int64_t M, int
                        const int64_t* EB, int32_t* out, int64_t plane, int64_t ob, int64_t oi, int64_t oj,
                        int64_t* oute, void* stream);
 
+/* count (r, c) blocks of limbs and exponents to (to_stack != 0) or from the stack m (L, count, rows, cols),
+ * e (count, rows, cols), r <= rows, c <= cols. `blocks` is host memory, read before the call returns; limb k of
+ * entry (i, j) of a block is at m[k * mp + i * mr + j * mc], its exponent at e[i * er + j * ec]. Entries of the
+ * stack outside a block are set to zero (exponent -2^40). Replaces the per-block copies of the batched solver's
+ * embedding (sdpvibe/solver.py:10-12). */
+typedef struct {
+    int32_t* m;
+    int64_t* e;
+    int64_t mp, mr, mc, er, ec, rows, cols;
+} sdpv_block;
+int sdpv_copy_blocks(const sdpv_block* blocks, int64_t count, int32_t* m, int64_t* e, int64_t L, int64_t rows,
+                     int64_t cols, int32_t to_stack, void* stream);
+
 /* [P1; P2] with one exponent per (block, column): P1 (L, nb, R1, C) and P2 (L, nb, R2, C) with column
  * exponents e1, e2 (nb, C), both rounded (shift_round) to EO = max(e1, e2) and written into one
  * (L, nb, R1 + R2, C) array. flag: optional int32, set when a rounding overflows. */

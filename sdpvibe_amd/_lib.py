@@ -28,6 +28,7 @@ SIGNATURES = {
     "sdpv_narrow": ([_P] * 3 + [_I64] * 4 + [_P] * 3 + [_I64] * 4 + [_I64] * 5 + [_I32, _P] + [_I64] * 4 + [_P, _I64, _P, _I64,
                      _P, _I64, _P] + [_I64] * 4 + [_P, _I32, _P, _P, _I64, _P], _I32),
     "sdpv_narrow_result": ([_P, _I64, _I64, _I64, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P], _I32),
+    "sdpv_copy_blocks": ([_P, _I64, _P, _P, _I64, _I64, _I64, _I32, _P], _I32),
     "sdpv_stack_common": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P], _I32),
     "sdpv_mpf_top": ([_P, _P, _I64, _I64, _P, _P], _I32),
     "sdpv_mpf_mul": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I32, _P], _I32),
@@ -87,6 +88,12 @@ def call(name, *args):
     rc = getattr(lib(), name)(*args)
     if rc != 0:
         raise HipLibraryError(f"{name}: {ERRORS.get(rc, rc)}")
+
+
+class Block(ctypes.Structure):
+    """sdpv_block: one (r, c) block of limbs and exponents and its strides"""
+    _fields_ = [("m", ctypes.c_void_p), ("e", ctypes.c_void_p)] + [(f, ctypes.c_int64) for f in
+                                                                   ("mp", "mr", "mc", "er", "ec", "rows", "cols")]
 
 
 def ptr(t):

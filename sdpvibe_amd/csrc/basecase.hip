@@ -1077,7 +1077,7 @@ __global__ void __launch_bounds__(TT) k_tile_trsv(const u32* __restrict__ Lw, co
 // entry after the other, odd stride) so that both the planes and the entry-major words are read and written
 // in runs, and every output word has a thread of its own. (With a thread per entry they were chains of L to
 // WL dependent strided accesses: one 32 x 32 tile at L = 24 took 17.8 us to widen, 14.7 to narrow, and 60 for the
-// bit lengths, their maximum and the rounding of the inverse; now 4.8, 7.1 and 6.0.
+// bit lengths, their maximum and the rounding of the inverse; now 4.8, 7.1 and 6.0.)
 
 // planes -> entry-major wide words, 40 more fractional bits; clears the tile's bit length
 __global__ void __launch_bounds__(256) k_tile_widen(const i32* __restrict__ A, i64 plane, i64 ldb, i64 ldr, int BT, int L,

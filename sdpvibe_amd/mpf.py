@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import batched as _batched
-from ._lib import call, ptr, stream
+from ._lib import Block, call, ptr, stream
 from .limbops import bitlen_words, shift_round
 from .mpmat import RES_BUDGET, ctx, residue_gemm
 from .rns import KMAX_LAUNCH, dev
@@ -598,6 +598,21 @@ class Chol:
         return self.solve_upper(self.solve_lower(B))
 
 
+def _copy_blocks(places, m, e, to_stack):
+    """blocks (limbs (L, r, c), exponents (r, c)), views allowed, to or from the stack m (L, nb, rows, cols),
+    e (nb, rows, cols); entries of the stack outside a block become zero (sdpv_copy_blocks)"""
+    L, nb, rows, cols = m.shape
+    blocks = (Block * nb)()
+    for b, (bm, be) in zip(blocks, places):
+        r, c = be.shape
+        if not bm.device == be.device == m.device or tuple(bm.shape) != (L, r, c) or r > rows or c > cols:
+            raise ValueError("blocks of a stack are 2-d MPF on its device that fit in it")
+        b.m, b.e, b.rows, b.cols = bm.data_ptr(), be.data_ptr(), r, c
+        b.mp, b.mr, b.mc = bm.stride()
+        b.er, b.ec = be.stride()
+    call("sdpv_copy_blocks", blocks, nb, ptr(m), ptr(e), L, rows, cols, int(to_stack), stream())
+
+
 class BucketedChol:
     """Cholesky factors and solves of SPD blocks of uneven dimension. Blocks whose dimension
     rounds up to the same multiple of bt share one batched factorisation: each is embedded with
@@ -624,12 +639,10 @@ class BucketedChol:
 
     def _embed(self, Bs, rows, cols):
         dev_ = Bs[0].m.device
-        m = torch.zeros((self.L, len(Bs), rows, cols), dtype=torch.int32, device=dev_)
-        e = torch.full((len(Bs), rows, cols), EZ, dtype=torch.int64, device=dev_)
-        for j, B in enumerate(Bs):
-            r, c = B.shape
-            m[:, j, :r, :c] = B.m
-            e[j, :r, :c] = B.e
+        m = torch.empty((self.L, len(Bs), rows, cols), dtype=torch.int32, device=dev_)
+        e = torch.empty((len(Bs), rows, cols), dtype=torch.int64, device=dev_)
+        places = [(B.m.to(m).expand(self.L, *B.shape), B.e.to(e)) for B in Bs]
+        _copy_blocks(places, m, e, True)
         return MPF(m, e)
 
     def _solve(self, Bs, which):
@@ -641,9 +654,11 @@ class BucketedChol:
             if len(cols) != 1 or any(Bs[i].shape[0] != self.dims[i] for i in idx):
                 raise ValueError("right-hand sides of one size class need the block's rows and one width")
             R = getattr(ch, which)(self._embed([Bs[i] for i in idx], ch.n, cols.pop()))
-            for j, i in enumerate(idx):
-                n = self.dims[i]
-                out[i] = MPF(R.m[:, j, :n].contiguous(), R.e[j, :n].contiguous())
+            m, e = R.m.contiguous(), R.e.contiguous()
+            for i in idx:
+                out[i] = MPF(*(torch.empty(s + (self.dims[i], e.shape[2]), dtype=x.dtype, device=x.device)
+                               for s, x in (((self.L,), m), ((), e))))
+            _copy_blocks([(out[i].m, out[i].e) for i in idx], m, e, False)
         return out
 
     def solve_lower(self, Bs):
