@@ -355,6 +355,24 @@ int sdpv_rns_crt_fixed(const int16_t* acc, int64_t n, int64_t ld_g, int64_t rows
                        int64_t ob, int64_t Mb, int64_t s0, const int64_t* scol, int64_t cld, const int32_t* X,
                        int64_t xplane, int64_t xld, int64_t xb, int32_t sgn, int32_t* flag, void* stream);
 
+/* The constants of an RNS context on its device, as the entry points above take them one by one. */
+typedef struct {
+    const int32_t *mods, *inv, *kcoef_crt, *C1;
+    const double* minv;
+    const int8_t *Thi, *Tlo, *Ct;
+    int64_t n, E, npad, NBp;
+} sdpv_rns_tables;
+
+/* mpf.gemm in one call: sdpv_row_exp and sdpv_rns_split of both operands (rows of op(A), rows of op(B)^T, strides
+ * as there), sdpv_rns_gemm over the whole inner dimension K (padded to kp) and sdpv_rns_crt's NORMALIZE mode to
+ * outm (L, nb, M, N), oute (nb, M, N). work: nwork bytes, at least the sum, each rounded up to 256, of
+ * 8 nb M, 8 nb N, n kp nb M twice, n kp nb N twice and 2 n nb M N. `T` is host memory.
+ * Replaces mpf.gemm's sequence of launches (sdpvibe/mpf.py:401-452). */
+int sdpv_rns_mpf_gemm(const sdpv_rns_tables* T, const int32_t* Am, const int64_t* Ae, int64_t aplane, int64_t aldb,
+                      int64_t aldr, int64_t aldk, const int32_t* Bm, const int64_t* Be, int64_t bplane, int64_t bldb,
+                      int64_t bldr, int64_t bldk, int64_t L, int64_t nb, int64_t M, int64_t N, int64_t K, int64_t kp,
+                      int32_t config, int32_t* outm, int64_t* oute, void* work, int64_t nwork, void* stream);
+
 /* D = A * B through one wave of v_mfma_i32_32x32x32_i8 using the same fragment mapping as the
  * GEMM kernels. A: (32, 32) int8 row-major, B: (32, 32) int8 row-major (k, n), D: (32, 32) int32.
  * No counterpart in the reference: a self-test of the matrix-core operand layout. */

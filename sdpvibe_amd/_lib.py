@@ -43,6 +43,7 @@ SIGNATURES = {
                       _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P], _I32),
     "sdpv_rns_crt_fixed": ([_P] + [_I64] * 6 + [_P] * 4 + [_I64] * 2 + [_P] + [_I64] * 7 + [_P, _I64, _P] + [_I64] * 3 + [_I32, _P, _P],
                            _I32),
+    "sdpv_rns_mpf_gemm": ([_P, _P, _P] + [_I64] * 4 + [_P, _P] + [_I64] * 10 + [_I32, _P, _P, _P, _I64, _P], _I32),
     "sdpv_tile_chol": ([_P, _I64, _I64, _I64, _P, _P, _P, _P, _P], _I32),
     "sdpv_tile_chol_inv": ([_P] + [_I64] * 6 + [_P] * 3 + [_I64] + [_P] * 3, _I32),
     "sdpv_tile_trsv": ([_P, _P, _P, _I64, _I64, _I64, _I64, _P], _I32),
@@ -94,6 +95,12 @@ class Block(ctypes.Structure):
     """sdpv_block: one (r, c) block of limbs and exponents and its strides"""
     _fields_ = [("m", ctypes.c_void_p), ("e", ctypes.c_void_p)] + [(f, ctypes.c_int64) for f in
                                                                    ("mp", "mr", "mc", "er", "ec", "rows", "cols")]
+
+
+class Tables(ctypes.Structure):
+    """sdpv_rns_tables: the device constants of an RNS context"""
+    _fields_ = [(f, ctypes.c_void_p) for f in ("mods", "inv", "kcoef_crt", "C1", "minv", "Thi", "Tlo", "Ct")] + \
+               [(f, ctypes.c_int64) for f in ("n", "E", "npad", "NBp")]
 
 
 def ptr(t):

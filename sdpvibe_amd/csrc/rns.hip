@@ -1296,6 +1296,48 @@ int sdpv_rns_crt_fixed(const int16_t* acc, int64_t n, int64_t ld_g, int64_t rows
                    nullptr, outm, nullptr, L, R, Mb, nullptr, nullptr, scol, flag, as_stream(stream));
 }
 
+// One call for the six launches of a small product: issued one by one through the bindings, each with its
+// own checks and allocations, they took 80 us of host time against 37 us on the device (20 blocks of
+// 27 x 14 x 27, L = 14); now 35 together.
+int sdpv_rns_mpf_gemm(const sdpv_rns_tables* T, const int32_t* Am, const int64_t* Ae, int64_t aplane, int64_t aldb,
+                      int64_t aldr, int64_t aldk, const int32_t* Bm, const int64_t* Be, int64_t bplane, int64_t bldb,
+                      int64_t bldr, int64_t bldk, int64_t L, int64_t nb, int64_t M, int64_t N, int64_t K, int64_t kp,
+                      int32_t config, int32_t* outm, int64_t* oute, void* work, int64_t nwork, void* stream) {
+    if (!T || L < 1 || nb < 1 || M < 1 || N < 1 || K < 1 || kp < K || kp % 32 || !work) return SDPV_EARG;
+    char* p = (char*)work;
+    i64 left = nwork;
+    bool fits = true;
+    auto take = [&](i64 bytes) {                      // the next 256-byte aligned part of the scratch
+        char* q = p;
+        const i64 step = (bytes + 255) / 256 * 256;
+        fits = fits && step <= left;
+        left -= step;
+        p += step;
+        return (void*)q;
+    };
+    const i64 G = T->n, ra = G * kp * nb * M, rb = G * kp * nb * N;
+    i64 *EA = (i64*)take(8 * nb * M), *EB = (i64*)take(8 * nb * N);
+    int8_t *Ah = (int8_t*)take(ra), *Al = (int8_t*)take(ra), *Bh = (int8_t*)take(rb), *Bl = (int8_t*)take(rb);
+    int16_t* acc = (int16_t*)take(2 * G * nb * M * N);
+    if (!fits) return SDPV_ESIZE;
+    int rc = sdpv_row_exp(Am, Ae, L, aplane, nb, M, K, aldb, aldr, aldk, EA, stream);
+    if (rc == SDPV_OK) rc = sdpv_row_exp(Bm, Be, L, bplane, nb, N, K, bldb, bldr, bldk, EB, stream);
+    if (rc == SDPV_OK)
+        rc = sdpv_rns_split(Am, Ae, EA, L, L, aplane, nb, M, aldb, aldr, aldk, 0, K, kp, T->Thi, T->Tlo, T->NBp, T->C1,
+                            T->mods, T->minv, 0, G, Ah, Al, nullptr, stream);
+    if (rc == SDPV_OK)
+        rc = sdpv_rns_split(Bm, Be, EB, L, L, bplane, nb, N, bldb, bldr, bldk, 0, K, kp, T->Thi, T->Tlo, T->NBp, T->C1,
+                            T->mods, T->minv, 0, G, Bh, Bl, nullptr, stream);
+    if (rc == SDPV_OK)
+        rc = sdpv_rns_gemm(Ah, Al, Bh, Bl, G, nb, M, N, kp, acc, nb * M * N, T->mods, T->minv, T->kcoef_crt, 0, 4, config,
+                           stream);
+    if (rc == SDPV_OK)
+        rc = sdpv_rns_crt(acc, G, nb * M * N, nb * M, N, 0, N, T->mods, T->minv, T->inv, T->Ct, T->E, T->npad,
+                          SDPV_CRT_NORMALIZE | SDPV_CRT_SCALED, nullptr, nullptr, outm, oute, L, nb * M * N, N, 0, M, EA,
+                          EB, nullptr, nullptr, stream);
+    return rc;
+}
+
 int sdpv_mfma_selftest(const int8_t* A, const int8_t* B, int32_t* D, void* stream) {
     if (!A || !B || !D) return SDPV_EARG;
     hipLaunchKernelGGL(k_mfma_selftest, dim3(1), dim3(64), 0, as_stream(stream), A, B, D);

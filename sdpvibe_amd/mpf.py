@@ -9,6 +9,7 @@ Elementwise ops are gfx950 kernels (one thread per entry); matrix products go th
 RNS GEMM on INT8 matrix cores with operands aligned per row (A) / per column (B) -- the usual
 normwise floating-point error -- and every output entry rounded once.
 """
+import ctypes
 import os
 
 import mpmath as mp
@@ -18,8 +19,8 @@ import torch
 from . import batched as _batched
 from ._lib import Block, call, ptr, stream
 from .limbops import bitlen_words, shift_round
-from .mpmat import RES_BUDGET, ctx, residue_gemm
-from .rns import KMAX_LAUNCH, dev
+from .mpmat import RES_BUDGET, ctx, panelled, residue_gemm
+from .rns import KMAX_LAUNCH, dev, tuned_config
 
 EZ = -(1 << 40)                                      # exponent of zero
 LMAX_WIDE = 1 << 20                                  # normalize() takes any input width
@@ -345,6 +346,11 @@ def _geometry(shape, trans):
     return r, c, r * c, c, 1
 
 
+# scratch up to which gemm issues its launches in one native call: one MI355X takes under about 150 us for
+# such a product, so that the host's time shows; above it one allocation would only grow
+SMALL_GEMM = 1 << 26
+
+
 def gemm(A, B, transA=False, transB=False):
     """C = op(A) op(B) (2-d, or batched 3-d (nb, ., .)); exact products, rounded once per entry
     (operands aligned per row of op(A) / column of op(B): normwise floating-point error)
@@ -364,6 +370,22 @@ def gemm(A, B, transA=False, transB=False):
     N, K2, bldb, bldr, bldk = _geometry(Be.shape, not transB)   # rows of op(B)^T = columns of op(B)
     assert K == K2, (A.shape, B.shape, transA, transB)
     R = ctx(L)
+    narrow = _batched._narrow(max(M, N), min(M, N), K, L)
+    if not narrow and nb * M * N * K != 0 and K <= R.kmax:
+        kp = R.kp_product(K)
+        up = lambda x: (x + 255) & ~255
+        nwork = up(8 * nb * M) + up(8 * nb * N) + 2 * up(R.n * kp * nb * M) + 2 * up(R.n * kp * nb * N) + \
+            up(2 * R.n * nb * M * N)
+        if nwork <= SMALL_GEMM and not panelled(R.n, nb, M, N, K):
+            if Am.numel() < L * Ae.numel() or Bm.numel() < L * Be.numel():
+                raise ValueError("gemm: limb planes smaller than the exponents")
+            out_m = torch.empty((L, nb, M, N), dtype=torch.int32, device=dev)
+            out_e = torch.empty((nb, M, N), dtype=torch.int64, device=dev)
+            work = torch.empty((nwork,), dtype=torch.uint8, device=dev)
+            call("sdpv_rns_mpf_gemm", ctypes.byref(R.tables), ptr(Am), ptr(Ae), Ae.numel(), aldb, aldr, aldk, ptr(Bm),
+                 ptr(Be), Be.numel(), bldb, bldr, bldk, L, nb, M, N, K, kp, tuned_config(R, nb, M, N, kp), ptr(out_m),
+                 ptr(out_e), ptr(work), nwork, stream())
+            return MPF(out_m, out_e)
     EA = _row_exp(Am, Ae, L, Ae.numel(), nb, M, K, aldb, aldr, aldk)
     EB = _row_exp(Bm, Be, L, Be.numel(), nb, N, K, bldb, bldr, bldk)
     out_m = torch.empty((L, nb, M, N), dtype=torch.int32, device=dev)
@@ -371,7 +393,7 @@ def gemm(A, B, transA=False, transB=False):
     if nb * M * N == 0:
         return MPF(out_m, out_e)
 
-    if _batched._narrow(max(M, N), min(M, N), K, L):
+    if narrow:
         # one side has few rows: the direct product, the other side read once as it is stored
         work, nwork = _batched.narrow_work(L, nb, max(M, N), min(M, N), K, out_m.device)
         opA = (ptr(Am), ptr(Ae), ptr(EA), Ae.numel(), aldb, aldr, aldk)

@@ -185,6 +185,11 @@ def ctx(L):
     return _ctx[key]
 
 
+def panelled(n, nb, M, N, K):
+    """whether residue_gemm takes column panels or parts of the inner dimension for this shape"""
+    return n * nb * M * N * 2 > ACC_BUDGET or K > max(64, min(KMAX_LAUNCH, RES_BUDGET // (4 * n * nb * (M + N)) // 64 * 64))
+
+
 def residue_gemm(R, A_desc, B_desc, nb, M, N, K, acc_rows_budget=None):
     """Generator of (j0, jw, acc) panels: acc (n, nb*M, jw) int16 holding the CRT coefficients
     (centred residue * (M/m)^-1 mod m, for crt(..., scaled=True)) of the exact products over the

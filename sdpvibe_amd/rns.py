@@ -24,7 +24,7 @@ import os
 import numpy as np
 import torch
 
-from ._lib import call, ptr, ptr_strided, stream
+from ._lib import Tables, call, ptr, ptr_strided, stream
 
 dev = "cuda"
 PMAX = 16257       # largest modulus with centred residues |r| <= 8128: h + l stays in int8
@@ -194,6 +194,9 @@ class RNS:
         Ct[:, n] = Md                                      # the CRT subtracts k*M with the digit products
         self.Ct = t(Ct, torch.int8).contiguous()
         self.Md = t(Md, torch.int32)
+        of = lambda x: x.data_ptr()
+        self.tables = Tables(of(self.m32), of(self.inv32), of(self.kcoef_crt), of(self.C1), of(self.minv), of(self.Thi),
+                             of(self.Tlo), of(self.Ct), n, self.E, self.npad, self.NBp)
 
     # ---- step 1: residues of rows x kc entries (limbs) -> (G, rows, kp) hi, lo
     def kp(self, kc):
