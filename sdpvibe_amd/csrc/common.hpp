@@ -35,8 +35,10 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // addition (the compiler forms the product with a zero addend and adds it in 64 bits twice). The four
 // multiplies go first, so that three instructions lie between a carry's write and its read (a VALU read of
 // an SGPR that a VALU wrote needs two wait states). CHAIN4: four terms a[u] b[u] of one sum; COLS4: one
-// factor x times y[u] into four sums; MAC96: one term alone. SETTLE(v, w): the wait states that a lane move of v or w needs after
-// such a block (the compiler does not see the block's instructions).
+// factor x times y[u] into four sums; MAC96: one term alone. The sums are early clobbers: the first multiply
+// writes a sum while later ones still read their factors, and a factor equal to a sum's start value (zero, or
+// half of it) would otherwise get its register. SETTLE(v, w): the wait states that a lane move of v or w needs
+// after such a block (the compiler does not see the block's instructions).
 #ifndef SDPV_MAC96_CHAIN4
 #define SDPV_MAC96_CHAIN4(acc, ov, a, b)                                                          \
     do {                                                                                          \
@@ -45,7 +47,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
             "v_mad_u64_u32 %0, %4, %8, %12, %0\n\tv_mad_u64_u32 %0, %5, %9, %13, %0\n\t"          \
             "v_addc_co_u32 %1, %2, 0, %1, %2\n\tv_addc_co_u32 %1, %3, 0, %1, %3\n\t"              \
             "v_addc_co_u32 %1, %4, 0, %1, %4\n\tv_addc_co_u32 %1, %5, 0, %1, %5"                  \
-            : "+v"(acc), "+v"(ov), "=&s"(m0_), "=&s"(m1_), "=&s"(m2_), "=&s"(m3_)                 \
+            : "+&v"(acc), "+&v"(ov), "=&s"(m0_), "=&s"(m1_), "=&s"(m2_), "=&s"(m3_)               \
             : "v"((a)[0]), "v"((a)[1]), "v"((a)[2]), "v"((a)[3]), "v"((b)[0]), "v"((b)[1]),       \
               "v"((b)[2]), "v"((b)[3]));                                                          \
     } while (0)
@@ -56,16 +58,16 @@ typedef int v16i __attribute__((ext_vector_type(16)));
             "v_mad_u64_u32 %2, %10, %12, %15, %2\n\tv_mad_u64_u32 %3, %11, %12, %16, %3\n\t"      \
             "v_addc_co_u32 %4, %8, 0, %4, %8\n\tv_addc_co_u32 %5, %9, 0, %5, %9\n\t"              \
             "v_addc_co_u32 %6, %10, 0, %6, %10\n\tv_addc_co_u32 %7, %11, 0, %7, %11"              \
-            : "+v"((acc)[0]), "+v"((acc)[1]), "+v"((acc)[2]), "+v"((acc)[3]), "+v"((ov)[0]),      \
-              "+v"((ov)[1]), "+v"((ov)[2]), "+v"((ov)[3]), "=&s"(m0_), "=&s"(m1_), "=&s"(m2_),    \
-              "=&s"(m3_)                                                                          \
+            : "+&v"((acc)[0]), "+&v"((acc)[1]), "+&v"((acc)[2]), "+&v"((acc)[3]), "+&v"((ov)[0]), \
+              "+&v"((ov)[1]), "+&v"((ov)[2]), "+&v"((ov)[3]), "=&s"(m0_), "=&s"(m1_),             \
+              "=&s"(m2_), "=&s"(m3_)                                                              \
             : "v"(x), "v"((y)[0]), "v"((y)[1]), "v"((y)[2]), "v"((y)[3]));                        \
     } while (0)
 #define SDPV_MAC96(acc, ov, a, b)                                                                 \
     do {                                                                                          \
         u64 m0_;                                                                                  \
         asm("v_mad_u64_u32 %0, %2, %3, %4, %0\n\ts_nop 1\n\tv_addc_co_u32 %1, %2, 0, %1, %2"       \
-            : "+v"(acc), "+v"(ov), "=&s"(m0_)                                                     \
+            : "+&v"(acc), "+&v"(ov), "=&s"(m0_)                                                   \
             : "v"(a), "v"(b));                                                                    \
     } while (0)
 #define SDPV_SETTLE(v, w) asm("s_nop 1" : "+v"(v), "+v"(w))
