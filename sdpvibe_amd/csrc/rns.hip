@@ -1120,10 +1120,18 @@ int crt_run(const int16_t* acc, i64 n, i64 ld_g, i64 rows, i64 N, i64 j0, i64 w,
     if (lds > 160 * 1024) return SDPV_ESIZE;
     const i64 grid = (Bq + 63) / 64;
     if (grid > 0x7fffffffLL) return SDPV_ESIZE;
-    // four waves per 64 entries up to 1024 workgroups (four per CU; more of them fill the device as single waves,
-    // which need a third of the LDS)
+    // Four waves per 64 entries up to 512 workgroups, two per CU, which the LDS always holds at once. Beyond, single
+    // waves (eight per CU by their registers, fewer by their LDS) are one round of one wave, the four-wave form
+    // contends or takes a second round (its registers hold three per CU); it is the better one again where the single
+    // waves need a second round themselves, and for words, which single waves store one by one, as long
+    // as three fit a CU. us at 512 / 768 / 1024 workgroups, four waves (single): L = 8 9.7 / 11.2 / 13.3
+    // (9.8 / 10.1 / 10.3), L = 24 15.7 / 17.6 / 26.6 (16.9 / 17.7 / 18.3), with the addend 15.5 / 25.8 / 28.0
+    // (18.0 / 18.8 / 19.3), to words 14.6 / 17.3 / 24.8 (19.3 / 19.8 / 20.5), L = 36 21.4 / 36.0 / 38.9 (25.9 / 27.0 / 53.2)
     const size_t lds4 = ybytes + (size_t)4096 * ndb + 2048 + (R.X ? 256 * (size_t)L : 0);
-    if (scaled && grid <= 1024 && lds4 <= 80 * 1024 && wbytes <= ybytes) {
+    const size_t fit = 160 * 1024 / lds;
+    const bool four = grid <= (omode == SDPV_CRT_WORDS && 3 * lds4 <= 160 * 1024 ? 768 : 512) ||
+                      (grid <= 1024 && grid > 256 * (i64)(fit < 8 ? fit : 8));
+    if (scaled && four && lds4 <= 80 * 1024 && wbytes <= ybytes) {
         static bool attr4 = false;
         if (!attr4) {
             (void)hipFuncSetAttribute((const void*)k_rns_crt4, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
