@@ -1200,11 +1200,13 @@ int sdpv_rns_split(const int32_t* X, const int64_t* e, const int64_t* Erow, int6
     if (stage == 1) lds += stage_bytes;
     if (lds > 160 * 1024) return SDPV_ESIZE;
     const int ks = NBp / 32 <= 4 ? (int)(NBp / 32) : 0;
-    // at most 512 workgroups (two per CU): the small form, up to 1024 with the prime blocks shared out; a caller
-    // that wants overflows flagged takes the staged form
-    const i64 npb = (G + 31) / 32;
+    // at most 512 workgroups (two per CU): the small form, the prime blocks shared out over as many workgroups as the
+    // device holds at once: four per CU by their registers, three with four table chunks (200 workgroups of
+    // shifted rows at L = 25: 16.2 us as 1000, 14.2 as 600, the staged form 14.7; 450 of them at L = 32: 28.7 as
+    // 900, 23.6 as 450, staged 26.2). A caller that wants overflows flagged takes the staged form
+    const i64 npb = (G + 31) / 32, most = ks == 4 ? 768 : 1024;
     const bool small = grid <= 512 && ks && L <= 8 * ks && L >= 8 * (ks - 1) && !flag;
-    const unsigned gy = (unsigned)(!small ? 1 : (1024 / grid < npb ? 1024 / grid : npb));
+    const unsigned gy = (unsigned)(!small ? 1 : (most / grid < npb ? most / grid : npb));
     static bool attr_set[10] = {};
 #define SDPV_SPLIT_LAUNCH(KSC, SM)                                                                             \
     do {                                                                                                       \
