@@ -133,7 +133,7 @@ def bgemm_nt(A, Bt, out_exp="col", kc=4096, bt_rowexp=None, bt_cache=None, plus=
     L = A.L
     R = ctx(L)
     eB = Bt.exp if bt_rowexp is None else bt_rowexp
-    if _narrow(M, N, K, L):
+    if _narrow(M, N, K, L, nb):
         C = _narrow_product(A, Bt, eB, out_exp if isinstance(out_exp, int) else "col")
         if plus is not None:
             C = badd(plus, C, sgn, out_exp=out_exp)
@@ -200,17 +200,44 @@ def bgemm_nt(A, Bt, out_exp="col", kc=4096, bt_rowexp=None, bt_cache=None, plus=
     return C
 
 
-# products with at most NARROW right-hand-side columns and at most NARROW_MK rows times inner length are
-# formed directly (sdpv_narrow): the matrix is read once and multiplied as bytes, where the residue path
-# reduces each of its entries modulo every prime. One MI355X, L = 24, one column: 60 blocks of 162 x 3000
-# in 1.55 ms against 5.83 ms; 32 x 32 in 0.022 ms against 0.135 ms
+# Products with at most NARROW right-hand-side columns may be formed directly (sdpv_narrow): the matrix is read
+# once and multiplied as bytes, where the residue path reduces each of its entries modulo every prime, whatever
+# the columns. NARROW_MK bounds rows times inner length of a block, so that its workgroups stay inside a launch's
+# grid; NARROW_K the inner dimension of one direct product.
 NARROW = 2
 NARROW_MK = 1 << 40
-NARROW_K = 1 << 17                             # inner dimension of one direct product
+NARROW_K = 1 << 17
 
 
-def _narrow(M, N, K, L):
-    return N <= NARROW and M * K <= NARROW_MK and K <= NARROW_K and L <= 63
+def _narrow(M, N, K, L, nb=1, rounded=False):
+    """whether nb products of (M, K) with (K, N) are formed directly. rounded: the operands carry exponents and are
+    rounded on the way in (mpf.gemm); else their limbs are multiplied as they are.
+
+    The direct kernel starts a workgroup per 32 rows, column and 128 k, and from 41 limbs on no longer holds its
+    operands in registers; the residue path's time is that of splitting M + N rows (and of one product tile per
+    32 rows). Residues over direct, time on one MI355X, full rows, one / two columns (60 x 162 x 1500, 20 x 160 x 1000):
+    rounded L = 24 3.5 / 2.1, L = 40 2.1 / 1.3, L = 48 0.98 / 0.57, L = 63 0.73 / 0.41; as they are L = 40 2.8 / 2.0, L = 48 1.4 / 0.89,
+    L = 63 0.96 / 0.55; a 200 x 200 block, where launches count: rounded L = 40 2.0 / 1.9, L = 48 1.3 / 1.1, L = 63
+    1.0 / 1.0; as they are 1.6 to 4 at every limb count. Few rows in large batches, rounded, two columns (500 x 2 x
+    1000): L = 8 0.92, L = 24 0.63, L = 40 0.39; (3000 x 2 x 42): L = 8 1.7, L = 24 1.3, L = 40 0.85."""
+    if N > NARROW or M * K > NARROW_MK or K > NARROW_K or L > 63:
+        return False
+    ks, tiles = -(-L // 8), -(-M // 32)
+    work = nb * N * tiles * K // 128                         # slices of 32 rows and 128 k
+    cols = nb * N * tiles
+    if cols <= 16 and (ks <= 6 or not rounded):              # too few product tiles to fill the device
+        return True
+    if not rounded:
+        if ks <= 5 or (ks == 6 and N == 1) or (M <= 2 and M * N * K <= 200):
+            return True
+        return work <= 256 if ks == 6 else N * work <= 200
+    if cols * -(-K // 128) <= 256 if ks <= 5 else N * work <= 128 if ks == 6 else N == 1 and 24 <= work <= 64:
+        return True                                          # both wait for launches: fewer of them
+    # per block, in times of a k of a split row: splits and a tile of the product against k of a slice
+    per_k = (4.5, 6.8, 6.8, 10, 11, 36, 54, 47)[ks - 1]
+    if ks <= 5:
+        return (M + N + 3 * tiles) * K + 900 * tiles >= N * tiles * (K + 20) * per_k
+    return (M + N + 3 * tiles) * K + 470 * tiles >= N * tiles * K * per_k
 
 
 def flat_view(X):
@@ -438,7 +465,7 @@ def _minus_product(X, A, P):
     """badd(X, A P, -1, 'align'): rows X of a right-hand side less a block of the factor times the part
     already solved; one direct product with few columns"""
     nb, M, K = A.shape
-    if _narrow(M, P.shape[2], K, A.L):
+    if _narrow(M, P.shape[2], K, A.L, nb):
         return _narrow_product(A, _as_rows(P), P.expt(), "col", plus=X, sgn=-1)
     return badd(X, bgemm_nt(A, _as_rows(P), out_exp="col", bt_rowexp=P.expt()), -1, out_exp="align")
 

@@ -9,7 +9,8 @@
 // R = sum_{u < 4L-1} 256^u), the vector with exact signed digits (4L + 1 of them, bytes of b + 128 ... less
 // 128). sum_k a b = sum_k a' b + 128 R sum_k b, and the second term depends on the vector alone.
 //
-// A workgroup takes 32 rows, one column and a slice of at most 128 k. It turns the vector's slice into
+// One or two rows with many columns: k_narrow_few. Otherwise a
+// workgroup takes 32 rows, one column and a slice of at most 128 k. It turns the vector's slice into
 // reversed digit strings in LDS once; then, for 16 k (8 when the limb count is large) at a time, each
 // thread rounds one or two entries of the matrix to their row's exponent (or copies their limbs) into LDS as
 // bytes while the next ones load, and each wave multiplies a quarter of the k on v_mfma_i32_32x32x32_i8:
@@ -596,41 +597,151 @@ __global__ void __launch_bounds__(Geo<KS>::NT, KS <= 3 ? 2 : 1) k_narrow(Operand
     }
 }
 
-// the slices' words added and carried, a wave per entry; COL leaves words and bit lengths for k_narrow_round
-template <int KS>
-__global__ void __launch_bounds__(256) k_narrow_finish(const i64* __restrict__ part, Operand A, Operand B, Dims D, Result R,
-                                                      u32* __restrict__ words, i32* __restrict__ bls) {
-    using g = Geo<KS>;
+// One or two rows: a workgroup of k_narrow has 32 of them and prepares its vector for all, so that most of its
+// work would be done for nothing. Here a wave takes a column (or a slice of its k) and one row after the
+// other: lane c sums column c (and c + 64) of the unsigned word products over k, 64 k at a time in LDS (odd
+// stride: lanes at different words use different banks), with the corrections that make the top words
+// signed (a = a_unsigned - s_a 2^(32 L)), then carries and rounds, or leaves the slice's word sums. Operands as
+// they are (no exponents). Bound: LDS reads. 3000 columns of one row, K = 42, rounded to their column: 54 us
+// at L = 24 (148 in k_narrow), 506 at L = 63 (2452).
+constexpr int FEW_M = 2, FEW_KC = 64, FEW_KS = FEW_KC + 1;
+template <int H>
+__global__ void __launch_bounds__(256) k_narrow_few(Operand A, Operand B, Dims D, Result R, i64* __restrict__ part) {
+    SDPV_DYNAMIC_LDS(unsigned char, lds);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), L = D.L;
+    const i64 cols = D.nb * D.N, task = blockIdx.x * (i64)4 + wave;
+    if (task >= cols * D.ns) return;                      // uniform per wave; no workgroup barrier below
+    const i64 col = task % cols, sl = task / cols, b = col / D.N, j = col % D.N;
+    const i64 k1 = (sl + 1) * D.ksl < D.K ? (sl + 1) * D.ksl : D.K;
+    u32* As = (u32*)lds + wave * 2 * L * FEW_KS;
+    u32* Bs = As + L * FEW_KS;
+    Value<H> val[FEW_M];
+    int mx = 0;
+#pragma unroll
+    for (int i = 0; i < FEW_M; i++) {
+        if (i >= (int)D.M) break;                         // uniform
+        const i32* ap = A.p + b * A.ldb + i * A.ldr;
+        const i32* bp = B.p + b * B.ldb + j * B.ldr;
+        i64 lo[H], hi[H];                                 // below 2^(12 + 6 + 32): within carry_words
+#pragma unroll
+        for (int h = 0; h < H; h++) lo[h] = hi[h] = 0;
+        for (i64 k0 = sl * D.ksl; k0 < k1; k0 += FEW_KC) {
+            const int kc = (int)(k1 - k0 < FEW_KC ? k1 - k0 : FEW_KC), kr = (kc + 3) & ~3;   // words past kc are zero
+            wave_sync();                                  // the previous chunk has been read
+            for (int u = 0; u < L; u++) {
+                As[u * FEW_KS + lane] = lane < kc ? (u32)ap[u * A.plane + (k0 + lane) * A.ldk] : 0u;
+                Bs[u * FEW_KS + lane] = lane < kc ? (u32)bp[u * B.plane + (k0 + lane) * B.ldk] : 0u;
+            }
+            wave_sync();
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                const int c = lane + 64 * h;
+                if (c > 2 * L) continue;
+                const int u0 = c - (L - 1) > 0 ? c - (L - 1) : 0, u1 = c < L - 1 ? c : L - 1;
+                for (int u = u0; u <= u1; u++) {
+                    const u32 *x = As + u * FEW_KS, *y = Bs + (c - u) * FEW_KS;
+                    for (int k = 0; k < kr; k += 4) {
+#pragma unroll
+                        for (int t = 0; t < 4; t++) {
+                            const u64 q = (u64)x[k + t] * y[k + t];
+                            lo[h] += (i64)(u32)q;
+                            hi[h] += (i64)(q >> 32);
+                        }
+                    }
+                }
+                if (c >= L) {
+                    const u32 *at = As + (L - 1) * FEW_KS, *bt = Bs + (L - 1) * FEW_KS;
+                    const int q = c < 2 * L ? c - L : 0;
+                    for (int k = 0; k < kc; k++) {
+                        const u32 sa = at[k] >> 31, sb = bt[k] >> 31;
+                        if (c < 2 * L) lo[h] -= (i64)(sa ? Bs[q * FEW_KS + k] : 0u) + (i64)(sb ? As[q * FEW_KS + k] : 0u);
+                        else lo[h] += (i64)(sa & sb);
+                    }
+                }
+            }
+        }
+        if (D.ns > 1) {                                   // word c gets the upper half of column c - 1
+            i64* p = part + (sl * cols * D.M + (b * D.M + i) * D.N + j) * (2 * L + 2);
+            u64 top = 0;
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                u64 hb = ((u64)lane_below((u32)((u64)hi[h] >> 32)) << 32) | lane_below((u32)hi[h]);
+                if (h > 0 && lane == 0) hb = top;
+                if (H > 1) top = lane_read64((u64)hi[h], 63);
+                if (lane + 64 * h < 2 * L + 2) p[lane + 64 * h] = lo[h] + (i64)hb;
+            }
+            continue;
+        }
+        val[i].NW = min(R.NW, 64 * H);
+        carry_words<H>((const u64*)lo, hi, val[i].NW, val[i].w);
+        if (R.mode != OUT_COL) {
+            emit<H>(R, D, A, B, b, i, j, val[i]);
+            continue;
+        }
+        val[i].sign();
+        mx = max(mx, val[i].bitlen());
+    }
+    if (D.ns > 1 || R.mode != OUT_COL) return;
+    const i64 s = (i64)mx - (32 * L - 32), ec = product_exp(R, D.N, b, j) + s;
+    if (lane == 0) R.oute[b * D.N + j] = R.X ? max((long long)R.eX[b * D.N + j], (long long)ec) + 1 : ec;
+#pragma unroll
+    for (int i = 0; i < FEW_M; i++) {
+        if (i >= (int)D.M) break;
+        bool bad;
+        const u32 cw = val[i].rounded(s, L, bad);
+        if (bad && R.flag && lane == 0) atomicOr(R.flag, 1);
+        emit_col(R, D, b, i, j, cw, ec);
+    }
+}
+
+// the slices' words (nwp each) added and carried, a wave per entry; COL leaves words and bit lengths for
+// k_narrow_round
+template <int H>
+__global__ void __launch_bounds__(256) k_narrow_finish(const i64* __restrict__ part, int nwp, Operand A, Operand B, Dims D,
+                                                      Result R, u32* __restrict__ words, i32* __restrict__ bls) {
     const int lane = threadIdx.x & 63;
     const i64 E = D.nb * D.M * D.N, e = blockIdx.x * (i64)4 + (threadIdx.x >> 6);
     if (e >= E) return;                                   // uniform per wave; no workgroup barrier below
-    u64 lo[g::H];
-    i64 hi[g::H];
+    u64 lo[H];
+    i64 hi[H];
 #pragma unroll
-    for (int h = 0; h < g::H; h++) lo[h] = 0, hi[h] = 0;
-    for (int s = 0; s < D.ns; s++) {
+    for (int h = 0; h < H; h++) {
+        lo[h] = 0;
+        hi[h] = 0;
+        const int w = lane + 64 * h;
+        if (w < nwp) {
+            const i64* p = part + e * nwp + w;
+            const i64 step = E * nwp;
+            int s = 0;
+            for (; s + 8 <= D.ns; s += 8) {               // eight loads in flight
+                i64 v[8];
 #pragma unroll
-        for (int h = 0; h < g::H; h++) {
-            const int w = lane + 64 * h;
-            if (w < g::NWP) {
-                const i64 v = part[((i64)s * E + e) * g::NWP + w];
+                for (int u = 0; u < 8; u++) v[u] = p[(s + u) * step];
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    lo[h] += (u32)v[u];
+                    hi[h] += v[u] >> 32;
+                }
+            }
+            for (; s < D.ns; s++) {
+                const i64 v = p[s * step];
                 lo[h] += (u32)v;
                 hi[h] += v >> 32;
             }
         }
     }
-    Value<g::H> val;
-    val.NW = min(R.NW, 64 * g::H);
-    carry_words<g::H>(lo, hi, val.NW, val.w);
+    Value<H> val;
+    val.NW = min(R.NW, 64 * H);
+    carry_words<H>(lo, hi, val.NW, val.w);
     const i64 j = e % D.N, i = e / D.N % D.M, b = e / (D.N * D.M);
     if (R.mode != OUT_COL) {
-        emit<g::H>(R, D, A, B, b, i, j, val);
+        emit<H>(R, D, A, B, b, i, j, val);
         return;
     }
     val.sign();
     const int bl = val.bitlen();
 #pragma unroll
-    for (int h = 0; h < g::H; h++) words[(e * g::H + h) * 64 + lane] = val.w[h];
+    for (int h = 0; h < H; h++) words[(e * H + h) * 64 + lane] = val.w[h];
     if (lane == 0) bls[e] = bl;
 }
 
@@ -696,8 +807,35 @@ inline void slices(i64 nb, i64 M, i64 N, i64 K, Dims& D) {
     D.ns = (int)(K > 0 ? (K + len - 1) / len : 1);
 }
 
+// slices of k_narrow_few: multiples of 64 k, at most 4096, shorter ones while the launch has fewer than FEW_WAVES waves
+constexpr i64 FEW_K = 4096, FEW_WAVES = 2048;
+inline void few_slices(i64 nb, i64 N, i64 K, Dims& D) {
+    const i64 cols = nb * N, nmax = (K + FEW_KC - 1) / FEW_KC;
+    i64 ns = (K + FEW_K - 1) / FEW_K;
+    const i64 want = (FEW_WAVES + cols - 1) / (cols > 0 ? cols : 1);
+    if (want > ns) ns = want < nmax ? want : nmax;
+    if (ns < 1) ns = 1;
+    const i64 len = ((K + ns - 1) / ns + FEW_KC - 1) / FEW_KC * FEW_KC;
+    D.ksl = (int)(len > 0 ? len : FEW_KC);
+    D.ns = (int)(K > 0 ? (K + D.ksl - 1) / D.ksl : 1);
+}
 inline int chunks(i64 L) { return (int)((L + 7) / 8); }
 inline int lane_words(i64 L) { return 16 * chunks(L) + 2 > 64 ? 2 : 1; }
+
+// Whether one or two rows take k_narrow_few: its time grows with the rows and k, k_narrow's with the columns and the
+// slices of 128 k that they start, the faster the more limbs. us for one row at 1024 columns of 42 k / 512 of 200 /
+// 128 of 3000, few (k_narrow): L = 8 24 / 34 / 84 (22 / 27 / 74), L = 24 39 / 62 / 189 (52 / 82 / 257), L = 35
+// 67 / 106 / 310 (133 / 220 / 727), L = 48 107 / 323 / 941 (322 / 642 / 2126); two rows and two columns a block, 512
+// blocks of 42 k / 256 of 200 / 256 of 1000: L = 24 76 / 113 / 471 (53 / 84 / 334), L = 35 127 / 200 / 772
+// (134 / 225 / 970), L = 48 206 / 605 / 2398 (325 / 649 / 2809)
+inline bool takes_few(i64 L, i64 nb, i64 M, i64 N, i64 K) {
+    if (M > FEW_M) return false;
+    const int ks = chunks(L);
+    const i64 w = nb * N * ((K + SLICE - 1) / SLICE);
+    if (L == 40) return M == 1 && w >= 1024;              // its operands' LDS fits a CU once, to L = 39 twice
+    if (ks <= 4) return (M == 1 || K <= SLICE / 2) && w >= (ks == 1 ? 2560 : 1024) * M;
+    return w >= (ks == 5 ? 512 * M : ks == 6 ? 256 * M * M : 256 * M);
+}
 
 // 64-bit words of scratch: the slices' words; the words and bit lengths that k_narrow_round reads
 inline i64 work_words(i64 L, i64 nb, i64 M, i64 N, i64 K) {
@@ -706,7 +844,31 @@ inline i64 work_words(i64 L, i64 nb, i64 M, i64 N, i64 K) {
     const i64 E = nb * M * N;
     i64 n = D.ns > 1 ? (i64)D.ns * E * 16 * chunks(L) : 0;
     if (D.ns > 1 || M > ROWS) n += E * 32 * lane_words(L) + (E + 1) / 2;
+    if (takes_few(L, nb, M, N, K)) {
+        few_slices(nb, N, K, D);
+        const i64 f = D.ns > 1 ? (i64)D.ns * E * (2 * L + 2) + E * 32 * lane_words(L) + (E + 1) / 2 : 0;
+        n = f > n ? f : n;
+    }
     return n;
+}
+
+// after the products: the slices' sums, and COL's rounding over all rows
+template <int H>
+int launch_rest(const Operand& A, const Operand& B, const Dims& D, const Result& R, const i64* part, int nwp, u32* words,
+                i32* bls, hipStream_t st) {
+    const i64 E = D.nb * D.M * D.N;
+    if (D.ns > 1) {
+        hipLaunchKernelGGL(k_narrow_finish<H>, dim3((unsigned)((E + 3) / 4)), dim3(256), 0, st, part, nwp, A, B, D, R, words,
+                           bls);
+        SDPV_TRY_LAUNCH();
+    }
+    if (R.mode == OUT_COL && (D.ns > 1 || D.M > ROWS)) {
+        const i64 rpw = D.M <= 4096 ? 4 : (D.M / 1024 + 3) / 4 * 4;
+        hipLaunchKernelGGL(k_narrow_round<H>, dim3((unsigned)(D.nb * D.N * ((D.M + rpw - 1) / rpw))), dim3(256), 0, st,
+                           words, bls, D, R, rpw);
+        SDPV_TRY_LAUNCH();
+    }
+    return SDPV_OK;
 }
 
 template <int KS>
@@ -729,17 +891,23 @@ int launch_narrow(const Operand& A, const Operand& B, const Dims& D, const Resul
     else
         hipLaunchKernelGGL((k_narrow<KS, false>), dim3((unsigned)grid), dim3(g::NT), (size_t)g::LDS, st, A, B, D, R, part, words, bls);
     SDPV_TRY_LAUNCH();
-    if (D.ns > 1) {
-        hipLaunchKernelGGL(k_narrow_finish<KS>, dim3((unsigned)((E + 3) / 4)), dim3(256), 0, st, part, A, B, D, R, words, bls);
-        SDPV_TRY_LAUNCH();
+    return launch_rest<g::H>(A, B, D, R, part, g::NWP, words, bls, st);
+}
+
+template <int H>
+int launch_few(const Operand& A, const Operand& B, const Dims& D, const Result& R, i64* work, hipStream_t st) {
+    const i64 E = D.nb * D.M * D.N, grid = (D.nb * D.N * D.ns + 3) / 4;
+    if (grid > 0x7fffffffLL) return SDPV_ESIZE;
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute((const void*)k_narrow_few<H>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        attr = true;
     }
-    if (R.mode == OUT_COL && (D.ns > 1 || D.M > ROWS)) {
-        const i64 rpw = D.M <= 4096 ? 4 : (D.M / 1024 + 3) / 4 * 4;
-        hipLaunchKernelGGL(k_narrow_round<g::H>, dim3((unsigned)(D.nb * D.N * ((D.M + rpw - 1) / rpw))), dim3(256), 0, st,
-                           words, bls, D, R, rpw);
-        SDPV_TRY_LAUNCH();
-    }
-    return SDPV_OK;
+    u32* words = (u32*)(work + (D.ns > 1 ? (i64)D.ns * E * (2 * D.L + 2) : 0));
+    hipLaunchKernelGGL(k_narrow_few<H>, dim3((unsigned)grid), dim3(256), (size_t)32 * D.L * FEW_KS, st, A, B, D, R, work);
+    SDPV_TRY_LAUNCH();
+    if (D.ns == 1) return SDPV_OK;
+    return launch_rest<H>(A, B, D, R, work, 2 * D.L + 2, words, (i32*)(words + E * 64 * H), st);
 }
 
 int narrow_run(const Operand& A, const Operand& B, i64 L, i64 nb, i64 M, i64 N, i64 K, const Result& R, i64* work,
@@ -749,6 +917,10 @@ int narrow_run(const Operand& A, const Operand& B, i64 L, i64 nb, i64 M, i64 N, 
     const i64 need = work_words(L, nb, M, N, K);
     if (need > 0 && (!work || nwork < need)) return SDPV_EARG;
     if ((nb * M * N + 3) / 4 > 0x7fffffffLL) return SDPV_ESIZE;
+    if (!A.e && !B.e && takes_few(L, nb, M, N, K)) {
+        few_slices(nb, N, K, D);
+        return lane_words(L) == 2 ? launch_few<2>(A, B, D, R, work, st) : launch_few<1>(A, B, D, R, work, st);
+    }
     switch (chunks(L)) {
         case 1: return launch_narrow<1>(A, B, D, R, work, st);
         case 2: return launch_narrow<2>(A, B, D, R, work, st);

@@ -370,7 +370,7 @@ def gemm(A, B, transA=False, transB=False):
     N, K2, bldb, bldr, bldk = _geometry(Be.shape, not transB)   # rows of op(B)^T = columns of op(B)
     assert K == K2, (A.shape, B.shape, transA, transB)
     R = ctx(L)
-    narrow = _batched._narrow(max(M, N), min(M, N), K, L)
+    narrow = _batched._narrow(max(M, N), min(M, N), K, L, nb, True)
     if not narrow and nb * M * N * K != 0 and K <= R.kmax:
         kp = R.kp_product(K)
         up = lambda x: (x + 255) & ~255
@@ -447,8 +447,9 @@ class KSum:
         self.M, self.N = EA.numel(), EB.numel()
         self.R = ctx(L)
         self.K = 0
-        # few columns: the exact words of every entry's sum (direct products), else its residues
-        self.direct = _batched._narrow(self.M, self.N, 0, L)
+        # few columns: the exact words of every entry's sum (direct products), else its residues; the segments' lengths
+        # are not known yet, the rule is that of a long one
+        self.direct = _batched._narrow(self.M, self.N, 4096, L, rounded=True)
         if self.direct:
             self.acc = torch.zeros((self.M * self.N, 2 * L + 2), dtype=torch.int32, device=dev)
         else:

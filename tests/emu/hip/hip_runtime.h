@@ -150,7 +150,7 @@ emu_v16i emu_mfma_i32_32x32x32_i8(emu_v4i a, emu_v4i b, emu_v16i c, int, int, in
     std::memcpy((unsigned char*)(ldsbase) + 16 * (threadIdx.x & 63), (const void*)(gptr), 16)
 #define SDPV_WAIT_VMCNT(n) ((void)(n))
 #define __builtin_amdgcn_s_setprio(p) ((void)(p))
-#define __builtin_amdgcn_readfirstlane(x) (x)
+#define __builtin_amdgcn_readfirstlane(x) ((int)emu_shfl_idx64((long long)(x), 0))   // every lane of the wave takes part
 
 // Dynamic shared memory of the block being run (blocks run one at a time).
 extern unsigned char* emu_dynamic_lds;

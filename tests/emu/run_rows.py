@@ -1,0 +1,31 @@
+"""Emulated products of one or two rows in large batches against the oracle. Usage: run_rows.py few L nb M N K"""
+import os
+import random
+import sys
+
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
+from tests.emu import harness  # noqa: E402
+
+harness.install()
+import numpy as np  # noqa: E402
+import torch  # noqa: E402
+
+from oracle import oracle as O  # noqa: E402
+from sdpvibe_amd import batched as Bm  # noqa: E402
+
+
+def few(L, nb, M, N, K):
+    from tests.test_gpu_few_rows import limbs
+    rng = random.Random(L + nb)
+    A, B = limbs(rng, L, nb, M, K), limbs(rng, L, nb, N, K)
+    eA = -(32 * L - 8)
+    eB = np.array([[rng.randrange(-40, 40) - 32 * L for _ in range(N)] for _ in range(nb)], np.int64)
+    for mode, om in (("col", 1), (17, 0)):
+        C = Bm.bgemm_nt(Bm.BMP(A, eA), Bm.BMP(B, 0), out_exp=mode, bt_rowexp=torch.from_numpy(eB))
+        ref, rexp = O.bgemm_nt(A.numpy(), B.numpy(), eA + eB, om, np.full((nb, N), 17, np.int64) if om == 0 else None)
+        assert np.array_equal(C.limbs.numpy(), ref) and (om == 0 or np.array_equal(C.exp.numpy(), rexp)), mode
+
+
+if __name__ == "__main__":
+    {"few": few}[sys.argv[1]](*(int(a) for a in sys.argv[2:]))
+    print("ok")
