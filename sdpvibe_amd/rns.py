@@ -306,15 +306,17 @@ class RNS:
         """columns j0..j0+w of out (L, nb, M, N), a view with unit column stride, from a scaled accumulator
         (n, nb * M, w): round(value / 2^s) for each column's shift s (scol (nb * N,), or the int s0), or
         plus + sgn * that modulo 2^(32 L) (plus: limbs laid out like out; it may be out itself)"""
-        L, N = out.shape[0], out.shape[3]
-        if acc.numel() < self.n * nb * M * w or not acc.is_contiguous() or j0 + w > N:
+        L, b, m, N = out.shape
+        op, ob, ld, oc = out.stride()
+        if acc.numel() < self.n * nb * M * w or j0 + w > N:
             raise ValueError("crt: block exceeds the residue accumulator")
-        if (tuple(out.shape[1:3]) != (nb, M) or out.stride(3) != 1 or (scol is not None and scol.numel() < nb * N)
-                or (plus is not None and (plus.shape != out.shape or plus.stride(3) != 1))):
+        x, xp, xb, xld, xc = None, 0, 0, 0, 1
+        if plus is not None:
+            xp, xb, xld, xc = plus.stride()
+            x = ptr_strided(plus[:, :, :, j0:] if j0 else plus)
+        if (b != nb or m != M or oc != 1 or xc != 1 or (scol is not None and scol.numel() < nb * N)
+                or (plus is not None and plus.shape != out.shape)):
             raise ValueError("crt: limb arrays of another shape or column stride")
-        op, ob, ld, _ = out.stride()
-        xp, xb, xld, _ = (0, 0, 0, 0) if plus is None else plus.stride()
-        x = None if plus is None else ptr_strided(plus[:, :, :, j0:])
         call("sdpv_rns_crt_fixed", ptr(acc), self.n, nb * M * w, nb * M, w, 0, w, ptr(self.m32), ptr(self.minv),
              ptr(self.inv32), ptr(self.Ct), self.E, self.npad, ptr_strided(out), L, op, ld, j0, ob, M, s0, ptr(scol), N,
              x, xp, xld, xb, sgn, ptr(flag), stream())
