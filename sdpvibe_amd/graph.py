@@ -6,9 +6,35 @@ C ABI and never synchronises with the host, so a whole call such as mpf.gemm can
 and replayed: the replay re-runs the same kernels on the same buffers with no host work and no
 launch gaps. Inputs are updated in place (copy_ into the captured tensors) between replays.
 """
+import contextlib
 import gc
+import threading
 
 import torch
+
+_lock = threading.Lock()
+_captures = 0                  # captures under way, on any thread
+_collecting = False            # whether collection was on before the first of them
+
+
+@contextlib.contextmanager
+def _no_collection():
+    """Cyclic garbage collection off while any thread captures: it may destroy another object's graph (a solver that
+    went out of use), whose destructor synchronises the device, which a capture forbids. The last capture to end
+    turns it on again."""
+    global _captures, _collecting
+    with _lock:
+        if _captures == 0:
+            _collecting = gc.isenabled()
+            gc.disable()
+        _captures += 1
+    try:
+        yield
+    finally:
+        with _lock:
+            _captures -= 1
+            if _captures == 0 and _collecting:
+                gc.enable()
 
 
 class Captured:
@@ -25,16 +51,8 @@ class Captured:
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        # no cyclic garbage collection while capturing: it may destroy another object's graph (a solver that
-        # went out of use), whose destructor synchronises the device, which a capture forbids
-        collecting = gc.isenabled()
-        gc.disable()
-        try:
-            with torch.cuda.graph(self.graph):
-                self.out = fn(*args)
-        finally:
-            if collecting:
-                gc.enable()
+        with _no_collection(), torch.cuda.graph(self.graph):
+            self.out = fn(*args)
 
     def replay(self):
         self.graph.replay()
