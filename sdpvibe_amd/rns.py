@@ -205,8 +205,10 @@ class RNS:
     def kp_product(self, kc):
         """padded inner dimension of an internal product: to a multiple of 32 for a short one (a tile of 32
         pays for no zero half: splitting and multiplying 32 x 32 leaves padded to 64 took twice the
-        work), of 64 otherwise, where the padding weighs little and every product tile applies"""
-        return -(-kc // 32) * 32 if kc <= 96 else self.kp(kc)
+        work), of 64 otherwise, where the padding weighs little and every product tile applies, or where the pinned
+        configuration has 64-byte stages only"""
+        half = kc <= 96 and (FORCED is None or FORCED in HALF_CONFIGS)
+        return -(-kc // 32) * 32 if half else self.kp(kc)
 
     def residues(self, X, k0, kc, g0=0, G=None):
         """X: (L, rows, K) int32 limb planes. Residues of X[:, :, k0:k0+kc] modulo primes
