@@ -704,8 +704,8 @@ __device__ __forceinline__ void tri_pair(int p, int& i, int& j) {
     j = p - r * (r + 1) / 2;
 }
 
-// (operands with words above N, which a factor of an SPD tile never has:) A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`): x, y magnitudes with top words
-// ta, tb, A a WL-word two's complement target. The column sums are formed four columns at a time:
+// A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`), taken where an operand has words above N (a factor of
+// an SPD tile never has): x, y magnitudes with top words ta, tb, A a WL-word two's complement target. The column sums are formed four columns at a time:
 // x[i] is read once per block and the four operand words y[kb + c - i] sit in a window of registers
 // that shifts by one word per i, so a block costs two LDS reads per i instead of eight; the target
 // words of a block are read before its columns are summed. The column sums, the carry chain and the
@@ -832,14 +832,16 @@ __device__ __forceinline__ void trail_update(const u32* xs, const u32* ys, int t
 // while the other waves update the pairs, one per thread. Wave 0 runs the pivot's first Newton steps
 // while the others scale, so a step is bound by wave 0's chain of products alone (18: one scale, one
 // update, 16 for the pivot). N: words that hold every |L_ik| < 1 (N >= LF).
-// 1024 threads (four waves per SIMD): 960 for the trailing products. One 32 x 32 tile at L = 24 on one
-// MI355X: 0.334 ms (0.795 ms with products out of line and trailing operands read term by term from
-// LDS); k_tile_inverse 0.088 ms (0.200 ms).
-constexpr int NT = 1024;
-template <int N>
-__global__ void __launch_bounds__(NT) k_tile_chol_lds(u32* __restrict__ Wg, u32* __restrict__ Rg, int BT, int WL,
-                                                     int LF) {
-    constexpr int NW = NT / 64;
+// 1024 threads (four waves per SIMD: 960 for the trailing products), fewer where the tile and the waves'
+// operands would not fit in LDS together. Updates of at most `lane_pairs` pairs run one
+// pair per wave instead (none: wave 0's chain hides them either way). One
+// 32 x 32 tile at L = 24 on one MI355X: 0.334 ms (0.795 ms with products out of line and trailing operands
+// read term by term from LDS); k_tile_inverse 0.088 ms (0.200 ms). DEFAULT: 1024 threads and no such pairs (known to
+// the compiler: 2% on one tile, 4% on 400).
+template <int N, bool DEFAULT>
+__global__ void __launch_bounds__(1024) k_tile_chol_lds(u32* __restrict__ Wg, u32* __restrict__ Rg, int BT, int WL,
+                                                       int LF, int lane_pairs) {
+    const int NT = DEFAULT ? 1024 : blockDim.x, NW = NT >> 6;
     SDPV_DYNAMIC_LDS(u32, lds);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const i64 tile = blockIdx.x;
@@ -931,6 +933,17 @@ __global__ void __launch_bounds__(NT) k_tile_chol_lds(u32* __restrict__ Wg, u32*
         const int m = BT - k - 1, npairs = m * (m + 1) / 2;
         if (wave == 0) {
             pivot(k + 1, dnext, rnext);
+        } else if (!DEFAULT && npairs - 1 <= lane_pairs) {
+            for (int p = wave; p < npairs; p += NW - 1) {
+                int ii, jj;
+                tri_pair(p, ii, jj);
+                const int r = k + 1 + ii, c = k + 1 + jj;
+                const LaneMag x = lane_mag(Q, lane < WL ? te(r, k)[lane] : 0u), y = lane_mag(Q, lane < WL ? te(c, k)[lane] : 0u);
+                const u32 w = lane_signed(Q, lane_mul<16>(Q, x, y, 0), x.neg != y.neg);
+                u32* a = te(r, c);
+                const u32 v = lane_add(Q, lane < WL ? a[lane] : 0u, ~w & Q.in, 1u);
+                if (lane < WL) a[lane] = v;
+            }
         } else {
             for (int p = 1 + tid - 64; p < npairs; p += NT - 64) {
                 int ii, jj;
@@ -959,11 +972,11 @@ constexpr int INV_PRE = 8;  // words of the next row each thread prefetches
 // truncated, the sum exact (modulo 2^(32 WL)). Step i: the NT / 64 waves take the products j = k..i-1
 // in turn and add them on the lanes, carries left pending; wave 0 adds the waves' sums, propagates the
 // carries once and finishes x_ik with one more product. Row i + 1 of L is loaded while step i computes.
-// Grid (nb, BT), INV_NT threads. X entries above the diagonal are written as zeros.
-constexpr int INV_NT = 512;
-__global__ void __launch_bounds__(INV_NT) k_tile_inverse(const u32* __restrict__ Wg, const u32* __restrict__ Rg,
-                                                    u32* __restrict__ Xg, int BT, int WL, int LF) {
-    constexpr int NW = INV_NT / 64;
+// Grid (nb, BT), 512 threads. X entries above the diagonal are written as zeros.
+template <bool DEFAULT>
+__global__ void __launch_bounds__(DEFAULT ? 512 : 1024) k_tile_inverse(const u32* __restrict__ Wg, const u32* __restrict__ Rg,
+                                                      u32* __restrict__ Xg, int BT, int WL, int LF) {
+    const int NT = DEFAULT ? 512 : blockDim.x, NW = NT >> 6;
     SDPV_DYNAMIC_LDS(u32, lds);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const i64 tile = blockIdx.x;
@@ -976,12 +989,12 @@ __global__ void __launch_bounds__(INV_NT) k_tile_inverse(const u32* __restrict__
     const u32* W = Wg + tile * BT * BT * WL;
     const u32* R = Rg + tile * BT * WL;
     u32* X = Xg + tile * BT * BT * WL;
-    for (int idx = tid; idx < BT * WL; idx += INV_NT) RI[idx] = R[idx];
+    for (int idx = tid; idx < BT * WL; idx += NT) RI[idx] = R[idx];
     for (int i = 0; i < k; i++)
-        for (int q = tid; q < WL; q += INV_NT) X[((i64)i * BT + k) * WL + q] = 0u;
+        for (int q = tid; q < WL; q += NT) X[((i64)i * BT + k) * WL + q] = 0u;
     // row k + 1 into buffer 0 (entries j = k..k, at slot j)
     if (k + 1 < BT)
-        for (int idx = tid; idx < WL; idx += INV_NT) LR[(i64)k * WL + idx] = W[((i64)(k + 1) * BT + k) * WL + idx];
+        for (int idx = tid; idx < WL; idx += NT) LR[(i64)k * WL + idx] = W[((i64)(k + 1) * BT + k) * WL + idx];
     __syncthreads();
     if (wave == 0 && lane < WL) {       // x_kk = r_k
         const u32 r = RI[k * WL + lane];
@@ -998,7 +1011,7 @@ __global__ void __launch_bounds__(INV_NT) k_tile_inverse(const u32* __restrict__
         const u32* src = W + ((i64)(i + 1) * BT + k) * WL;
 #pragma unroll
         for (int u = 0; u < INV_PRE; u++) {
-            const int idx = tid + u * INV_NT;
+            const int idx = tid + u * NT;
             pre[u] = idx < nw ? src[idx] : 0u;
         }
         // this wave's products, summed exactly: words of two's complement numbers in 64 bits per lane, the
@@ -1016,7 +1029,7 @@ __global__ void __launch_bounds__(INV_NT) k_tile_inverse(const u32* __restrict__
         }
 #pragma unroll
         for (int u = 0; u < INV_PRE; u++) {
-            const int idx = tid + u * INV_NT;
+            const int idx = tid + u * NT;
             if (idx < nw) nxt[k * WL + idx] = pre[u];
         }
         __syncthreads();
@@ -1172,16 +1185,21 @@ __global__ void __launch_bounds__(256) k_tile_narrow(const u32* __restrict__ W, 
 inline unsigned nblk(i64 n, int tpb) { return (unsigned)((n + tpb - 1) / tpb); }
 
 // the factorisation for magnitudes of N words
-template <int N>
-int launch_factor(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, size_t lds, hipStream_t st) {
+template <int N, bool DEFAULT>
+int launch_factor_form(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, int nt, size_t lds, hipStream_t st) {
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<N>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<N, DEFAULT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
-    hipLaunchKernelGGL(k_tile_chol_lds<N>, dim3((unsigned)nb), dim3(NT), lds, st, W, RI, BT, WL, LF);
+    hipLaunchKernelGGL((k_tile_chol_lds<N, DEFAULT>), dim3((unsigned)nb), dim3(nt), lds, st, W, RI, BT, WL, LF, 0);
     SDPV_TRY_LAUNCH();
     return SDPV_OK;
+}
+template <int N>
+int launch_factor(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, int nt, size_t lds, hipStream_t st) {
+    return nt == 1024 ? launch_factor_form<N, true>(W, RI, nb, BT, WL, LF, nt, lds, st)
+                                                : launch_factor_form<N, false>(W, RI, nb, BT, WL, LF, nt, lds, st);
 }
 
 // Xe null: the inverse as WL words; else rounded to hb bits, its exponents (nb, BT) to Xe
@@ -1213,20 +1231,27 @@ int tile_run(const i32* A, i64 plane, i64 ldb, i64 ldr, i64 L, i64 nb, i64 BT, i
     hipLaunchKernelGGL(k_tile_widen, dim3((unsigned)nrow), dim3(256), (size_t)4 * BT * (L | 1), st, A, plane, ldb, ldr,
                        (int)BT, (int)L, WL, W, top);
     SDPV_TRY_LAUNCH();
-    const size_t lds_f = (size_t)lds_factor_words((int)BT, WL, NT / 64) * 4;
-    const size_t lds_i = (size_t)lds_inverse_words((int)BT, WL, INV_NT / 64) * 4;
-    if (WL <= 64 && lds_f <= 160 * 1024 && BT * WL <= INV_PRE * INV_NT) {
+    int nt = 1024, ni = 512;
+    auto lds_f = [&] { return (size_t)lds_factor_words((int)BT, WL, nt / 64) * 4; };
+    while (nt > 256 && lds_f() > 160 * 1024) nt /= 2;   // a wave's operands take 1 KB: BT = 38 at L = 24 fits with eight
+    while (ni < 512 && BT * WL > INV_PRE * ni) ni *= 2;
+    const size_t lds_i = (size_t)lds_inverse_words((int)BT, WL, ni / 64) * 4;
+    if (WL <= 64 && lds_f() <= 160 * 1024 && BT * WL <= INV_PRE * ni) {
         // the tile stays in LDS; the inverse one workgroup per column
-        const int rc = L <= 8 ? launch_factor<8>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
-                     : L <= 16 ? launch_factor<16>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
-                     : L <= 24 ? launch_factor<24>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
-                     : L <= 28 ? launch_factor<28>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
-                     : L <= 32 ? launch_factor<32>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
-                     : L <= 36 ? launch_factor<36>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st)
-                               : launch_factor<40>(W, RI, nb, (int)BT, WL, (int)L, lds_f, st);
+        const int rc = L <= 8 ? launch_factor<8>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st)
+                     : L <= 16 ? launch_factor<16>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st)
+                     : L <= 24 ? launch_factor<24>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st)
+                     : L <= 28 ? launch_factor<28>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st)
+                     : L <= 32 ? launch_factor<32>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st)
+                     : L <= 36 ? launch_factor<36>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st)
+                               : launch_factor<40>(W, RI, nb, (int)BT, WL, (int)L, nt, lds_f(), st);
         if (rc != SDPV_OK) return rc;
-        hipLaunchKernelGGL(k_tile_inverse, dim3((unsigned)nb, (unsigned)BT), dim3(INV_NT), lds_i, st, W, RI, X,
-                           (int)BT, WL, (int)L);
+        if (ni == 512)
+            hipLaunchKernelGGL(k_tile_inverse<true>, dim3((unsigned)nb, (unsigned)BT), dim3(ni), lds_i, st, W, RI, X,
+                               (int)BT, WL, (int)L);
+        else
+            hipLaunchKernelGGL(k_tile_inverse<false>, dim3((unsigned)nb, (unsigned)BT), dim3(ni), lds_i, st, W, RI, X,
+                               (int)BT, WL, (int)L);
         SDPV_TRY_LAUNCH();
     } else {
         hipLaunchKernelGGL(k_tile_factor, dim3((unsigned)nb), dim3(TT), lds, st, W, X, S, RI, (int)BT, WL, (int)L);

@@ -8,6 +8,7 @@
 #include <sys/mman.h>
 #include <cstdio>
 #include <cstdlib>
+#include <map>
 #include <memory>
 
 thread_local dim3 threadIdx, blockIdx, blockDim, gridDim;
@@ -185,12 +186,17 @@ emu_v16i emu_mfma_i32_32x32x32_i8(emu_v4i a, emu_v4i b, emu_v16i c, int, int, in
     return d;
 }
 
+// launches so far with this many threads per block
+static std::map<unsigned, int> g_launched;
+extern "C" int emu_launched(int threads) { return g_launched[threads]; }
+
 void emu_run_grid(dim3 grid, dim3 block, size_t lds_bytes, const std::function<void()>& body) {
     if (lds_bytes > LDS_MAX) {
         fprintf(stderr, "emu: dynamic LDS %zu exceeds %zu\n", lds_bytes, LDS_MAX);
         abort();
     }
     const unsigned nt = block.x * block.y * block.z;
+    g_launched[nt]++;
     if (nt > g_nstacks) {
         if (g_stacks) munmap(g_stacks, g_nstacks * STACK);
         g_stacks = (char*)mmap(nullptr, nt * STACK, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE,
