@@ -9,6 +9,8 @@
 // and ballot carry-lookahead (lane_mul). When the tile's lower triangle fits in LDS
 // (k_tile_chol_lds) the factorisation runs there and the inverse is built column-parallel
 // (k_tile_inverse); otherwise k_tile_factor works on the tile in HBM.
+#include <cstdlib>
+
 #include "common.hpp"
 
 namespace {
@@ -833,8 +835,8 @@ __device__ __forceinline__ void trail_update(const u32* xs, const u32* ys, int t
 // while the others scale, so a step is bound by wave 0's chain of products alone (18: one scale, one
 // update, 16 for the pivot). N: words that hold every |L_ik| < 1 (N >= LF).
 // 1024 threads (four waves per SIMD: 960 for the trailing products), fewer where the tile and the waves'
-// operands would not fit in LDS together. Updates of at most `lane_pairs` pairs run one
-// pair per wave instead (none: wave 0's chain hides them either way). One
+// operands would not fit in LDS together, or by SDPV_TILE_THREADS. Updates of at most `lane_pairs` pairs run one
+// pair per wave instead (SDPV_TILE_LANE_PAIRS, 0 unless set: wave 0's chain hides them either way). One
 // 32 x 32 tile at L = 24 on one MI355X: 0.334 ms (0.795 ms with products out of line and trailing operands
 // read term by term from LDS); k_tile_inverse 0.088 ms (0.200 ms). DEFAULT: 1024 threads and no such pairs (known to
 // the compiler: 2% on one tile, 4% on 400).
@@ -972,7 +974,7 @@ constexpr int INV_PRE = 8;  // words of the next row each thread prefetches
 // truncated, the sum exact (modulo 2^(32 WL)). Step i: the NT / 64 waves take the products j = k..i-1
 // in turn and add them on the lanes, carries left pending; wave 0 adds the waves' sums, propagates the
 // carries once and finishes x_ik with one more product. Row i + 1 of L is loaded while step i computes.
-// Grid (nb, BT), 512 threads. X entries above the diagonal are written as zeros.
+// Grid (nb, BT), 512 threads, or 256 or 1024 by SDPV_INV_THREADS. X entries above the diagonal are written as zeros.
 template <bool DEFAULT>
 __global__ void __launch_bounds__(DEFAULT ? 512 : 1024) k_tile_inverse(const u32* __restrict__ Wg, const u32* __restrict__ Rg,
                                                       u32* __restrict__ Xg, int BT, int WL, int LF) {
@@ -1184,6 +1186,26 @@ __global__ void __launch_bounds__(256) k_tile_narrow(const u32* __restrict__ W, 
 
 inline unsigned nblk(i64 n, int tpb) { return (unsigned)((n + tpb - 1) / tpb); }
 
+// a setting of the environment, read once
+inline int setting(const char* name, int unset) {
+    const char* e = getenv(name);
+    return e ? atoi(e) : unset;
+}
+// threads of the factorisation and, per column, of the inverse (see the kernels; the results are the same
+// whatever they are)
+inline int tile_threads() {
+    static const int v = setting("SDPV_TILE_THREADS", 1024);
+    return v == 256 || v == 512 ? v : 1024;
+}
+inline int inverse_threads() {
+    static const int v = setting("SDPV_INV_THREADS", 512);
+    return v == 256 || v == 1024 ? v : 512;
+}
+inline int tile_lane_pairs() {
+    static const int v = setting("SDPV_TILE_LANE_PAIRS", 0);
+    return v;
+}
+
 // the factorisation for magnitudes of N words
 template <int N, bool DEFAULT>
 int launch_factor_form(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, int nt, size_t lds, hipStream_t st) {
@@ -1192,13 +1214,14 @@ int launch_factor_form(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, int nt, 
         (void)hipFuncSetAttribute((const void*)k_tile_chol_lds<N, DEFAULT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
-    hipLaunchKernelGGL((k_tile_chol_lds<N, DEFAULT>), dim3((unsigned)nb), dim3(nt), lds, st, W, RI, BT, WL, LF, 0);
+    hipLaunchKernelGGL((k_tile_chol_lds<N, DEFAULT>), dim3((unsigned)nb), dim3(nt), lds, st, W, RI, BT, WL, LF,
+                       tile_lane_pairs());
     SDPV_TRY_LAUNCH();
     return SDPV_OK;
 }
 template <int N>
 int launch_factor(u32* W, u32* RI, i64 nb, int BT, int WL, int LF, int nt, size_t lds, hipStream_t st) {
-    return nt == 1024 ? launch_factor_form<N, true>(W, RI, nb, BT, WL, LF, nt, lds, st)
+    return nt == 1024 && tile_lane_pairs() <= 0 ? launch_factor_form<N, true>(W, RI, nb, BT, WL, LF, nt, lds, st)
                                                 : launch_factor_form<N, false>(W, RI, nb, BT, WL, LF, nt, lds, st);
 }
 
@@ -1231,7 +1254,7 @@ int tile_run(const i32* A, i64 plane, i64 ldb, i64 ldr, i64 L, i64 nb, i64 BT, i
     hipLaunchKernelGGL(k_tile_widen, dim3((unsigned)nrow), dim3(256), (size_t)4 * BT * (L | 1), st, A, plane, ldb, ldr,
                        (int)BT, (int)L, WL, W, top);
     SDPV_TRY_LAUNCH();
-    int nt = 1024, ni = 512;
+    int nt = tile_threads(), ni = inverse_threads();
     auto lds_f = [&] { return (size_t)lds_factor_words((int)BT, WL, nt / 64) * 4; };
     while (nt > 256 && lds_f() > 160 * 1024) nt /= 2;   // a wave's operands take 1 KB: BT = 38 at L = 24 fits with eight
     while (ni < 512 && BT * WL > INV_PRE * ni) ni *= 2;

@@ -1,4 +1,4 @@
-"""Threads of the tile kernels: a tile that fits in LDS
+"""Threads of the tile kernels: the documented settings take effect (and change no result), and a tile that fits in LDS
 beside the operands of fewer waves is factored there by fewer waves. Run under the CPU emulation of the kernels,
 against the oracle."""
 import subprocess
@@ -11,6 +11,9 @@ from tests.emu import harness
 
 @pytest.mark.parametrize("L,BT,settings,launches", [
     (2, 9, {}, "1 1"),                                           # inverse 512, factorisation 1024 threads
+    (2, 9, dict(SDPV_TILE_THREADS="256", SDPV_INV_THREADS="1024"), "0 1"),
+    (2, 9, dict(SDPV_TILE_THREADS="512", SDPV_INV_THREADS="256"), "1 0"),
+    (2, 9, dict(SDPV_TILE_LANE_PAIRS="20"), "1 1"),
     (2, 51, {}, "2 0"),                                          # 1024 threads' operands do not fit beside the tile
 ])
 def test_tile_launches(L, BT, settings, launches):
