@@ -800,7 +800,7 @@ int sdpv_copy_blocks(const sdpv_block* blocks, int64_t count, int32_t* m, int64_
     const i64 n = rows * cols;
     if (count == 0 || n == 0) return SDPV_OK;
     if (!blocks || !m || !e) return SDPV_EARG;
-    if (n > (1LL << 30) || L > 8 * 65535) return SDPV_ESIZE;
+    if (n > (1LL << 32) - TPB || L > 8 * 65535) return SDPV_ESIZE;   // 32-bit places, a launch's threads
     for (i64 j = 0; j < count; j++) {
         const sdpv_block& b = blocks[j];
         if (b.rows < 0 || b.cols < 0 || b.rows > rows || b.cols > cols) return SDPV_EARG;
