@@ -1,4 +1,5 @@
-"""Emulated products of one or two rows in large batches against the oracle. Usage: run_rows.py few L nb M N K"""
+"""Emulated products of one or two rows in large batches, and sums over segments with one or two columns, against
+the oracle. Usage: run_rows.py few L nb M N K | ksum L M N"""
 import os
 import random
 import sys
@@ -26,6 +27,12 @@ def few(L, nb, M, N, K):
         assert np.array_equal(C.limbs.numpy(), ref) and (om == 0 or np.array_equal(C.exp.numpy(), rexp)), mode
 
 
+def ksum(L, M, N):
+    from tests.test_gpu_ksum_oracle import ksum_parity
+    Bm._narrow = lambda *a, **k: True
+    ksum_parity(lambda t: t, L, M, N, [5, 0, 18])
+
+
 if __name__ == "__main__":
-    {"few": few}[sys.argv[1]](*(int(a) for a in sys.argv[2:]))
+    {"few": few, "ksum": ksum}[sys.argv[1]](*(int(a) for a in sys.argv[2:]))
     print("ok")
