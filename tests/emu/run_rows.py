@@ -1,5 +1,6 @@
 """Emulated products of one or two rows in large batches, and sums over segments with one or two columns, against
-the oracle. Usage: run_rows.py few L nb M N K | ksum L M N"""
+the oracle; sdpv_exact_dot against integers. Usage: run_rows.py few L nb M N K | ksum L M N |
+exact_dot L nb M N K NW ldk"""
 import os
 import random
 import sys
@@ -33,6 +34,11 @@ def ksum(L, M, N):
     ksum_parity(lambda t: t, L, M, N, [5, 0, 18])
 
 
+def exact_dot(*case):
+    from tests.test_gpu_exact_dot import exact_dot_parity
+    exact_dot_parity(lambda t: t, *case, lambda: None)
+
+
 if __name__ == "__main__":
-    {"few": few, "ksum": ksum}[sys.argv[1]](*(int(a) for a in sys.argv[2:]))
+    {"few": few, "ksum": ksum, "exact_dot": exact_dot}[sys.argv[1]](*(int(a) for a in sys.argv[2:]))
     print("ok")
