@@ -220,15 +220,17 @@ def _narrow(M, N, K, L, nb=1, rounded=False):
     L = 63 0.96 / 0.55; a 200 x 200 block, where launches count: rounded L = 40 2.0 / 1.9, L = 48 1.3 / 1.1, L = 63
     1.0 / 1.0; as they are 1.6 to 4 at every limb count. Few rows in large batches, rounded, two columns (500 x 2 x
     1000): L = 8 0.92, L = 24 0.63, L = 40 0.39; (3000 x 2 x 42): L = 8 1.7, L = 24 1.3, L = 40 0.85."""
-    if N > NARROW or M * K > NARROW_MK or K > NARROW_K or L > 63:
+    if N > NARROW or L > 63 or K > NARROW_K or M * K > NARROW_MK:
         return False
+    if L <= 40 and not rounded:
+        return True
     ks, tiles = -(-L // 8), -(-M // 32)
-    work = nb * N * tiles * K // 128                         # slices of 32 rows and 128 k
     cols = nb * N * tiles
     if cols <= 16 and (ks <= 6 or not rounded):              # too few product tiles to fill the device
         return True
+    work = cols * K // 128                                   # slices of 32 rows and 128 k
     if not rounded:
-        if ks <= 5 or (ks == 6 and N == 1) or (M <= 2 and M * N * K <= 200):
+        if M <= 2 and M * N * K <= 200 or ks == 6 and N == 1:
             return True
         return work <= 256 if ks == 6 else N * work <= 200
     if cols * -(-K // 128) <= 256 if ks <= 5 else N * work <= 128 if ks == 6 else N == 1 and 24 <= work <= 64:
