@@ -79,10 +79,8 @@ int sdpv_badd_align(const int32_t* A, const int32_t* Bm, const int64_t* EA, cons
  * written exactly as NW >= 2L + 2 words W[w * E + e] (E = nb * M * N), with its bit length (of ~S
  * when S < 0) in bitlen[e]: the words and bit lengths that sdpv_rns_crt's word mode returns for the
  * same product. K is split into slices whose sums go through `work` (sdpv_exact_dot_work(...) int64
- * entries, 0 when there is one slice of at most 32 rows). No counterpart in the reference, which
- * always goes through residues: the direct path for products with one or two right-hand-side
- * columns (triangular solves with one vector), where the residue path's fixed costs dominate.
- * L <= 63. */
+ * entries, also what sdpv_narrow takes for the same sizes; may be 0). No counterpart in the reference,
+ * which always goes through residues. L <= 63. */
 int64_t sdpv_exact_dot_work(int64_t L, int64_t nb, int64_t M, int64_t N, int64_t K);
 int sdpv_exact_dot(const int32_t* A, int64_t planeA, int64_t ldAb, int64_t ldAr, int64_t ldAk,
                    const int32_t* B, int64_t planeB, int64_t ldBb, int64_t ldBr, int64_t ldBk,

@@ -329,7 +329,8 @@ class BTile:
 
 def bchol_tile(A, LI=24, threads=256):
     """factor and invert the bt x bt tiles A (nb, bt, bt) (fixed point at -(32L - 40)) on the GPU:
-    (L as a BMP, BTile) with X rounded to headroom_bits(L) below its largest entry, per block"""
+    (L as a BMP, BTile) with X rounded to headroom_bits(L) below its largest entry, per block. LI and threads are the
+    reference's; the kernels have their own (24 words more, and as many threads as the tile takes)"""
     from .basecase import tile_factor_inverse
     nb, b, _ = A.shape
     L = A.L

@@ -706,9 +706,9 @@ __device__ __forceinline__ void tri_pair(int p, int& i, int& j) {
     j = p - r * (r + 1) / 2;
 }
 
-// A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`), taken where an operand has words above N (a factor of
-// an SPD tile never has): x, y magnitudes with top words ta, tb, A a WL-word two's complement target. The column sums are formed four columns at a time:
-// x[i] is read once per block and the four operand words y[kb + c - i] sit in a window of registers
+// A -= s * mulfx(x, y, 0) on LDS words (s = +1, or -1 when `add`), taken where an operand has words above N
+// (ta >= N or tb >= N; a factor of an SPD tile never has): x, y magnitudes with top words ta, tb, A a WL-word two's
+// complement target. The column sums are formed four columns at a time: x[i] is read once per block and the four operand words y[kb + c - i] sit in a window of registers
 // that shifts by one word per i, so a block costs two LDS reads per i instead of eight; the target
 // words of a block are read before its columns are summed. The column sums, the carry chain and the
 // target words equal those of mulfx_mag and its consumer (terms outside the tops are zero).

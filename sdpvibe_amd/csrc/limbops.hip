@@ -101,8 +101,6 @@ __global__ void __launch_bounds__(TPB) k_badd_align(const i32* __restrict__ A, c
     if ((e / cols) % rows == 0) EO[col] = ex;
 }
 
-// both parts of a stacked solve re-rounded to their columns' larger exponent and joined, one pass (a
-// rounding each, a broadcast shift per entry and a concatenation took seven launches)
 // blocks of uneven dimension to and from a stack: up to 32 per launch, their places passed with the launch
 // (no table to copy, none to keep). One workgroup row of grid.y per block, 8 limb planes per grid.z. Two copies
 // per block and array before: factoring and solving 400 uneven blocks
@@ -136,6 +134,8 @@ __global__ void __launch_bounds__(TPB) k_copy_blocks(BlockList list, i32* __rest
     }
 }
 
+// both parts of a stacked solve re-rounded to their columns' larger exponent and joined, one pass (a
+// rounding each, a broadcast shift per entry and a concatenation took seven launches)
 __global__ void __launch_bounds__(TPB) k_stack_common(const i32* __restrict__ P1, const i64* __restrict__ E1,
                                                       const i32* __restrict__ P2, const i64* __restrict__ E2,
                                                       i32* __restrict__ O, i64* __restrict__ EO, int L, i64 nb, i64 R1,
@@ -256,7 +256,8 @@ __device__ void mul_any(const PlaneSrc& xa, const PlaneSrc& xb, int L, i64 n, i6
 
 // one entry per thread. Limbs sit in the upper L of N words, so the product of two normalised entries has
 // its rounded words at static places whatever L is. 787 320 products at L = 24 on one MI355X:
-// 0.061 ms, 4.0 TB/s (operands in LDS slices, word by word: 0.511 ms).
+// 0.061 ms, 4.0 TB/s (operands in LDS slices, word by word: 0.511 ms); one after the other on the same operands,
+// as they stay in the caches, L = 14 / 24 / 32 / 40 0.033 / 0.052 / 0.081 / 0.114 ms (0.128 / 0.420 / 1.04 / 1.48).
 template <int N>
 __global__ void __launch_bounds__(256) k_mul_regs(const i32* __restrict__ A, const i64* __restrict__ eA,
                                                   const i32* __restrict__ Bm, const i64* __restrict__ eB,
@@ -355,7 +356,9 @@ __device__ __forceinline__ void round_down(u32* x, i64 s) {
 
 // A + sgn B (mpf.py:92-124): the operand with the larger exponent one word up, the other rounded to the same
 // place, magnitudes added or subtracted, the result normalised. 787 320 sums at L = 24 on one
-// MI355X: 0.079 ms, 3.1 TB/s (operands read word by word at every use, sums in LDS: 0.344 ms).
+// MI355X: 0.079 ms, 3.1 TB/s (operands read word by word at every use, sums in LDS: 0.344 ms); one after the
+// other on the same operands, L = 14 / 24 / 32 / 40 0.037 / 0.053 / 0.105 / 0.149 ms (0.090 / 0.189 / 0.319 / 0.472):
+// above 24 limbs the registers hold three waves per SIMD, above 32 two.
 template <int N>
 __global__ void __launch_bounds__(256) k_add_regs(const i32* __restrict__ A, const i64* __restrict__ eA,
                                                   const i32* __restrict__ Bm, const i64* __restrict__ eB,

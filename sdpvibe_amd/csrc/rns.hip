@@ -75,7 +75,7 @@ __device__ __forceinline__ u32 pack4(int a, int b, int c, int d) {  // low bytes
 // fits 128 VGPRs, four workgroups per CU. SMALL (KSC 1..4): small launches, whose time is one chain of
 // dependent steps: the prime blocks are shared out over grid.y (each workgroup repeats phase 1) and the limbs
 // rounded in registers. The splits of chol(Q) at N = 3000, mostly of 32 to 1504 rows of 32 entries: 12.8 us on
-// average before, 7.4 now. For large launches this form measured equal or slower (60 x 192 x 3000: 0.50
+// average before, 6.1 now. For large launches this form measured equal or slower (60 x 192 x 3000: 0.50
 // against 0.47 ms).
 template <int KSC, bool SMALL>
 __global__ void __launch_bounds__(256, (KSC >= 1 && KSC <= 3) ? 4 : 1) k_rns_split(
@@ -922,7 +922,7 @@ __global__ void __launch_bounds__(64) k_rns_crt(
 // input): a launch then takes one chain of dependent steps, which is a quarter as long here. Each wave takes
 // a quarter of the primes in phase 1 (all its loads at once) and every fourth digit block in phase 2, whose
 // 64-bit word partials meet in LDS; wave 0 carries and rounds. The reconstructions of chol(Q) at N = 3000,
-// L = 24: 17.2 us on average before, 13.4 now (15.6 with the addend, whose own pass took 9.3).
+// L = 24: 17.2 us on average before, 13.9 now with the addend of most of them, whose own pass took 9.3.
 __global__ void __launch_bounds__(256) k_rns_crt4(
     const int16_t* __restrict__ acc, int n, i64 ld_g, i64 rows, i64 N, i64 j0, i64 w, const double* __restrict__ minv,
     const int8_t* __restrict__ Ct, int E, int npad, int mode, i32* __restrict__ W, i64* __restrict__ bitlen,

@@ -438,8 +438,8 @@ class KSum:
     """C = sum over segments s of A_s^T B_s (A_s (K_s, M), B_s (K_s, N), 2-d MPF), equal bit for bit
     to gemm(cat(A_s), cat(B_s), transA=True) over the segments stacked along K: every entry is
     rounded at the row exponents of the whole stack (EA = max over segments of col_exps(A_s), EB
-    likewise), the exact products are summed as residues over all segments, and one reconstruction
-    rounds the sum. The segments need not be on the device together (a segment may be fetched,
+    likewise), the exact products are summed over all segments (as residues; with one or two columns as
+    the exact words of every entry), and one reconstruction rounds the sum. The segments need not be on the device together (a segment may be fetched,
     added and dropped), and the result does not depend on how the rows are split."""
 
     def __init__(self, EA, EB, L):
