@@ -370,7 +370,7 @@ def gemm(A, B, transA=False, transB=False):
     N, K2, bldb, bldr, bldk = _geometry(Be.shape, not transB)   # rows of op(B)^T = columns of op(B)
     assert K == K2, (A.shape, B.shape, transA, transB)
     R = ctx(L)
-    narrow = _batched._narrow(max(M, N), min(M, N), K, L, nb, True)
+    narrow = min(M, N) <= _batched.NARROW and _batched._narrow(max(M, N), min(M, N), K, L, nb, True)
     if not narrow and nb * M * N * K != 0 and K <= R.kmax:
         kp = R.kp_product(K)
         up = lambda x: (x + 255) & ~255
