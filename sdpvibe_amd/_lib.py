@@ -124,5 +124,12 @@ def ptr_strided(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
+def ptr_view(t):
+    """Device pointer of a GPU tensor view of any strides, which the caller passes to the entry point"""
+    if not t.is_cuda:
+        raise ValueError("the HIP library takes GPU tensors only")
+    return ctypes.c_void_p(t.data_ptr())
+
+
 def stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)

@@ -33,6 +33,8 @@ def tile_factor_inverse(limbs, BT, hb):
     """limbs as for tile_factor, any view -> (Lout, X (L, nb, BT, BT) rounded to hb bits below the largest
     entry of its tile, its exponents (nb, BT))"""
     L, nb = limbs.shape[0], limbs.shape[1]
+    if limbs.shape != (L, nb, BT, BT):         # the kernel trusts these sizes
+        raise ValueError(f"tiles of {BT} rows from {tuple(limbs.shape)} limbs")
     if limbs.stride(3) != 1:
         limbs = limbs.contiguous()
     Lout = torch.empty((L, nb, BT, BT), dtype=torch.int32, device=limbs.device)

@@ -11,7 +11,7 @@ array instead of being concatenated level by level.
 """
 import torch
 
-from ._lib import call, lib, ptr, stream
+from ._lib import call, lib, ptr, ptr_view, stream
 from .limbops import _errbuf, add_same, shift_round
 from .mpmat import ctx, headroom_bits, residue_gemm
 from .rns import dev
@@ -133,7 +133,7 @@ def bgemm_nt(A, Bt, out_exp="col", kc=4096, bt_rowexp=None, bt_cache=None, plus=
     L = A.L
     R = ctx(L)
     eB = Bt.exp if bt_rowexp is None else bt_rowexp
-    if _narrow(M, N, K, L, nb):
+    if Bt.L == L and _narrow(M, N, K, L, nb):
         C = _narrow_product(A, Bt, eB, out_exp if isinstance(out_exp, int) else "col")
         if plus is not None:
             C = badd(plus, C, sgn, out_exp=out_exp)
@@ -242,47 +242,52 @@ def _narrow(M, N, K, L, nb=1, rounded=False):
     return (M + N + 3 * tiles) * K + 470 * tiles >= N * tiles * K * per_k
 
 
-def flat_view(X):
-    """the storage of a view with non-negative strides from its first entry to its last, as a contiguous
-    1-d tensor (for entry points that take base pointer and strides)"""
-    if X.numel() == 0:
-        return X.reshape(-1)
-    return torch.as_strided(X, (sum((n - 1) * s for n, s in zip(X.shape, X.stride())) + 1,), (1,))
-
-
 def narrow_work(L, nb, M, N, K, device):
     """scratch of sdpv_narrow for this shape: (tensor, int64 entries)"""
     n = int(lib().sdpv_exact_dot_work(L, nb, M, N, K))
     return torch.empty((max(n, 1),), dtype=torch.int64, device=device), n
 
 
+def _exponents(e, nb, C):
+    """exponents that broadcast to (nb, C) as a contiguous int64 tensor of that shape"""
+    if e.shape != (nb, C):
+        e = e.expand(nb, C)
+    return (e if e.dtype == torch.int64 else e.to(torch.int64)).contiguous()
+
+
 def _narrow_product(A, Bt, eB, out_exp, plus=None, sgn=1):
     """A Bt^T with few rows of Bt as one direct product, rounded to the int out_exp or per (block,
     column) ('col'); plus: a BMP X (possibly a view), the result is then badd(X, A Bt^T, sgn, 'align')"""
-    nb, M, K = A.shape
-    N, L = Bt.shape[1], A.L
     Al, Bl = A.limbs, Bt.limbs
-    sa, sb = Al.stride(), Bl.stride()
+    L, nb, M, K = Al.shape
+    N = Bl.shape[2]
+    fixed = isinstance(out_exp, int)
+    if Bl.shape != (L, nb, N, K):              # the kernel trusts these sizes
+        raise ValueError(f"product of {tuple(Al.shape)} and {tuple(Bl.shape)} limbs")
+    if M == 0 and not fixed:
+        raise IndexError("no rows to take the columns' exponents from")
     out = torch.empty((L, nb, M, N), dtype=torch.int32, device=Al.device)
     e0, ea, lea, eb = 0, None, 0, None
     if isinstance(A.exp, int):
         e0 += A.exp
     else:
-        ea = A.exp.contiguous()                # (nb, C), read at column 0
-        lea = ea.shape[1]
+        ea = _exponents(A.exp[:, :1], nb, 1)   # (nb, C), read at column 0
+        lea = 1
     if isinstance(eB, int):
         e0 += eB
     else:
-        eb = (eB[:, None].expand(nb, N) if eB.dim() == 1 else eB).contiguous()
-    fixed = isinstance(out_exp, int)
+        eb = _exponents(eB[:, None] if eB.dim() == 1 else eB, nb, N)
     exps = None if fixed else torch.empty((nb, N), dtype=torch.int64, device=Al.device)
     X, sx, eX = None, (0, 0, 0, 0), None
     if plus is not None:
-        X, sx, eX = flat_view(plus.limbs), plus.limbs.stride(), plus.expt().contiguous()
+        Xl = plus.limbs
+        if Xl.shape != out.shape:
+            raise ValueError(f"sum of {tuple(Xl.shape)} and {tuple(out.shape)} limbs")
+        X, sx, eX = ptr_view(Xl), Xl.stride(), _exponents(plus.expt(), nb, N)
     work, nwork = narrow_work(L, nb, M, N, K, Al.device)
-    call("sdpv_narrow", ptr(flat_view(Al)), None, None, *sa, ptr(flat_view(Bl)), None, None, *sb, L, nb, M, N, K,
+    call("sdpv_narrow", ptr_view(Al), None, None, *Al.stride(), ptr_view(Bl), None, None, *Bl.stride(), L, nb, M, N, K,
          2 if fixed else 3, ptr(out), nb * M * N, M * N, N, 1, ptr(exps), e0, ptr(ea), lea, ptr(eb),
-         out_exp if fixed else 0, ptr(X), *sx, ptr(eX), sgn, ptr(_errbuf()), ptr(work), nwork, stream())
+         out_exp if fixed else 0, X, *sx, ptr(eX), sgn, ptr(_errbuf()), ptr(work), nwork, stream())
     return BMP(out, out_exp if fixed else exps)
 
 
@@ -454,11 +459,14 @@ def _apply_tile(X, Lm, B, refine):
 
 def _stack_common(P1, P2):
     """[P1; P2] with one exponent per (block, column): both parts re-rounded to the larger"""
-    nb, R1, C = P1.shape
-    R2, L = P2.shape[1], P1.L
-    out = torch.empty((L, nb, R1 + R2, C), dtype=torch.int32, device=P1.limbs.device)
-    ee = torch.empty((nb, C), dtype=torch.int64, device=P1.limbs.device)
-    m1, e1, m2, e2 = (x.contiguous() for x in (P1.limbs, P1.expt(), P2.limbs, P2.expt()))
+    m1, m2 = P1.limbs.contiguous(), P2.limbs.contiguous()
+    L, nb, R1, C = m1.shape
+    R2 = m2.shape[2]
+    if m2.shape != (L, nb, R2, C):             # the kernel trusts these sizes
+        raise ValueError(f"halves of {tuple(m1.shape)} and {tuple(m2.shape)} limbs")
+    out = torch.empty((L, nb, R1 + R2, C), dtype=torch.int32, device=m1.device)
+    ee = torch.empty((nb, C), dtype=torch.int64, device=m1.device)
+    e1, e2 = _exponents(P1.expt(), nb, C), _exponents(P2.expt(), nb, C)
     call("sdpv_stack_common", ptr(m1), ptr(e1), ptr(m2), ptr(e2), ptr(out), ptr(ee), L, nb, R1, R2, C, ptr(_errbuf()),
          stream())
     return BMP(out, ee)
@@ -468,7 +476,7 @@ def _minus_product(X, A, P):
     """badd(X, A P, -1, 'align'): rows X of a right-hand side less a block of the factor times the part
     already solved; one direct product with few columns"""
     nb, M, K = A.shape
-    if _narrow(M, P.shape[2], K, A.L, nb):
+    if P.L == A.L and _narrow(M, P.shape[2], K, A.L, nb):
         return _narrow_product(A, _as_rows(P), P.expt(), "col", plus=X, sgn=-1)
     return badd(X, bgemm_nt(A, _as_rows(P), out_exp="col", bt_rowexp=P.expt()), -1, out_exp="align")
 

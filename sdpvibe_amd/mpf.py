@@ -369,6 +369,8 @@ def gemm(A, B, transA=False, transB=False):
     M, K, aldb, aldr, aldk = _geometry(Ae.shape, transA)
     N, K2, bldb, bldr, bldk = _geometry(Be.shape, not transB)   # rows of op(B)^T = columns of op(B)
     assert K == K2, (A.shape, B.shape, transA, transB)
+    if Am.numel() < L * Ae.numel() or Bm.numel() < L * Be.numel():   # the kernels trust these sizes
+        raise ValueError("gemm: limb planes smaller than the exponents")
     R = ctx(L)
     narrow = min(M, N) <= _batched.NARROW and _batched._narrow(max(M, N), min(M, N), K, L, nb, True)
     if not narrow and nb * M * N * K != 0 and K <= R.kmax:
@@ -377,8 +379,6 @@ def gemm(A, B, transA=False, transB=False):
         nwork = up(8 * nb * M) + up(8 * nb * N) + 2 * up(R.n * kp * nb * M) + 2 * up(R.n * kp * nb * N) + \
             up(2 * R.n * nb * M * N)
         if nwork <= SMALL_GEMM and not panelled(R.n, nb, M, N, K):
-            if Am.numel() < L * Ae.numel() or Bm.numel() < L * Be.numel():
-                raise ValueError("gemm: limb planes smaller than the exponents")
             out_m = torch.empty((L, nb, M, N), dtype=torch.int32, device=dev)
             out_e = torch.empty((nb, M, N), dtype=torch.int64, device=dev)
             work = torch.empty((nwork,), dtype=torch.uint8, device=dev)
@@ -464,6 +464,8 @@ class KSum:
             raise ValueError(f"KSum: inner dimension {self.K + K} exceeds the RNS bound {R.kmax}")
         Am, Ae, Bm, Be = A.m.contiguous(), A.e.contiguous(), B.m.contiguous(), B.e.contiguous()
         if self.direct:                          # K is within sdpv_narrow's bound: it is the RNS bound above
+            if Am.numel() < L * K * M or Bm.numel() < L * K * N:
+                raise ValueError("KSum.add: limb planes smaller than the exponents")
             if K and M and N:
                 work, nwork = _batched.narrow_work(L, 1, M, N, K, Am.device)
                 call("sdpv_narrow", ptr(Am), ptr(Ae), ptr(self.EA), K * M, K * M, 1, M, ptr(Bm), ptr(Be), ptr(self.EB),

@@ -58,6 +58,8 @@ def install():
             mod.ptr = emu_ptr
         if hasattr(mod, "ptr_strided"):
             mod.ptr_strided = emu_ptr_strided
+        if hasattr(mod, "ptr_view"):
+            mod.ptr_view = lambda t: ctypes.c_void_p(t.data_ptr())
         if hasattr(mod, "stream"):
             mod.stream = lambda: None
         if hasattr(mod, "dev"):
