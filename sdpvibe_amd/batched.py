@@ -230,11 +230,15 @@ def _narrow(M, N, K, L, nb=1, rounded=False):
         return True
     work = cols * K // 128                                   # slices of 32 rows and 128 k
     if not rounded:
-        if M <= 2 and M * N * K <= 200 or ks == 6 and N == 1:
+        if (M <= 2 and M * N * K <= 200) or (ks == 6 and N == 1):
             return True
         return work <= 256 if ks == 6 else N * work <= 200
-    if cols * -(-K // 128) <= 256 if ks <= 5 else N * work <= 128 if ks == 6 else N == 1 and 24 <= work <= 64:
-        return True                                          # both wait for launches: fewer of them
+    if ks <= 5:
+        few = cols * -(-K // 128) <= 256
+    else:
+        few = N * work <= 128 if ks == 6 else N == 1 and 24 <= work <= 64
+    if few:                                                  # both routes wait for launches: fewer of them
+        return True
     # per block, in times of a k of a split row: splits and a tile of the product against k of a slice
     per_k = (4.5, 6.8, 6.8, 10, 11, 36, 54, 47)[ks - 1]
     if ks <= 5:
